@@ -74,22 +74,6 @@ template <int B, int E, class F> __device__ __forceinline__ void for_nb(F &&f) {
 }
 template <class F> __device__ __forceinline__ void for_each_nb(F &&f) { for_nb<0, 26>(f); }
 
-// Calls f(integral_constant B, integral_constant E) for each part [B, E) of the 26 neighbours that
-// has a set bit in m; Batch = neighbours per part (26, 13 or 9).
-template <int Batch, class F> __device__ __forceinline__ void for_parts(unsigned m, F &&f) {
-  using std::integral_constant;
-  if constexpr (Batch >= 26) {
-    if (m) f(integral_constant<int, 0>{}, integral_constant<int, 26>{});
-  } else if constexpr (Batch >= 13) {
-    if (m & 0x1FFFu) f(integral_constant<int, 0>{}, integral_constant<int, 13>{});
-    if (m >> 13) f(integral_constant<int, 13>{}, integral_constant<int, 26>{});
-  } else {
-    if (m & 0x1FFu) f(integral_constant<int, 0>{}, integral_constant<int, 9>{});
-    if ((m >> 9) & 0x1FFu) f(integral_constant<int, 9>{}, integral_constant<int, 18>{});
-    if (m >> 18) f(integral_constant<int, 18>{}, integral_constant<int, 26>{});
-  }
-}
-
 // ---- device-memory access in the global address space -------------------------------------------
 // Pointers that reach a kernel inside a struct are generic, and generic accesses compile to FLAT
 // instructions, which also count against the LDS counter (so every LDS wait waits for them too)
@@ -157,24 +141,12 @@ __device__ __forceinline__ void st_u64(unsigned long long *p, unsigned long long
 #ifndef BROOK_LABEL_SCOPE
 #define BROOK_LABEL_SCOPE __HIP_MEMORY_SCOPE_WORKGROUP
 #endif
-__device__ __forceinline__ float lp_f(const float *p) { return __hip_atomic_load(gp(p), __ATOMIC_RELAXED, BROOK_LABEL_SCOPE); }
 __device__ __forceinline__ int lp_i(const int *p) { return __hip_atomic_load(gp(p), __ATOMIC_RELAXED, BROOK_LABEL_SCOPE); }
-__device__ __forceinline__ unsigned lp_u(const unsigned *p) { return __hip_atomic_load(gp(p), __ATOMIC_RELAXED, BROOK_LABEL_SCOPE); }
 __device__ __forceinline__ unsigned long long lp_u64(const unsigned long long *p) {
   return __hip_atomic_load(gp(p), __ATOMIC_RELAXED, BROOK_LABEL_SCOPE);
 }
-__device__ __forceinline__ void sp_f(float *p, float v) { __hip_atomic_store(gp(p), v, __ATOMIC_RELAXED, BROOK_LABEL_SCOPE); }
 __device__ __forceinline__ void sp_u64(unsigned long long *p, unsigned long long v) {
   __hip_atomic_store(gp(p), v, __ATOMIC_RELAXED, BROOK_LABEL_SCOPE);
-}
-
-// One vertex-weighted step fl(d + f) that never returns d itself for a positive cost: one ulp up
-// instead (the rule of the reference's brook_vw_step, common.cuh:123-127), which keeps distances
-// strictly increasing along every step so predecessor walks terminate.
-__device__ __forceinline__ float vw_step(float d, float f) {
-  float c = d + f;
-  if (c == d && f > 0.0f && d < kInf) c = __int_as_float(__float_as_int(d) + 1);
-  return c;
 }
 
 // atomicMin of a non-negative float through its int bits (monotone for floats >= 0, +inf included);
@@ -197,76 +169,61 @@ __device__ __forceinline__ int wave_slot(int *counter) {
   return base + __popcll(act & ((1ULL << lane) - 1ULL));
 }
 
-// Reserves n slots per lane in a list whose length lives at *counter; returns the lane's first
-// slot. All 64 lanes must be active: one inclusive scan and one atomic per wave.
-__device__ __forceinline__ int wave_reserve(int *counter, int n) {
-  const int lane = __lane_id();
-  int x = n;
-  for (int off = 1; off < 64; off <<= 1) {
-    const int y = __shfl_up(x, off, 64);
-    if (lane >= off) x += y;
-  }
-  const int total = __shfl(x, 63, 64);
-  int base = 0;
-  if (lane == 63 && total) base = atomicAdd(counter, total);
-  base = __shfl(base, 63, 64);
-  return base + x - n;
+// What the floods and the tracer touch per voxel, in three arrays, so that each phase's neighbour
+// walk reads 8 bytes per neighbour:
+//   mask   u32, bits [0, 26): the neighbours of the voxel's own nonzero id (0 for background)
+//   road   u64, floods and railroad: distance (31 bits: a float's without its sign, which is 0) << 33
+//          | far listed << 32 | not queued << 31 | cost (the PDRF's 31 bits; rails 0). One load gives a
+//          neighbour's cost and its distance, and words of one voxel, whose cost is the same, order
+//          by (distance, flags), so one atomic minimum both improves the distance and tells what
+//          the voxel was. Unreached: distance +inf, not queued, so a candidate of infinite cost never
+//          improves one.
+//   claim  u64, invalidation: bottleneck << 32 | (source + 1) << 1 | queued; kDead (low half 0, which
+//          no claim has) once the voxel is invalidated, kFree while it is alive and unclaimed.
+// Background words of road and claim are never written, and both arrays have word_pad() words before
+// and after the volume's, so a neighbour walk loads all 26 neighbours' words and lets the mask bits,
+// which arrive beside them, say which count.
+constexpr unsigned kCostBits = 0x7FFFFFFFu;
+constexpr unsigned kInfBits = 0x7F800000u;
+constexpr unsigned long long kNotQueued = 1ULL << 31, kFarListed = 1ULL << 32;
+constexpr unsigned long long kUnreached = ((unsigned long long)kInfBits << 33) | kNotQueued;  // or'ed with the cost
+__host__ __device__ constexpr unsigned road_dist(unsigned long long w) { return unsigned(w >> 33); }
+__host__ __device__ constexpr unsigned road_cost(unsigned long long w) { return unsigned(w) & kCostBits; }
+__host__ __device__ constexpr unsigned long long road_word(unsigned dist, unsigned long long flags, unsigned cost) {
+  return ((unsigned long long)dist << 33) | flags | cost;
+}
+constexpr unsigned long long kFloodFree = kUnreached | kCostBits;  // the floods' words (no cost yet)
+
+constexpr unsigned long long kDead = 0ULL, kFree = ~0ULL;
+
+constexpr long long word_pad(const Dims &d) { return (long long)d.sx * d.sy + d.sx + 1; }
+// Volumes whose padded words lie within 32-bit byte offsets: the kernels' narrow form, which adds a
+// 32-bit offset per lane to a scalar base instead of computing 64-bit addresses.
+constexpr bool narrow_words(const Dims &d) {
+  return (long long)d.sx * d.sy * d.sz + 2 * word_pad(d) <= (1LL << 29);
 }
 
-// Appends u + off[k] for every set bit k of mask (all 64 lanes active; off: neighbour offsets).
-__device__ __forceinline__ void emit_neighbours(int *list, int *counter, unsigned mask, int u, const int *off) {
-  int pos = wave_reserve(counter, __popc(mask));
-  while (mask) {
-    const int k = __ffs(mask) - 1;
-    mask &= mask - 1;
-    g_st(list + pos++, u + off[k]);
-  }
-}
-
-// Minimum over the wave (all 64 lanes active).
-__device__ __forceinline__ unsigned long long wave_min_u64(unsigned long long v) {
-  for (int off = 32; off > 0; off >>= 1) {
-    unsigned long long o = __shfl_xor(v, off, 64);
-    v = o < v ? o : v;
-  }
-  return v;
-}
-
-// Everything the floods and the tracer touch per voxel, in one 16-byte record (one cache line holds
-// eight voxels of a row): a neighbour costs one line instead of one per array.
-//   pdrf  the penalty field (rails 0)
-//   meta  bits [0,26) the same-label neighbour mask, then kAlive and kWaiting (invalidation: waiting
-//         for a later band)
-//   word  a distance word (see word_dist_bits; the railroad also keeps bit 1 = "far listed") or an
-//         invalidation claim (bottleneck, source, queued bit); ~0 between uses
-struct alignas(16) VoxelRec {
-  float pdrf;
-  unsigned meta;
-  unsigned long long word;
+// Division of 0 <= n < 2^31 by a constant d >= 1 as a high product and a shift: with 2^l the power
+// of two at or above d and m = ceil(2^(31 + l) / d) < 2^32, m * d exceeds 2^(31 + l) by less than
+// d <= 2^l, so n * m / 2^(31 + l) exceeds n / d by less than 1 / d and has its integer part. d = 1
+// has l = 0, no such form: `one` passes n through.
+struct FastDiv {
+  unsigned m = 0, shift = 0, one = 0;
 };
-constexpr unsigned kNbrBits = (1u << 26) - 1u;
-constexpr unsigned kAlive = 1u << 26, kWaiting = 1u << 29;
-
-__device__ __forceinline__ float rec_pdrf(const VoxelRec *r, int v) { return lp_f(&r[v].pdrf); }
-__device__ __forceinline__ unsigned rec_meta(const VoxelRec *r, int v) { return lp_u(&r[v].meta); }
-// The whole record in one 16-byte load (x = pdrf bits, y = meta, z = word low, w = word high), for
-// walks that need two of its fields: one scattered access instead of two. During the flood and
-// trace kernels only the workgroup that owns the voxel's label touches its record, as for the
-// workgroup-scope loads above.
-typedef unsigned RecWords __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ RecWords rec_load(const VoxelRec *r, int v) {
-  return *gp(reinterpret_cast<const RecWords *>(r + v));
+constexpr FastDiv fast_div(unsigned d) {
+  FastDiv f;
+  if (d <= 1) {
+    f.one = ~0u;
+    return f;
+  }
+  unsigned l = 0;
+  while ((1ULL << l) < d) ++l;
+  f.m = unsigned(((1ULL << (31 + l)) + d - 1) / d);
+  f.shift = l - 1;
+  return f;
 }
-// The high half of the word (distance bits or claim bottleneck) without the 64-bit load.
-__device__ __forceinline__ unsigned rec_word_hi(const VoxelRec *r, int v) {
-  return lp_u(reinterpret_cast<const unsigned *>(&r[v].word) + 1);
-}
-
-// A 64-bit voxel word of the distance floods: high half = the distance's float bits, low half bit 0
-// = "not queued". ~0 (the shared sentinel) reads as +inf, not queued.
-__device__ __forceinline__ unsigned word_dist_bits(unsigned long long w) {
-  const unsigned hi = (unsigned)(w >> 32);
-  return hi == 0xFFFFFFFFu ? 0x7f800000u : hi;
+__host__ __device__ __forceinline__ unsigned fast_quotient(unsigned n, const FastDiv &f) {
+  return unsigned((unsigned long long)n * f.m >> 32 >> f.shift) + (n & f.one);
 }
 
 // Shuffle of any integer width up by `delta` lanes (wave64).
@@ -275,19 +232,16 @@ template <class T> __device__ __forceinline__ T shfl_up_any(T v, unsigned delta)
   else return T(__shfl_up((unsigned)v, delta, 64));
 }
 
-// A group of lanes per front entry, for fronts of at most a quarter of the workgroup: each entry
-// gets G lanes (the largest power of two up to 32 that fits every entry into the workgroup, at
-// least 4); lane g of a group handles neighbours [g*S, g*S + S), S = ceil(26 / G) <= kSpan, so all
-// of an entry's loads, then all of its atomics, are in flight together instead of part after part.
-// One code path serves every G (a span is kSpan slots, the tail predicated off), which keeps a
-// kernel's register pressure at the level of its one-thread-per-entry path. (Pairs of lanes for
-// fronts up to half a workgroup, two spans each, measured no faster on the 512^3 workload.)
+// A group of lanes per front entry: each of n entries gets G lanes of the workgroup (the largest power
+// of two up to 32 that fits every entry, at least 4); lane g of a group handles neighbours
+// [g*S, g*S + S), S = ceil(26 / G) <= kSpan. The frontier kernels use the layout of block / 32
+// entries: half a wave per entry, a neighbour per lane (front.hpp).
 constexpr int kSpan = 7;
 struct Group {
   int G, i, g, lead, kb, cnt;  // lanes per entry, entry, lane in group, group's first lane, span
 };
-// The group of thread `tid` for a front of n entries in a workgroup of `block` threads (host-callable,
-// so the CPU tests check the layout for every n, block and thread).
+// The group of thread `tid` for n entries in a workgroup of `block` threads (host-callable, so the CPU
+// tests check the layout for every n, block and thread).
 __host__ __device__ constexpr Group group_at(int n, int block, int tid) {
   Group q{};
   q.G = 32;
@@ -302,7 +256,6 @@ __host__ __device__ constexpr Group group_at(int n, int block, int tid) {
   q.cnt = span < 26 - q.kb ? span : 26 - q.kb;  // may be <= 0: nothing to do
   return q;
 }
-__device__ __forceinline__ Group group_of(int n, int block) { return group_at(n, block, int(threadIdx.x)); }
 
 // Mask of lanes 0..lane.
 __device__ __forceinline__ unsigned long long lanes_upto(int lane) {

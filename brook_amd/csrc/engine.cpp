@@ -272,8 +272,9 @@ class Sample {
         root_dev.upload(ax, none.data(), k);
         const std::vector<float> W = step_weights(o_.aniso);
         weights.upload(ax, W.data(), 26);
-        Buffer<VoxelRec> rec(ax, size_t(n_));
-        voxel_records(ax, cc_.labels.data(), cc_.cc_bytes, d_, rec.data());
+        Buffer<unsigned> mask(ax, size_t(n_));
+        Buffer<unsigned long long> road = words(ax);
+        voxel_words(ax, cc_.labels.data(), cc_.cc_bytes, d_, mask.data(), first_word(road));
         Buffer<int> la(ax, F), lb(ax, F), fa(ax, 2 * F), fb(ax, 2 * F);
         FloodJob j;
         j.d = d_;
@@ -285,7 +286,9 @@ class Sample {
         j.t.target = target_dev.data();
         j.t.max_daf = max_daf_dev.data();
         j.t.weights = weights.data();
-        j.t.rec = rec.data();
+        j.t.mask = mask.data();
+        j.t.road0 = road.data();
+        j.t.road = first_word(road);
         j.lists_a = la.data();
         j.lists_b = lb.data();
         j.far_a = fa.data();
@@ -294,7 +297,8 @@ class Sample {
         // one workgroup per label, at most a quarter of the chip: the EDT runs beside it
         prepare_fields(ax, {j}, items, std::max(1, ax.compute_units() / 4));
         std::vector<long long> roots = root_dev.download(ax);  // (synchronizes the auxiliary stream)
-        early_rec_ = std::move(rec);
+        early_mask_ = std::move(mask);
+        early_road_ = std::move(road);
         early_seg_start_ = std::move(seg_start_dev);
         early_vox_ = std::move(vox);
         return roots;
@@ -391,7 +395,7 @@ class Sample {
     // before any soma painting: they serve the floods too unless a soma's voids were painted.
     std::vector<long long> early_roots;
     if (root_job_.valid()) early_roots = root_job_.get();
-    const bool reuse = !any_fill && early_roots.size() == k_ && early_rec_.size() == size_t(n_);
+    const bool reuse = !any_fill && early_roots.size() == k_ && early_road_.size() != 0;
     std::vector<int> seg_start(k_ + 1, 0), seg_count(k_, 0);
     for (size_t id = 1; id < k_; ++id) seg_count[id] = int(boxes_[id].count);
     for (size_t id = 0; id < k_; ++id) seg_start[id + 1] = seg_start[id] + seg_count[id];
@@ -463,17 +467,20 @@ class Sample {
     daf_ = Buffer<float>(*cx_, size_t(n_));
     fill_value(*cx_, daf_.data(), n_, kInf);
     if (reuse) {
-      rec_ = std::move(early_rec_);  // the root searches left every word ~0
+      mask_ = std::move(early_mask_);
+      road_ = std::move(early_road_);  // the root searches left every word as it was
     } else {
-      rec_ = Buffer<VoxelRec>(*cx_, size_t(n_));  // 16 bytes per voxel: PDRF, neighbour mask + flags, distance word
-      voxel_records(*cx_, cc_.labels.data(), cc_.cc_bytes, d_, rec_.data());
+      mask_ = Buffer<unsigned>(*cx_, size_t(n_));
+      road_ = words(*cx_);
+      voxel_words(*cx_, cc_.labels.data(), cc_.cc_bytes, d_, mask_.data(), first_word(road_));
     }
-    early_rec_ = Buffer<VoxelRec>();
+    early_mask_ = Buffer<unsigned>();
+    early_road_ = Buffer<unsigned long long>();
     early_seg_start_ = Buffer<int>();
     early_vox_ = Buffer<int>();
-    if (in_.graph) {  // push masks in the records, pull masks beside them
+    if (in_.graph) {  // the masks become push masks, pull masks beside them
       inmask_ = Buffer<unsigned>(*cx_, size_t(n_));
-      graph_gates(*cx_, rec_.data(), in_.graph, d_, inmask_.data());
+      graph_gates(*cx_, mask_.data(), in_.graph, d_, inmask_.data());
     }
     // lists 2 and 3 are the railroad's far lists: two entries per voxel (trace.hip far_compact)
     for (int i = 0; i < 6; ++i) lists_.emplace_back(*cx_, size_t(std::max<int64_t>(F_, 1)) * (i == 2 || i == 3 ? 2 : 1));
@@ -576,6 +583,10 @@ class Sample {
     for (size_t id = 1; id < k_; ++id) cc_.roots[id - 1] = first[id];
   }
 
+  // Padded word arrays (common.hpp).
+  Buffer<unsigned long long> words(Context &c) const { return Buffer<unsigned long long>(c, size_t(n_ + 2 * word_pad(d_))); }
+  unsigned long long *first_word(const Buffer<unsigned long long> &b) const { return b.data() + word_pad(d_); }
+
   FloodJob flood_job() const {
     FloodJob j;
     j.d = d_;
@@ -588,7 +599,9 @@ class Sample {
     j.t.max_daf = max_daf_dev_.data();
     j.t.weights = weights_.data();
     j.t.free_radius = free_radius_dev_.size() ? free_radius_dev_.data() : nullptr;
-    j.t.rec = rec_.data();
+    j.t.mask = mask_.data();
+    j.t.road0 = road_.data();
+    j.t.road = first_word(road_);
     j.daf = daf_.data();
     j.lists_a = lists_[0].data();
     j.lists_b = lists_[1].data();
@@ -631,8 +644,10 @@ class Sample {
     use_dev.upload(*cx_, use.data(), k_);
     Buffer<float> pdrf;  // the PDRF as a volume of its own only when the fields are asked for
     if (fields_ && fields_->pdrf) pdrf = Buffer<float>(*cx_, size_t(n_));
+    claim_ = words(*cx_);
     pdrf_and_alive(*cx_, cc_.labels.data(), cc_.cc_bytes, n_, dbf_.data(), daf_.data(), M_dev.data(), inv_dev.data(),
-                   use_dev.data(), squarings, float(o_.teasar.pdrf_scale), pdrf.size() ? pdrf.data() : nullptr, rec_.data());
+                   use_dev.data(), squarings, float(o_.teasar.pdrf_scale), pdrf.size() ? pdrf.data() : nullptr, first_word(road_),
+                   first_word(claim_));
     Buffer<int> labels_dev(*cx_, std::max<size_t>(labels_.size(), 1));
     labels_dev.upload(*cx_, labels_.data(), labels_.size());
     if (fields_) {
@@ -649,7 +664,7 @@ class Sample {
       if (fields_->stop) return finish_empty();
     }
     // the root becomes a rail (lockstep.cu:183); the fix_branching=False field floods from it
-    if (o_.fix_branching) root_rails(*cx_, rec_.data(), root_dev_.data(), labels_dev.data(), int(labels_.size()));
+    if (o_.fix_branching) root_rails(*cx_, first_word(road_), root_dev_.data(), labels_dev.data(), int(labels_.size()));
     const size_t fl = size_t(std::max<int64_t>(F_, 1));
     order_ = Buffer<int>(*cx_, fl);
     snap_a_ = Buffer<unsigned long long>(*cx_, fl);
@@ -723,7 +738,13 @@ class Sample {
   TraceArgs trace_args() const {
     TraceArgs ta;
     ta.d = d_;
-    ta.rec = rec_.data();
+    ta.by_row = fast_div(unsigned(d_.sx));
+    ta.by_plane = fast_div(unsigned(d_.sx) * unsigned(d_.sy));
+    ta.mask = mask_.data();
+    ta.road0 = road_.data();
+    ta.road = first_word(road_);
+    ta.claim0 = claim_.data();
+    ta.claim = first_word(claim_);
     ta.dbf = dbf_.data();
     ta.seg_start = seg_start_dev_.data();
     ta.seg_count = seg_count_dev_.data();
@@ -994,7 +1015,8 @@ class Sample {
   std::future<std::vector<std::vector<Point>>> border_job_;
   // The early root searches: the records and voxel lists they built, and per id the root found, or
   // -1 (written by the job, read after joining it).
-  Buffer<VoxelRec> early_rec_;
+  Buffer<unsigned> early_mask_;
+  Buffer<unsigned long long> early_road_;
   Buffer<int> early_seg_start_, early_vox_;
   std::future<std::vector<long long>> root_job_;
   LabelVolume in_;
@@ -1021,7 +1043,8 @@ class Sample {
   Buffer<float> dbf_, daf_, weights_, max_daf_dev_;
   Buffer<int> seg_start_dev_, vox_, seg_count_dev_;
   Buffer<long long> first_dev_, root_dev_, target_dev_;
-  Buffer<VoxelRec> rec_;
+  Buffer<unsigned> mask_;             // neighbour masks (common.hpp)
+  Buffer<unsigned long long> road_, claim_;  // road and claim words
   Buffer<unsigned> inmask_;  // voxel graph: pull masks (empty: no graph)
   std::vector<Buffer<int>> lists_;
   Buffer<int> order_;

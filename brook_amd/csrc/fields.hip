@@ -9,6 +9,7 @@
 #include <cmath>
 
 #include "fields.hpp"
+#include "front.hpp"
 #include "tuned.hpp"
 
 namespace brook {
@@ -63,14 +64,15 @@ __global__ void __launch_bounds__(256) fill_segments(const CC *cc, int n, Dims d
   }
 }
 
-// Voxel records: the neighbour mask (bit k = neighbour k of v is inside the volume and has v's
-// nonzero id; every later neighbour walk reads this instead of 26 ids and bounds checks),
-// PDRF +inf, word ~0. A workgroup covers a kRecX x kRecY x kRecZ box: its ids and a one-voxel
-// halo (0 outside the volume, which never equals an id) are staged in LDS by coalesced row loads,
-// the 26 comparisons of a voxel read LDS, and each wave stores one row of 64 records contiguously.
+// Voxel words: the neighbour mask (bit k = neighbour k of v is inside the volume and has v's nonzero
+// id; every later neighbour walk reads this instead of 26 ids and bounds checks), and road words
+// kFloodFree where a label is. A workgroup covers a kRecX x kRecY x kRecZ box: its ids and a one-voxel halo (0
+// outside the volume, which never equals an id) are staged in LDS by coalesced row loads, the 26
+// comparisons of a voxel read LDS, and each wave stores a row of 64 words of each array. Bound by
+// the 12 bytes per foreground voxel and 4 per background one that it writes.
 constexpr int kRecX = 64, kRecY = 4, kRecZ = 4;
 template <class CC>
-__global__ void __launch_bounds__(256) init_records(const CC *cc, Dims d, VoxelRec *rec) {
+__global__ void __launch_bounds__(256) init_words(const CC *cc, Dims d, unsigned *mask, unsigned long long *road) {
   constexpr int TX = kRecX + 2, TY = kRecY + 2, TZ = kRecZ + 2;
   __shared__ CC tile[TZ][TY][TX];
   const int bx = int(blockIdx.x) * kRecX, by = int(blockIdx.y) * kRecY, bz = int(blockIdx.z) * kRecZ;
@@ -95,11 +97,9 @@ __global__ void __launch_bounds__(256) init_records(const CC *cc, Dims d, VoxelR
         if (tile[tz + 1 + kDZ[k]][ty + 1 + kDY[k]][tx + 1 + kDX[k]] == l) m |= 1u << k;
       });
     }
-    VoxelRec r;
-    r.pdrf = kInf;
-    r.meta = m;
-    r.word = kMaxKey;
-    rec[x + (long long)d.sx * (y + (long long)d.sy * (bz + tz))] = r;
+    const long long at = x + (long long)d.sx * (y + (long long)d.sy * (bz + tz));
+    mask[at] = m;
+    if (l != CC(0)) road[at] = kFloodFree;
   }
 }
 
@@ -109,365 +109,211 @@ __global__ void fill_float(float *p, long long n, float v) {
 }
 
 constexpr int kFloodBlock = BROOK_FLOOD_BLOCK;  // threads per label workgroup
-// Near-far bands in the floods (see flood_bands); the band width is BROOK_FLOOD_BAND times the
-// longest step.
-#ifndef BROOK_FLOOD_NEARFAR
-#define BROOK_FLOOD_NEARFAR 1
-#endif
+constexpr int kFloodWaves = kFloodBlock / 64;
+constexpr int kFloodPairs = BROOK_FLOOD_NB_BATCH;
+// The band width is BROOK_FLOOD_BAND times the longest step.
 #ifndef BROOK_FLOOD_BAND
 #define BROOK_FLOOD_BAND 2.0f
 #endif
-constexpr int kFloodBatch = BROOK_FLOOD_NB_BATCH;  // neighbours in flight per thread
 
-// Relaxes masked neighbours B..E-1 of u (distance du): all loads, then all atomics, in flight
-// together. Returns the neighbours this thread must queue (improved and found not queued).
-template <int B, int E>
-__device__ __forceinline__ unsigned flood_part(VoxelRec *rec, Dims d, int u, unsigned m, float du, const float *W) {
-  unsigned seen[E - B];
-  for_nb<B, E>([&](auto K) {
-    constexpr int k = decltype(K)::value, i = k - B;
-    seen[i] = (m >> k) & 1u ? rec_word_hi(rec, u + nb_offset<k>(d)) : 0u;
-  });
-  unsigned long long old[E - B];
-  for_nb<B, E>([&](auto K) {
-    constexpr int k = decltype(K)::value, i = k - B;
-    const unsigned cb = __float_as_uint(du + W[k]);
-    old[i] = 0;
-    if (cb < seen[i]) old[i] = g_min(&rec[u + nb_offset<k>(d)].word, (unsigned long long)cb << 32);
-  });
-  unsigned push = 0;
-  for_nb<B, E>([&](auto K) {
-    constexpr int k = decltype(K)::value, i = k - B;
-    const unsigned cb = __float_as_uint(du + W[k]);
-    if ((old[i] & 1ULL) && old[i] > ((unsigned long long)cb << 32)) push |= 1u << k;
-  });
-  return push;
-}
-
-// Neighbours kb..kb+cnt-1 (those set in m; cnt <= kSpan) of u: flood_part with a run-time span.
-__device__ __forceinline__ unsigned flood_span(VoxelRec *rec, int u, unsigned m, int kb, int cnt, float du, const float *W,
-                                               const int *off) {
-  constexpr int S = kSpan;
-  unsigned seen[S];
-  int v[S];
-#pragma unroll
-  for (int j = 0; j < S; ++j) {
-    const bool on = j < cnt && ((m >> (kb + j)) & 1u);
-    v[j] = u + off[on ? kb + j : 0];
-    seen[j] = on ? rec_word_hi(rec, v[j]) : 0u;
-  }
-  unsigned long long old[S];
-#pragma unroll
-  for (int j = 0; j < S; ++j) {
-    const unsigned cb = __float_as_uint(du + W[j < cnt ? kb + j : 0]);
-    old[j] = 0;
-    if (cb < seen[j]) old[j] = g_min(&rec[v[j]].word, (unsigned long long)cb << 32);
-  }
-  unsigned push = 0;
-#pragma unroll
-  for (int j = 0; j < S; ++j) {
-    const unsigned cb = __float_as_uint(du + W[j < cnt ? kb + j : 0]);
-    if ((old[j] & 1ULL) && old[j] > ((unsigned long long)cb << 32)) push |= 1u << (kb + j);
-  }
-  return push;
-}
-
-// Geometric flood of one label from one source inside one workgroup, on the records' packed words
-// (distance bits high, "not queued" bit 0 low; ~0 = +inf, not queued). Words of the label must be
-// ~0 on entry; on exit they hold the distances, every voxel dequeued (bit 0 set).
-// Label-correcting rounds: a voxel is dequeued by one atomic that also returns its distance, and
-// an improvement that finds the voxel not queued queues it, so no update is ever lost.
-// The front's words hold their start distances (queued) on entry; counts[0] is its length.
-// Returns false when the rounds exceed `budget` (far above what the label-correcting rounds need:
-// a logic error then ends as a host-visible error instead of a hang).
-__device__ __forceinline__ bool flood_rounds(VoxelRec *rec, Dims d, const float *W, const int *off, int *cur, int *nxt,
-                                             int *counts /*LDS [2]*/, long long budget) {
-  for (long long round = 0;; ++round) {
-    const int nc = counts[0];
-    if (nc == 0) break;
-    if (round >= budget) return false;  // uniform: counts[0] and round are the same in every thread
-    if (nc <= kFloodBlock / 4) {  // a group of lanes per front voxel; its first lane dequeues
-      const Group q = group_of(nc, kFloodBlock);
-      int u = 0;
-      unsigned m = 0;
-      float du = 0.0f;
-      if (q.g == 0 && q.i < nc) {
-        u = lp_i(cur + q.i);
-        m = rec_meta(rec, u) & kNbrBits;
-        du = __uint_as_float((unsigned)(g_or(&rec[u].word, 1ULL) >> 32));
-      }
-      u = __shfl(u, q.lead, 64);
-      m = __shfl(m, q.lead, 64);
-      du = __shfl(du, q.lead, 64);
-      const unsigned push = q.i < nc ? flood_span(rec, u, m, q.kb, q.cnt, du, W, off) : 0u;
-      emit_neighbours(nxt, &counts[1], push, u, off);
-    } else {
-      for (int base = 0; base < nc; base += blockDim.x) {  // uniform: every lane reaches the append
-        const int i = base + threadIdx.x;
-        unsigned push = 0;
-        int u = 0;
-        if (i < nc) {
-          u = lp_i(cur + i);
-          const unsigned m = rec_meta(rec, u) & kNbrBits;
-          const float du = __uint_as_float((unsigned)(g_or(&rec[u].word, 1ULL) >> 32));
-          for_parts<kFloodBatch>(m, [&](auto B, auto E) {
-            push |= flood_part<decltype(B)::value, decltype(E)::value>(rec, d, u, m, du, W);
-          });
-        }
-        emit_neighbours(nxt, &counts[1], push, u, off);
-      }
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) { counts[0] = counts[1]; counts[1] = 0; }
-    int *t = cur; cur = nxt; nxt = t;
-    __syncthreads();
-  }
-  return true;
-}
-
-// Rounds one flood of a label of `count` voxels may take (see flood_rounds).
+// Rounds one flood of a label of `count` voxels may take (see flood_front).
 __device__ __forceinline__ long long flood_budget(int count) { return 4LL * count + 4096; }
 
 // ---- near-far bands -------------------------------------------------------------------------
-// The same fixpoint, with the label-correcting rounds kept inside a distance band [.., T]: an
+// The geometric flood of a label: label-correcting rounds kept inside a distance band [.., T]. An
 // improvement beyond T goes to a far list instead of the next round, and when the band has no
 // front left, T moves to the nearest far distance plus the band width and the far voxels inside
 // it start the next band. A voxel is then relaxed about once instead of re-queued each time a
 // cheaper path with more steps arrives (30 % of pops on the 512^3 workload with anisotropy
-// (8, 8, 40)). Word bits as the railroad's: bit 0 "not queued", bit 1 "far listed"; near
-// candidates store 00 (queued), far candidates 11; a near improvement of a far-listed voxel
-// clears its far bit (its far entry goes stale). Far lists hold 2 * count entries (one append per
+// (8, 8, 40)). The words are the railroad's (common.hpp) with a constant cost field (all ones):
+// near candidates are queued, far candidates far-listed; a near improvement of a far-listed voxel
+// clears its far flag (its far entry goes stale). Far lists hold 2 * count entries (one append per
 // voxel per round; a list longer than count after a round is compacted to one entry per voxel).
+constexpr int kFloodFront = 4096, kFloodFar = 2048;  // entries of the lists that live in LDS
+using NearList = SplitList<kFloodFront>;
+using FarList = SplitList<kFloodFar>;
+// n[0..2]: front lengths, rotating (round r reads n[r], appends to n[r+1], clears n[r+2]: one barrier
+// per round); n[kFar0], n[kFar1]: far list lengths; n[kNone]: not appended to.
+constexpr int kFar0 = 3, kFar1 = 4, kNone = 5;
+constexpr int kLong = 1, kFull = 2;  // flags of a round's far list, rotating: above count, at its end
 struct FloodShared {
-  int near[2];          // front lengths: current, next
-  int n_far, n_farnxt;  // far list lengths
-  unsigned minfar;      // smallest far distance (float bits) since the band moved
-  float T;              // the band's upper end
-  int overflow;         // a far append found the list full (never expected)
+  int n[6], flags[3];
+  unsigned minfar;  // smallest far distance (float bits) since the band moved
+  float T;          // the band's upper end
+  int near[2][kFloodFront], far[2][kFloodFar];
+  Stage stage[kFloodWaves];
 };
 
-__device__ __forceinline__ bool flood_far_listed(unsigned long long w) {
-  return (w & 2ULL) && (unsigned)(w >> 32) != 0xFFFFFFFFu;
-}
+struct FloodLists {
+  NearList near[2];
+  FarList far[2];
+};
 
-// Masked neighbours B..E-1 of u: the near and far masks to append, the smallest far distance.
-template <int B, int E>
-__device__ __forceinline__ void band_part(VoxelRec *rec, Dims d, int u, unsigned m, float du, const float *W, float T,
-                                          unsigned &near, unsigned &far, unsigned &minfar) {
-  unsigned seen[E - B];
-  for_nb<B, E>([&](auto K) {
-    constexpr int k = decltype(K)::value, i = k - B;
-    seen[i] = (m >> k) & 1u ? rec_word_hi(rec, u + nb_offset<k>(d)) : 0u;
-  });
-  unsigned long long old[E - B];
-  for_nb<B, E>([&](auto K) {
-    constexpr int k = decltype(K)::value, i = k - B;
-    const float c = du + W[k];
-    const unsigned cb = __float_as_uint(c);
-    old[i] = 0;
-    if (cb < seen[i]) old[i] = g_min(&rec[u + nb_offset<k>(d)].word, ((unsigned long long)cb << 32) | (c <= T ? 0ULL : 3ULL));
-  });
-  for_nb<B, E>([&](auto K) {
-    constexpr int k = decltype(K)::value, i = k - B;
-    const float c = du + W[k];
-    const unsigned cb = __float_as_uint(c);
-    const bool in = c <= T;
-    if (!(old[i] > (((unsigned long long)cb << 32) | (in ? 0ULL : 3ULL)))) return;
-    if (in) {
-      if (old[i] & 1ULL) near |= 1u << k;
-    } else {
-      minfar = min(minfar, cb);
-      if (!flood_far_listed(old[i])) far |= 1u << k;
-    }
-  });
-}
-
-// Neighbours kb..kb+cnt-1 (those set in m; cnt <= kSpan) of u: band_part with a run-time span.
-__device__ __forceinline__ void band_span(VoxelRec *rec, int u, unsigned m, int kb, int cnt, float du, const float *W,
-                                          const int *off, float T, unsigned &near, unsigned &far, unsigned &minfar) {
-  constexpr int S = kSpan;
-  unsigned seen[S];
-  int v[S];
-#pragma unroll
-  for (int j = 0; j < S; ++j) {
-    const bool on = j < cnt && ((m >> (kb + j)) & 1u);
-    v[j] = u + off[on ? kb + j : 0];
-    seen[j] = on ? rec_word_hi(rec, v[j]) : 0u;
-  }
-  unsigned long long old[S];
-#pragma unroll
-  for (int j = 0; j < S; ++j) {
-    const float c = du + W[j < cnt ? kb + j : 0];
-    const unsigned cb = __float_as_uint(c);
-    old[j] = 0;
-    if (cb < seen[j]) old[j] = g_min(&rec[v[j]].word, ((unsigned long long)cb << 32) | (c <= T ? 0ULL : 3ULL));
+// Front entries b .. of one round over nc entries, at most 2P (the wave's batch): the neighbours whose
+// distance they improve go to the wave's stage. W is the lane's step weight, T the band's end.
+template <int P, bool Wide, class Flush>
+__device__ __forceinline__ void flood_batch(const LabelTables &t, const Lane<Wide> &ln, float W, const NearList &cur, int b,
+                                            int nc, unsigned T, Stage &st, int &staged, Flush &&flush) {
+  int u[P];
+  const int ue = batch_entries<P>(ln, cur, b, nc, u);
+  unsigned long long q = 0;
+  unsigned me = 0, hi[P];
+  if (ln.lane < min(2 * P, nc - b)) {  // lane e: entry e's distance by the dequeue, and its mask
+    q = g_or(t.road + ue, kNotQueued);
+    me = g_ld(t.mask + ue);
   }
 #pragma unroll
-  for (int j = 0; j < S; ++j) {
-    const float c = du + W[j < cnt ? kb + j : 0];
-    const unsigned cb = __float_as_uint(c);
-    const bool in = c <= T;
-    if (!(old[j] > (((unsigned long long)cb << 32) | (in ? 0ULL : 3ULL)))) continue;
-    if (in) {
-      if (old[j] & 1ULL) near |= 1u << (kb + j);
-    } else {
-      minfar = min(minfar, cb);
-      if (!flood_far_listed(old[j])) far |= 1u << (kb + j);
-    }
-  }
+  for (int p = 0; p < P; ++p) hi[p] = g_ld(reinterpret_cast<const unsigned *>(word_at(t.road0, ln.at(u[p]))) + 1);
+  const unsigned de = road_dist(q);
+  staged_pairs<P>([&](int p) {
+    const unsigned m = of_entry(ln, me, 2 * p);
+    const unsigned c = __float_as_uint(__uint_as_float(of_entry(ln, de, 2 * p)) + W);
+    const bool later = c > T;
+    const unsigned nhi = (c << 1) | unsigned(later);
+    stage_put(st, staged, ((m & ln.bit) != 0u) & ((nhi | 1u) < hi[p]), u[p] + ln.off,
+              ((unsigned long long)nhi << 32) | (later ? ~0u : kCostBits));
+  }, flush);
 }
 
-__device__ __forceinline__ void fold_minfar(FloodShared &fs, unsigned m) {
-  for (int o = 32; o > 0; o >>= 1) m = min(m, (unsigned)__shfl_xor((int)m, o, 64));
-  if (__lane_id() == 0 && m != 0x7f800000u) atomicMin(&fs.minfar, m);
+// The staged improvements of a wave (full groups, or all of them).
+__device__ __forceinline__ void flood_minima(const LabelTables &t, FloodShared &fs, Stage &st, int &staged, bool all,
+                                             const NearList &nxt, int n_nxt, const FarList &far, int n_far, int count,
+                                             unsigned &minfar) {
+  stage_take(st, staged, all, [&](bool on, int v, unsigned long long nv) {
+    unsigned long long old = 0;  // "nothing changed" unless the atomic says otherwise
+    if (on) old = g_min(t.road + v, nv);
+    const bool won = old > nv, later = nv & kFarListed;
+    const bool near = won & !later & (int(unsigned(old)) < 0), fars = won & later & !(old & kFarListed);
+    if (won & later) minfar = min(minfar, road_dist(nv));
+    Appends out;
+    if (!out.begin(fs.n, kNone, false, n_nxt, near, n_far, fars)) return;
+    const int end = out.at[2] + out.count(2);
+    const bool full = end > 2 * count;  // a wave whose appends would pass the far list's end writes none
+    if (out.set[2] && end > count) atomicOr(&fs.flags[n_nxt], full ? kLong | kFull : kLong);
+    if (near) nxt.put(out.place(1), v);
+    if (fars & !full) far.put(out.place(2), v);
+  });
 }
 
-// Appends u + off[k] for every set bit k of mask to a list of `cap` entries (all lanes active);
-// a wave whose appends would pass the end writes nothing and raises `overflow`.
-__device__ __forceinline__ void emit_capped_list(int *list, int *counter, unsigned mask, int u, const int *off, int cap,
-                                                 int *overflow) {
-  const int n = __popc(mask);
-  int pos = wave_reserve(counter, n);
-  if (pos + n > cap) {
-    if (n) *overflow = 1;
-    return;
+__device__ __forceinline__ void fold_minfar(FloodShared &fs, unsigned &m) {
+  if (any_lane(m != kInfBits)) {
+    m = wave_min_u32(m);
+    if (__lane_id() == 0) atomicMin(&fs.minfar, m);
   }
-  while (mask) {
-    const int k = __ffs(mask) - 1;
-    mask &= mask - 1;
-    g_st(list + pos++, u + off[k]);
-  }
+  m = kInfBits;
 }
 
-// The near list `cur` (fs.near[0] queued entries) starts the flood; far lists hold 2 * count.
-__device__ __forceinline__ bool flood_bands(VoxelRec *rec, Dims d, const float *W, const int *off, int *cur, int *nxt,
-                                            int *fcur, int *fnxt, FloodShared &fs, int count, long long budget) {
+// The near list l.near[0] (fs.n[0] entries, whose words hold their start distances, queued; the other
+// counters and flags 0) starts the flood. Words of the label are kFloodFree on entry but for these; on exit
+// they hold the distances, every voxel dequeued. Returns false when the rounds exceed their budget
+// (far above what the label-correcting rounds need: a logic error then ends as a host-visible error
+// instead of a hang) or a far list its end.
+template <bool Wide>
+__device__ __forceinline__ bool flood_front(const LabelTables &t, const Lane<Wide> &ln, const float *W, const FloodLists &l,
+                                            FloodShared &fs, int count) {
+  const long long budget = flood_budget(count);
   float wmax = 0.0f;
   for (int k = 0; k < 26; ++k) wmax = fmaxf(wmax, W[k]);
-  const float width = BROOK_FLOOD_BAND * wmax;
+  const float width = BROOK_FLOOD_BAND * wmax, weight = W[ln.k];
+  Stage &st = fs.stage[ln.wave];
+  NearList cur = l.near[0], nxt = l.near[1];
+  FarList fcur = l.far[0], fnxt = l.far[1];
+  int fc = kFar0, fn = kFar1, r = 0;
+  auto swap_far = [&] {
+    const FarList f = fcur; fcur = fnxt; fnxt = f;
+    const int n = fc; fc = fn; fn = n;
+  };
   if (threadIdx.x == 0) {
-    fs.near[1] = fs.n_far = fs.n_farnxt = fs.overflow = 0;
     fs.minfar = 0x7f800000u;
     fs.T = width;
   }
   __syncthreads();
+  unsigned minfar = 0x7f800000u;
   long long rounds = 0;
   for (;;) {
-    for (;;) {  // the band's rounds
-      const int nc = fs.near[0];
+    const unsigned T = unsigned(__builtin_amdgcn_readfirstlane(__float_as_int(fs.T)));  // moved between two barriers below
+    for (;;) {             // the band's rounds
+      const int nc = __builtin_amdgcn_readfirstlane(fs.n[r]);
       if (nc == 0) break;
-      if (++rounds > budget || fs.overflow) return false;  // uniform: read after the round's barrier
-      const float T = fs.T;
-      unsigned minfar = 0x7f800000u;
-      if (nc <= kFloodBlock / 4) {  // a group of lanes per front voxel; its first lane dequeues
-        const Group q = group_of(nc, kFloodBlock);
-        int u = 0;
-        unsigned m = 0;
-        float du = 0.0f;
-        if (q.g == 0 && q.i < nc) {
-          u = lp_i(cur + q.i);
-          m = rec_meta(rec, u) & kNbrBits;
-          du = __uint_as_float((unsigned)(g_or(&rec[u].word, 1ULL) >> 32));
-        }
-        u = __shfl(u, q.lead, 64);
-        m = __shfl(m, q.lead, 64);
-        du = __shfl(du, q.lead, 64);
-        unsigned near = 0, far = 0;
-        if (q.i < nc) band_span(rec, u, m, q.kb, q.cnt, du, W, off, T, near, far, minfar);
-        emit_neighbours(nxt, &fs.near[1], near, u, off);
-        emit_capped_list(fcur, &fs.n_far, far, u, off, 2 * count, &fs.overflow);
-      } else {
-        for (int base = 0; base < nc; base += blockDim.x) {  // uniform: every lane reaches the appends
-          const int i = base + threadIdx.x;
-          unsigned near = 0, far = 0;
-          int u = 0;
-          if (i < nc) {
-            u = lp_i(cur + i);
-            const unsigned m = rec_meta(rec, u) & kNbrBits;
-            const float du = __uint_as_float((unsigned)(g_or(&rec[u].word, 1ULL) >> 32));
-            for_parts<kFloodBatch>(m, [&](auto B, auto E) {
-              band_part<decltype(B)::value, decltype(E)::value>(rec, d, u, m, du, W, T, near, far, minfar);
-            });
-          }
-          emit_neighbours(nxt, &fs.near[1], near, u, off);
-          emit_capped_list(fcur, &fs.n_far, far, u, off, 2 * count, &fs.overflow);
-        }
-      }
+      if (++rounds > budget) return false;  // uniform
+      const int rn = rot_next(r);
+      if (threadIdx.x == 0) fs.n[rot_prev(r)] = fs.flags[rot_prev(r)] = 0;
+      int staged = 0;
+      with_pairs<kFloodPairs>(nc, kFloodWaves, [&](auto Pairs) {
+        constexpr int P = decltype(Pairs)::value;
+        for (int b = ln.wave * 2 * P; b < nc; b += kFloodWaves * 2 * P)
+          flood_batch<P>(t, ln, weight, cur, b, nc, T, st, staged,
+                         [&] { flood_minima(t, fs, st, staged, false, nxt, rn, fcur, fc, count, minfar); });
+      });
+      flood_minima(t, fs, st, staged, true, nxt, rn, fcur, fc, count, minfar);
       fold_minfar(fs, minfar);
       __syncthreads();
-      if (threadIdx.x == 0) { fs.near[0] = fs.near[1]; fs.near[1] = 0; }
-      int *t = cur; cur = nxt; nxt = t;
-      __syncthreads();
-      if (fs.n_far > count) {  // one entry per far-listed voxel (the one whose atomic clears its far bit)
-        const int nf = fs.n_far;
+      r = rn;
+      const NearList f = cur; cur = nxt; nxt = f;
+      const int flags = fs.flags[r];
+      if (flags & kFull) return false;
+      if (flags & kLong) {  // one entry per far-listed voxel (the one whose atomic clears its far flag)
+        const int nf = fs.n[fc];
         for (int i = threadIdx.x; i < nf; i += blockDim.x) {
-          const int w = lp_i(fcur + i);
-          if (flood_far_listed(g_and(&rec[w].word, ~2ULL))) g_st(fnxt + wave_slot(&fs.n_farnxt), w);
+          const int w = fcur.get(i);
+          if (g_and(t.road + w, ~kFarListed) & kFarListed) fnxt.put(wave_slot(&fs.n[fn]), w);
         }
         __syncthreads();
-        const int kept = fs.n_farnxt;
-        for (int i = threadIdx.x; i < kept; i += blockDim.x) g_or(&rec[lp_i(fnxt + i)].word, 2ULL);
+        const int kept = fs.n[fn];
+        for (int i = threadIdx.x; i < kept; i += blockDim.x) g_or(t.road + fnxt.get(i), kFarListed);
+        if (threadIdx.x == 0) fs.n[fc] = 0;
         __syncthreads();
-        if (threadIdx.x == 0) { fs.n_far = kept; fs.n_farnxt = 0; }
-        int *tf = fcur; fcur = fnxt; fnxt = tf;
-        __syncthreads();
+        swap_far();
       }
     }
-    const int nf = fs.n_far;
+    const int nf = fs.n[fc];
     if (nf == 0) return true;
-    if (++rounds > budget || fs.overflow) return false;
+    if (++rounds > budget) return false;
+    const float next = __uint_as_float(fs.minfar) + width;  // the band moves to the nearest far distance
     __syncthreads();
-    if (threadIdx.x == 0) {  // the band moves to the nearest far distance
-      fs.T = __uint_as_float(fs.minfar) + width;
+    if (threadIdx.x == 0) {
+      fs.T = next;
       fs.minfar = 0x7f800000u;
     }
     __syncthreads();
-    const float T = fs.T;
-    unsigned minfar = 0x7f800000u;
     for (int i = threadIdx.x; i < nf; i += blockDim.x) {  // far voxels inside the band start it
-      const int w = lp_i(fcur + i);
-      if (!flood_far_listed(lp_u64(&rec[w].word))) continue;
-      const unsigned long long was = g_and(&rec[w].word, ~3ULL);
-      if (!flood_far_listed(was)) continue;
-      const float dw = __uint_as_float((unsigned)(was >> 32));
-      if (dw <= T) {
-        g_st(cur + wave_slot(&fs.near[0]), w);
+      const int w = fcur.get(i);
+      if (!(lp_u64(t.road + w) & kFarListed)) continue;
+      const unsigned long long was = g_and(t.road + w, ~(kFarListed | kNotQueued));
+      if (!(was & kFarListed)) continue;
+      if (__uint_as_float(road_dist(was)) <= next) {
+        cur.put(wave_slot(&fs.n[r]), w);
       } else {
-        g_or(&rec[w].word, 3ULL);
-        minfar = min(minfar, (unsigned)(was >> 32));
-        g_st(fnxt + wave_slot(&fs.n_farnxt), w);
+        g_or(t.road + w, kFarListed | kNotQueued);
+        minfar = min(minfar, road_dist(was));
+        fnxt.put(wave_slot(&fs.n[fn]), w);
       }
     }
     fold_minfar(fs, minfar);
     __syncthreads();
-    if (threadIdx.x == 0) { fs.n_far = fs.n_farnxt; fs.n_farnxt = 0; }
-    int *tf = fcur; fcur = fnxt; fnxt = tf;
-    __syncthreads();
+    if (threadIdx.x == 0) fs.n[fc] = 0;  // appended to again after two more barriers
+    swap_far();
   }
 }
 
-// The flood from the queued front `cur` (fs.near[0] entries).
-__device__ __forceinline__ bool flood_front(VoxelRec *rec, Dims d, const float *W, const int *off, int *cur, int *nxt,
-                                            int *fcur, int *fnxt, FloodShared &fs, int count) {
-#if BROOK_FLOOD_NEARFAR
-  return flood_bands(rec, d, W, off, cur, nxt, fcur, fnxt, fs, count, flood_budget(count));
-#else
-  return flood_rounds(rec, d, W, off, cur, nxt, fs.near, flood_budget(count));
-#endif
+__device__ __forceinline__ void flood_clear(FloodShared &fs) {
+  if (threadIdx.x < 6) fs.n[threadIdx.x] = 0;
+  if (threadIdx.x < 3) fs.flags[threadIdx.x] = 0;
 }
 
-__device__ __forceinline__ bool flood_label(VoxelRec *rec, Dims d, int src, const float *W, const int *off, int *cur,
-                                            int *nxt, int *fcur, int *fnxt, FloodShared &fs, int count) {
+template <bool Wide>
+__device__ __forceinline__ bool flood_label(const LabelTables &t, const Lane<Wide> &ln, int src, const float *W,
+                                            const FloodLists &l, FloodShared &fs, int count) {
+  flood_clear(fs);
+  __syncthreads();
   if (threadIdx.x == 0) {
-    sp_u64(&rec[src].word, 0ULL);  // distance 0, queued
-    g_st(cur, src);
-    fs.near[0] = 1;
-    fs.near[1] = 0;
+    sp_u64(t.road + src, road_word(0u, 0ULL, kCostBits));  // distance 0, queued
+    l.near[0].put(0, src);
+    fs.n[0] = 1;
   }
   __syncthreads();
-  return flood_front(rec, d, W, off, cur, nxt, fcur, fnxt, fs, count);
+  return flood_front(t, ln, W, l, fs, count);
 }
-
 
 // The free-space length of a soma voxel at offset (dxi, dyi, dzi) from the root, when its physical
 // distance is within `radius`: the shortest 26-connected path through empty space, in float32 in
@@ -486,10 +332,10 @@ __device__ __forceinline__ bool free_space(int dxi, int dyi, int dzi, float wx, 
 
 // A soma's DAF flood (batched.cu:222-231): every voxel of the label inside the free-space ball
 // starts at its free-space length (the root at 0), then the label-correcting rounds.
-__device__ __forceinline__ bool flood_free_space(VoxelRec *rec, Dims d, const int *list, int cnt, int root, float radius,
-                                                 const float *W, const int *off, int *cur, int *nxt, int *fcur, int *fnxt,
-                                                 FloodShared &fs) {
-  if (threadIdx.x == 0) { fs.near[0] = 0; fs.near[1] = 0; }
+template <bool Wide>
+__device__ __forceinline__ bool flood_free_space(const LabelTables &t, Dims d, const Lane<Wide> &ln, const int *list, int cnt, int root,
+                                                 float radius, const float *W, const FloodLists &l, FloodShared &fs) {
+  flood_clear(fs);
   __syncthreads();
   int rx, ry, rz;
   unravel(root, d, rx, ry, rz);
@@ -499,22 +345,23 @@ __device__ __forceinline__ bool flood_free_space(VoxelRec *rec, Dims d, const in
     unravel(v, d, x, y, z);
     float val;
     if (!free_space(x - rx, y - ry, z - rz, W[0], W[2], W[4], radius, val)) continue;
-    sp_u64(&rec[v].word, (unsigned long long)__float_as_uint(val) << 32);  // queued
-    g_st(cur + wave_slot(&fs.near[0]), v);
+    sp_u64(t.road + v, road_word(__float_as_uint(val), 0ULL, kCostBits));  // queued
+    l.near[0].put(wave_slot(&fs.n[0]), v);
   }
   __syncthreads();
-  return flood_front(rec, d, W, off, cur, nxt, fcur, fnxt, fs, cnt);
+  return flood_front(t, ln, W, l, fs, cnt);
 }
 
 // Argmax of the flooded distance over the label's voxel list: largest finite value, ties -> lowest
 // flat index (the packed key of batched_regular.inc:9-22). Returns the key (0: none).
-__device__ __forceinline__ unsigned long long label_argmax(const VoxelRec *rec, const int *list, int count, unsigned long long *lds) {
+__device__ __forceinline__ unsigned long long label_argmax(const unsigned long long *road, const int *list, int count,
+                                                           unsigned long long *lds) {
   if (threadIdx.x == 0) *lds = 0;
   __syncthreads();
   unsigned long long best = 0;
   for (int j = threadIdx.x; j < count; j += blockDim.x) {
     int v = g_ld(list + j);
-    unsigned fb = word_dist_bits(lp_u64(&rec[v].word));
+    const unsigned fb = road_dist(lp_u64(road + v));  // unreached: +inf
     if (!(fb < 0x7f800000u)) continue;
     unsigned long long key = ((unsigned long long)fb << 32) | (unsigned long long)(0xFFFFFFFFu - (unsigned)v);
     best = key > best ? key : best;
@@ -535,11 +382,11 @@ __device__ __forceinline__ unsigned long long label_argmax(const VoxelRec *rec, 
 // the start, at most the queue's length) takes item w first (workgroups go to the XCDs in turn, so
 // the largest labels start on different XCDs); every other item comes from the shared cursor,
 // from item nfixed on.
+template <bool Wide>
 __global__ void __launch_bounds__(kFloodBlock) prepare_labels(const FloodJob *__restrict__ jobs,
                                                               const int2 *__restrict__ queue, int nqueue, int nfixed,
                                                               int *next, int *stalled) {
   __shared__ float W[26];
-  __shared__ int off[26];
   __shared__ FloodShared fs;
   __shared__ unsigned long long best;
   __shared__ int item;
@@ -553,52 +400,54 @@ __global__ void __launch_bounds__(kFloodBlock) prepare_labels(const FloodJob *__
     const int L = __builtin_amdgcn_readfirstlane(q.y);
     const Dims d = job.d;
     const LabelTables &t = job.t;
-    if (threadIdx.x < 26) {
-      W[threadIdx.x] = g_ld(t.weights + threadIdx.x);
-      off[threadIdx.x] = nb_offset(int(threadIdx.x), d);
-    }
+    if (threadIdx.x < 26) W[threadIdx.x] = g_ld(t.weights + threadIdx.x);
+    const Lane<Wide> ln = lane_of<Wide>(d, kFloodBlock);
     __syncthreads();
-    const int s0 = g_ld(t.seg_start + L), cnt = g_ld(t.seg_count + L);
+    const int s0 = __builtin_amdgcn_readfirstlane(g_ld(t.seg_start + L));  // uniform: scalar registers
+    const int cnt = __builtin_amdgcn_readfirstlane(g_ld(t.seg_count + L));
     const int *list = t.vox + s0;
-    int *a = job.lists_a + s0, *b = job.lists_b + s0, *fa = job.far_a + 2LL * s0, *fb = job.far_b + 2LL * s0;
+    const FloodLists lists{{NearList{job.lists_a + s0, fs.near[0]}, NearList{job.lists_b + s0, fs.near[1]}},
+                           {FarList{job.far_a + 2LL * s0, fs.far[0]}, FarList{job.far_b + 2LL * s0, fs.far[1]}}};
     long long root = g_ld(t.root + L);
     if (root < 0) {  // no border target: flood from the component's first voxel, root = argmax
-      if (!flood_label(t.rec, d, int(g_ld(t.first + L)), W, off, a, b, fa, fb, fs, cnt)) {
+      if (!flood_label(t, ln, int(g_ld(t.first + L)), W, lists, fs, cnt)) {
         if (threadIdx.x == 0) atomicOr(stalled, 1);
         continue;
       }
-      unsigned long long key = label_argmax(t.rec, list, cnt, &best);
+      unsigned long long key = label_argmax(t.road, list, cnt, &best);
       root = key ? (long long)(0xFFFFFFFFu - (unsigned)key) : -1;
-      for (int j = threadIdx.x; j < cnt; j += blockDim.x) sp_u64(&t.rec[g_ld(list + j)].word, kMaxKey);
+      for (int j = threadIdx.x; j < cnt; j += blockDim.x) sp_u64(t.road + g_ld(list + j), kFloodFree);
       __syncthreads();
       if (threadIdx.x == 0) g_st(t.root + L, root);
       if (job.root_only) continue;
     }
     const float radius = t.free_radius ? g_ld(t.free_radius + L) : 0.0f;
-    const bool converged = radius > 0.0f ? flood_free_space(t.rec, d, list, cnt, int(root), radius, W, off, a, b, fa, fb, fs)
-                                         : flood_label(t.rec, d, int(root), W, off, a, b, fa, fb, fs, cnt);
+    const bool converged = radius > 0.0f ? flood_free_space(t, d, ln, list, cnt, int(root), radius, W, lists, fs)
+                                         : flood_label(t, ln, int(root), W, lists, fs, cnt);
     if (!converged) {
       if (threadIdx.x == 0) atomicOr(stalled, 1);
       continue;
     }
-    unsigned long long key = label_argmax(t.rec, list, cnt, &best);
+    unsigned long long key = label_argmax(t.road, list, cnt, &best);
     if (threadIdx.x == 0) {
       g_st(t.target + L, key ? (long long)(0xFFFFFFFFu - (unsigned)key) : -1LL);
       g_st(t.max_daf + L, key ? __uint_as_float((unsigned)(key >> 32)) : 0.0f);
     }
     for (int j = threadIdx.x; j < cnt; j += blockDim.x) {  // DAF out, words back to ~0
       const int v = g_ld(list + j);
-      g_st(job.daf + v, __uint_as_float(word_dist_bits(lp_u64(&t.rec[v].word))));
-      sp_u64(&t.rec[v].word, kMaxKey);
+      g_st(job.daf + v, __uint_as_float(road_dist(lp_u64(t.road + v))));
+      sp_u64(t.road + v, kFloodFree);
     }
   }
 }
 
-// PDRF (batched_regular.inc:93-108) and the alive mask in one pass. use[l] 0: not traced.
+// PDRF (batched_regular.inc:93-108), the road word that carries it and the claim word (alive) in one
+// pass. use[l] 0: not traced.
 template <class CC>
 __global__ void __launch_bounds__(256) pdrf_alive(const CC *cc, const float *dbf, const float *daf, const float *M,
                                                   const float *inv, const unsigned char *use, int squarings, float scale,
-                                                  long long n, float *pdrf, VoxelRec *rec) {
+                                                  long long n, float *pdrf, unsigned long long *road,
+                                                  unsigned long long *claim) {
   long long i = (long long)blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
   CC l = cc[i];
@@ -618,15 +467,13 @@ __global__ void __launch_bounds__(256) pdrf_alive(const CC *cc, const float *dbf
     p = p + a * inv[l];
   }
   if (pdrf) pdrf[i] = p;
-  // the record's first half (PDRF, meta) in one 8-byte load and store
-  unsigned long long *head = reinterpret_cast<unsigned long long *>(rec + i);
-  const unsigned meta = unsigned(*head >> 32) | kAlive;
-  *head = ((unsigned long long)meta << 32) | __float_as_uint(p);
+  road[i] = kUnreached | (__float_as_uint(p) & kCostBits);
+  claim[i] = kFree;
 }
 
-__global__ void set_rails(VoxelRec *rec, const long long *root, const int *labels, int count) {
+__global__ void set_rails(unsigned long long *road, const long long *root, const int *labels, int count) {
   int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < count) rec[root[labels[i]]].pdrf = 0.0f;
+  if (i < count) road[root[labels[i]]] = kUnreached;
 }
 
 unsigned grid_for(long long n) { return unsigned((n + 255) / 256); }
@@ -654,19 +501,19 @@ void build_segments(Context &ctx, const void *cc, int cc_bytes, Dims d, const st
   BROOK_LAUNCHED();
 }
 
-void voxel_records(Context &ctx, const void *cc, int cc_bytes, Dims d, VoxelRec *rec) {
+void voxel_words(Context &ctx, const void *cc, int cc_bytes, Dims d, unsigned *mask, unsigned long long *road) {
   const long long n = (long long)d.sx * d.sy * d.sz;
   if (n == 0) return;
-  KernelTimer kt(ctx, "init_records");
+  KernelTimer kt(ctx, "init_words");
   if ((d.sy + kRecY - 1) / kRecY > 65535 || (d.sz + kRecZ - 1) / kRecZ > 65535)
     throw std::invalid_argument("volume too tall for the record tiles");
   const dim3 g(unsigned((d.sx + kRecX - 1) / kRecX), unsigned((d.sy + kRecY - 1) / kRecY), unsigned((d.sz + kRecZ - 1) / kRecZ));
   if (cc_bytes == 1)
-    init_records<uint8_t><<<g, 256, 0, ctx.stream()>>>(static_cast<const uint8_t *>(cc), d, rec);
+    init_words<uint8_t><<<g, 256, 0, ctx.stream()>>>(static_cast<const uint8_t *>(cc), d, mask, road);
   else if (cc_bytes == 2)
-    init_records<uint16_t><<<g, 256, 0, ctx.stream()>>>(static_cast<const uint16_t *>(cc), d, rec);
+    init_words<uint16_t><<<g, 256, 0, ctx.stream()>>>(static_cast<const uint16_t *>(cc), d, mask, road);
   else
-    init_records<uint32_t><<<g, 256, 0, ctx.stream()>>>(static_cast<const uint32_t *>(cc), d, rec);
+    init_words<uint32_t><<<g, 256, 0, ctx.stream()>>>(static_cast<const uint32_t *>(cc), d, mask, road);
   BROOK_LAUNCHED();
 }
 
@@ -687,12 +534,14 @@ void prepare_fields(Context &ctx, const std::vector<FloodJob> &jobs, const std::
   Buffer<int> next(ctx, 2);  // [0] queue cursor, [1] stalled
   next.clear(ctx);
   const int nq = int(q.size());
+  bool wide = false;  // one launch serves every sample of the group
+  for (const FloodJob &j : jobs) wide |= !narrow_words(j.d);
   // every workgroup takes labels from the queue until it is spent, so any grid drains it
   int grid = std::min(nq, BROOK_FLOOD_GRID > 0 ? BROOK_FLOOD_GRID : ctx.compute_units() * 2);
   if (max_grid > 0) grid = std::min(grid, max_grid);
   {
     KernelTimer kt(ctx, "prepare_labels");
-    prepare_labels<<<grid, kFloodBlock, 0, ctx.stream()>>>(jobs_dev.data(), queue.data(), nq,
+    (wide ? prepare_labels<true> : prepare_labels<false>)<<<grid, kFloodBlock, 0, ctx.stream()>>>(jobs_dev.data(), queue.data(), nq,
                                                            std::min(grid, ctx.compute_units()), next.data(),
                                                            next.data() + 1);
     BROOK_LAUNCHED();
@@ -702,23 +551,26 @@ void prepare_fields(Context &ctx, const std::vector<FloodJob> &jobs, const std::
 
 void pdrf_and_alive(Context &ctx, const void *cc, int cc_bytes, long long n, const float *dbf, const float *daf,
                     const float *M, const float *inv, const unsigned char *use, int squarings, float scale, float *pdrf,
-                    VoxelRec *rec) {
+                    unsigned long long *road, unsigned long long *claim) {
   KernelTimer kt(ctx, "pdrf_alive");
   if (cc_bytes == 1)
     pdrf_alive<uint8_t><<<grid_for(n), 256, 0, ctx.stream()>>>(static_cast<const uint8_t *>(cc), dbf, daf, M, inv, use,
-                                                               squarings, scale, n, pdrf, rec);
+                                                               squarings, scale, n, pdrf, road,
+                                                               claim);
   else if (cc_bytes == 2)
     pdrf_alive<uint16_t><<<grid_for(n), 256, 0, ctx.stream()>>>(static_cast<const uint16_t *>(cc), dbf, daf, M, inv, use,
-                                                                squarings, scale, n, pdrf, rec);
+                                                                squarings, scale, n, pdrf, road,
+                                                               claim);
   else
     pdrf_alive<uint32_t><<<grid_for(n), 256, 0, ctx.stream()>>>(static_cast<const uint32_t *>(cc), dbf, daf, M, inv, use,
-                                                                squarings, scale, n, pdrf, rec);
+                                                                squarings, scale, n, pdrf, road,
+                                                               claim);
   BROOK_LAUNCHED();
 }
 
-void root_rails(Context &ctx, VoxelRec *rec, const long long *root, const int *labels, int count) {
+void root_rails(Context &ctx, unsigned long long *road, const long long *root, const int *labels, int count) {
   if (!count) return;
-  set_rails<<<grid_for(count), 256, 0, ctx.stream()>>>(rec, root, labels, count);
+  set_rails<<<grid_for(count), 256, 0, ctx.stream()>>>(road, root, labels, count);
   BROOK_LAUNCHED();
 }
 

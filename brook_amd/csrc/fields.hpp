@@ -19,17 +19,18 @@ struct LabelTables {
   // > 0: the id is a soma; its DAF flood starts from the free-space ball of this radius around
   // the root (null: no somata)
   const float *free_radius = nullptr;
-  VoxelRec *rec = nullptr;         // voxel records (masks in; words ~0 in and out)
+  const unsigned *mask = nullptr;      // neighbour masks
+  unsigned long long *road = nullptr, *road0 = nullptr;  // road words (kFloodFree in and out) and their first pad word
 };
 
-// rec[v]: neighbour mask (bit k = neighbour k of v is inside the volume and has v's nonzero id),
-// PDRF +inf, word ~0, no flags.
-void voxel_records(Context &ctx, const void *cc, int cc_bytes, Dims d, VoxelRec *rec);
+// mask[v]: bit k = neighbour k of v is inside the volume and has v's nonzero id; road[v] = kFloodFree
+// on the foreground (background words are left as they are: no mask bit leads to one).
+void voxel_words(Context &ctx, const void *cc, int cc_bytes, Dims d, unsigned *mask, unsigned long long *road);
 
 void build_segments(Context &ctx, const void *cc, int cc_bytes, Dims d, const std::vector<int> &seg_start,
                     Buffer<int> &seg_start_dev, Buffer<int> &vox);
 void fill_value(Context &ctx, float *p, long long n, float v);
-// One sample's flood inputs: t.rec words ~0 in and out; daf receives the DAF on the traced ids'
+// One sample's flood inputs: t.road kFloodFree in and out; daf receives the DAF on the traced ids'
 // voxels; lists_*: scratch in segment layout.
 struct FloodJob {
   Dims d{0, 0, 0};
@@ -43,10 +44,12 @@ struct FloodJob {
 // max_grid workgroups at once (0: two per compute unit).
 void prepare_fields(Context &ctx, const std::vector<FloodJob> &jobs, const std::vector<LabelItem> &items,
                     int max_grid = 0);
+// On every traced voxel (use != 0): its road word (unreached, cost = the PDRF) and its claim word
+// (free); the PDRF as a volume too when `pdrf` is given (+inf elsewhere).
 void pdrf_and_alive(Context &ctx, const void *cc, int cc_bytes, long long n, const float *dbf, const float *daf,
                     const float *M, const float *inv, const unsigned char *use, int squarings, float scale, float *pdrf,
-                    VoxelRec *rec);
-void root_rails(Context &ctx, VoxelRec *rec, const long long *root, const int *labels, int count);
+                    unsigned long long *road, unsigned long long *claim);
+void root_rails(Context &ctx, unsigned long long *road, const long long *root, const int *labels, int count);
 // Per-id target order in segment layout: order[seg_start[id] + j] = the id's voxels by descending
 // DAF (inf and 0 as 0), ties by descending flat index (lockstep_order.cu:21-43); F foreground voxels.
 void target_order(Context &ctx, const void *cc, int cc_bytes, long long n, const float *daf, long long F, int64_t count,

@@ -254,21 +254,21 @@ void run_graph_edt(Context &ctx, const CC *cc, Dims d, const unsigned *graph, co
 }
 
 // ---- gates of the neighbour masks -------------------------------------------------------------
-// meta's same-label mask keeps the steps the voxel's own word permits (pushes: floods, railroads,
+// The same-label mask keeps the steps the voxel's own word permits (pushes: floods, railroads,
 // joins, invalidation offers); in[v] bit k: neighbour u = v + N[k] is of v's id and u's word permits
 // the step u -> v (pulls: backtraces, band-boundary pulls, parents).
-__global__ void __launch_bounds__(256) g_gates(VoxelRec *rec, const unsigned *graph, Dims d, long long n,
+__global__ void __launch_bounds__(256) g_gates(unsigned *mask, const unsigned *graph, Dims d, long long n,
                                                unsigned *in) {
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
-  const unsigned meta = rec[i].meta, same = meta & kNbrBits;
+  const unsigned same = mask[i];
   unsigned pull = 0;
   for_each_nb([&](auto K) {
     constexpr int k = decltype(K)::value;
     if ((same >> k) & 1u) pull |= ((graph[i + nb_offset<k>(d)] >> kGraphBit[kOppositeOf[k]]) & 1u) << k;
   });
   in[i] = pull;
-  rec[i].meta = (meta & ~kNbrBits) | (same & step_mask(graph[i], false));
+  mask[i] = same & step_mask(graph[i], false);
 }
 
 }  // namespace
@@ -310,10 +310,10 @@ void widen_words(Context &ctx, const uint8_t *in, long long n, unsigned *out) {
   BROOK_LAUNCHED();
 }
 
-void graph_gates(Context &ctx, VoxelRec *rec, const unsigned *graph, Dims d, unsigned *in_masks) {
+void graph_gates(Context &ctx, unsigned *mask, const unsigned *graph, Dims d, unsigned *in_masks) {
   const long long n = (long long)d.sx * d.sy * d.sz;
   if (n == 0) return;
-  g_gates<<<blocks_of(n), 256, 0, ctx.stream()>>>(rec, graph, d, n, in_masks);
+  g_gates<<<blocks_of(n), 256, 0, ctx.stream()>>>(mask, graph, d, n, in_masks);
   BROOK_LAUNCHED();
 }
 

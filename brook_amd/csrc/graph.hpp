@@ -22,7 +22,7 @@ void graph_edt(Context &ctx, const void *cc, int cc_bytes, Dims dims, const unsi
                bool black_border, float *out, unsigned *label_max = nullptr);
 // A uint8 plane graph widened to one uint32 word per voxel, value for value.
 void widen_words(Context &ctx, const uint8_t *in, long long n, unsigned *out);
-// Gates the records' same-label masks by the graph (pushes) and writes the pull masks (n words).
-void graph_gates(Context &ctx, VoxelRec *rec, const unsigned *graph, Dims dims, unsigned *in_masks);
+// Gates the same-label masks by the graph (pushes) and writes the pull masks (n words).
+void graph_gates(Context &ctx, unsigned *mask, const unsigned *graph, Dims dims, unsigned *in_masks);
 
 }  // namespace brook

@@ -16,11 +16,13 @@
 //   invalidate rolling ball, bands of the bottleneck M on a fixed grid, synchronous rounds from
 //              a snapshot inside a band, exact pulls at band boundaries
 //                                                         (invalidation_kernels.cuh:105-299)
-// Neighbour walks read the per-voxel same-label mask (one word instead of 26 ids).
+// Neighbour walks read the per-voxel same-label mask (one word instead of 26 ids), and half a wave
+// serves a front entry, a lane per neighbour (front.hpp).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 
+#include "front.hpp"
 #include "trace.hpp"
 #include "tuned.hpp"
 
@@ -28,89 +30,71 @@ namespace brook {
 namespace {
 
 constexpr int kBlock = BROOK_TRACE_BLOCK;  // threads per label workgroup
+constexpr int kWaves = kBlock / 64;
+constexpr int kMaxPairs = BROOK_NB_BATCH;
 constexpr unsigned long long kMinfarNone = 0x7f8000007f800000ULL;
-constexpr unsigned long long kClaimed = 0xFFFFFFFFFFFFFFFEULL;
 constexpr int kProf = kTraceProfileSlots;
-// Neighbours whose memory operations one thread keeps in flight together (26: all; 13: two parts;
-// 9: three parts). Fewer in flight, fewer registers.
-constexpr int kNbBatch = BROOK_NB_BATCH;
+// A railroad band's width in costs of its first voxel. Narrow bands relax a voxel less often, wide
+// ones take fewer rounds. Slowest label of the 512^3 workload, railroads in ms (entries relaxed):
+// width 4 54.9 (1.65 M), 2 35.7 (936 k), 1 31.0 (696 k), 0.5 30.6 (523 k); a 48-voxel crop of three
+// tubes 1.73, 1.76, 1.80, 2.02; a 31 M voxel request 9.4, 7.0, 6.6, 6.9.
+#ifndef BROOK_ROAD_BAND
+#define BROOK_ROAD_BAND 1.0f
+#endif
 
-
-__device__ __forceinline__ int wave_min(int v) {
-  for (int off = 32; off > 0; off >>= 1) v = min(v, __shfl_xor(v, off, 64));
-  return v;
-}
-
-// Front lists (the near rounds of the railroad and the invalidation rounds): entry j lives in LDS for
-// j < kLdsFront and in the label's global list beyond, so a round's appends and the next round's
-// reads of a small front never wait for device memory.
-constexpr int kLdsFront = 4096;
+// Entries of the near fronts and of the far (waiting) lists that live in LDS; longer lists go on in
+// the label's device memory. (Registers allow one workgroup of 1024 threads per compute unit, so the
+// workgroup may take most of its 160 KB.)
+constexpr int kLdsFront = 3072, kLdsFar = 2048;
 constexpr int kRadiusSlots = 4096;
+using Front = SplitList<kLdsFront>;
+using Far = SplitList<kLdsFar>;
+
+// List lengths (Shared::n). Front lengths rotate over three counters: round r reads n[r], appends to
+// n[r+1] and clears n[r+2] (read in round r-1), so a round needs one barrier. The far (waiting)
+// lengths rotate likewise over kFar .. kFar + 2, a step per phase (band).
+constexpr int kFar = 3, kTouched = 6, kStale = 7, kDirty = 8, kCounters = 9;
+
+// What a round found about the railroad's far list, in the rotation of the front lengths (a wave
+// ahead by a barrier writes another slot than the one its workgroup still reads): kLong, more than
+// `count` entries (compacted); kFull, an append found the list at its end (never expected).
+constexpr int kLong = 1, kFull = 2;
 
 struct Shared {
-  // Front-list lengths rotate over three counters: round r reads cnt[r], appends to cnt[r+1] and
-  // clears cnt[r+2] (read in round r-1), which saves the barrier that a swap of two would need.
-  int cnt[3];
-  int n_far, n_farnxt, n_touched, n_keep;
-  int done, target, path_len, found, band;
+  int n[kCounters], flags[3];
+  int done, target, path_len, found;
   long long cursor, seg_end;
   int pcount, ordered, after_used;  // ordered: the current target came from the DAF order
-  unsigned lowest;
+  unsigned lowest[3];               // invalidation: least waiting bottleneck, rotating per band
   float T;
   unsigned long long rail_best, minfar;
   int store_pos;
-  // The railroad's far lists hold 2 * count entries; a list longer than count after a round is
-  // compacted (see far_compact). `overflow`: an append found the list full (never expected).
-  int far_cap, overflow;
-  int off[26];  // flat offsets of the 26 neighbours
   // per-label profile: [0] total [1] target [2] railroad [3] backtrace [4] invalidation (wall-clock
   // ticks), [5] railroad rounds, [6] invalidation rounds, [7] paths, [8] railroad phases,
   // [9] far entries scanned, [10] near entries expanded, [11] invalidation entries expanded,
-  // [12] waiting entries pulled, [13] bands
+  // [12] waiting entries scanned, [13] bands, [14] entries pulled
   unsigned long long prof[kProf];
   long long tick;
   int front[2][kLdsFront];
+  int far[2][kLdsFar];
   // invalidation: ball radii of the path's voxels by source (see source_radius)
   unsigned long long radius[kRadiusSlots];
+  Stage stage[kWaves];
 };
 
-__device__ __forceinline__ int rot_next(int r) { return r == 2 ? 0 : r + 1; }
-__device__ __forceinline__ int rot_prev(int r) { return r == 0 ? 2 : r - 1; }
-
-struct Front {
-  int *g;  // the label's list in device memory (entries >= kLdsFront)
-  int *s;  // LDS (entries < kLdsFront)
+// A label's lists: near fronts, far lists (the far device lists hold two entries per voxel), and the
+// invalidation's scratch (two ints, or one snapshot, per voxel each).
+struct Lists {
+  Front near[2];
+  Far far[2];
+  int *touched, *walk;
+  unsigned long long *snap;
+  int *stale;
 };
-__device__ __forceinline__ int front_get(const Front &f, int j) { return j < kLdsFront ? f.s[j] : lp_i(f.g + j); }
-__device__ __forceinline__ void front_put(const Front &f, int j, int v) {
-  if (j < kLdsFront) f.s[j] = v;
-  else g_st(f.g + j, v);
-}
-// emit_neighbours into a front list.
-__device__ __forceinline__ void emit_front(const Front &f, int *counter, unsigned mask, int u, const int *off) {
-  int pos = wave_reserve(counter, __popc(mask));
-  while (mask) {
-    const int k = __ffs(mask) - 1;
-    mask &= mask - 1;
-    front_put(f, pos++, u + off[k]);
-  }
-}
-
-// emit_neighbours into a list of `cap` entries: a wave whose appends would pass the end writes
-// nothing and raises `overflow` instead.
-__device__ __forceinline__ void emit_capped(int *list, int *counter, unsigned mask, int u, const int *off, int cap,
-                                            int *overflow) {
-  const int n = __popc(mask);
-  int pos = wave_reserve(counter, n);
-  if (pos + n > cap) {
-    if (n) *overflow = 1;
-    return;
-  }
-  while (mask) {
-    const int k = __ffs(mask) - 1;
-    mask &= mask - 1;
-    g_st(list + pos++, u + off[k]);
-  }
+__device__ __forceinline__ Lists lists_of(const TraceArgs &a, Shared &sh, int seg) {
+  return Lists{{Front{a.lists[0] + seg, sh.front[0]}, Front{a.lists[1] + seg, sh.front[1]}},
+               {Far{a.lists[2] + 2LL * seg, sh.far[0]}, Far{a.lists[3] + 2LL * seg, sh.far[1]}},
+               a.lists[4] + seg, a.lists[5] + seg, a.snaps[0] + seg, reinterpret_cast<int *>(a.snaps[1] + seg)};
 }
 
 // Rounds (and phases) one railroad or invalidation may take before the label is given up as not
@@ -134,213 +118,133 @@ __device__ __forceinline__ void lap(Shared &sh, int slot) {
   }
 }
 
+__device__ __forceinline__ unsigned mask_of(const TraceArgs &a, int v) { return g_ld(a.mask + v); }
 // The neighbours v may pull from (see TraceArgs::inmask).
 __device__ __forceinline__ unsigned in_mask(const TraceArgs &a, int v) {
-  return a.inmask ? g_ld(a.inmask + v) : rec_meta(a.rec, v) & kNbrBits;
+  return a.inmask ? g_ld(a.inmask + v) : mask_of(a, v);
+}
+// Voxel coordinates by high products instead of divisions.
+__device__ __forceinline__ void place(const TraceArgs &a, int v, int &x, int &y, int &z) {
+  z = int(fast_quotient(unsigned(v), a.by_plane));
+  const int r = v - z * (a.d.sx * a.d.sy);
+  y = int(fast_quotient(unsigned(r), a.by_row));
+  x = r - y * a.d.sx;
 }
 
 // ---- railroad -------------------------------------------------------------------------------
-// Distances live in the records' packed words: high half the distance bits, bit 0 "not
-// queued", bit 1 "far listed". A front voxel is dequeued by one atomicOr that also returns its
-// distance; an improvement is one atomicMin whose old value says whether the voxel still has to
-// be queued or far-listed. Near candidates store 00 (queued), rails 01, far candidates 11; a near
-// improvement of a far-listed voxel clears its far bit, so its far-list entry goes stale.
+// Distances live in the road words (common.hpp). A front voxel is dequeued by one atomic or that
+// also returns its distance; an improvement is one atomic minimum whose old value says whether the
+// voxel still has to be queued or far-listed. Near candidates are queued (no flag), rails not queued,
+// far candidates far-listed and not queued; a near improvement of a far-listed voxel clears its far
+// flag, so its far-list entry goes stale. A rail is recognised by its zero cost.
 // Per-thread minima of the reached rails and far distances are folded into LDS once per round.
-constexpr unsigned long long kRoadNear = 0, kRoadRail = 1, kRoadFar = 3;
-// A word whose far bit is set by a far candidate (the unreached sentinel ~0 is not far-listed).
-__device__ __forceinline__ bool far_listed(unsigned long long w) {
-  return (w & 2ULL) && (unsigned)(w >> 32) != 0xFFFFFFFFu;
-}
-
 struct RoadMins {
   unsigned long long rail = kMaxKey, far = kMinfarNone;
 };
 
-// Neighbours (bit k = neighbour k) to append to the touched, near and far lists.
-struct Pushes {
-  unsigned touched = 0, near = 0, far = 0;
-};
-
 __device__ __forceinline__ void road_fold(Shared &sh, RoadMins &mins) {
-  const unsigned long long r = wave_min_u64(mins.rail), f = wave_min_u64(mins.far);
-  if (__lane_id() == 0) {
-    if (r != kMaxKey) atomicMin(&sh.rail_best, r);
-    if (f != kMinfarNone) atomicMin(&sh.minfar, f);
+  if (any_lane(mins.rail != kMaxKey)) {
+    const unsigned long long r = wave_least(mins.rail);
+    if (__lane_id() == 0) atomicMin(&sh.rail_best, r);
+  }
+  if (any_lane(mins.far != kMinfarNone)) {
+    const unsigned long long f = wave_least(mins.far);
+    if (__lane_id() == 0) atomicMin(&sh.minfar, f);
   }
   mins = RoadMins{};
 }
 
-// Masked neighbours B..E-1 of u at once: every load, then every atomic, is issued before any result
-// is waited for; the outcome is a set of bit masks (list appends happen once per loop iteration).
-// A rail is recognised by cand == du (vw_step adds nothing only for a zero cost).
-template <int B, int E>
-__device__ __forceinline__ void relax_part(const TraceArgs &a, RoadMins &mins, int u, unsigned m, float du, float bound,
-                                           Pushes &p) {
-  float c[E - B];
-  unsigned seen[E - B];
-  for_nb<B, E>([&](auto K) {
-    constexpr int k = decltype(K)::value, i = k - B;
-    const bool on = (m >> k) & 1u;
-    const RecWords r = on ? rec_load(a.rec, u + nb_offset<k>(a.d)) : RecWords{0x7f800000u, 0u, 0u, 0u};
-    c[i] = __uint_as_float(r.x);
-    seen[i] = r.w;
-  });
-  unsigned long long old[E - B];
-  for_nb<B, E>([&](auto K) {
-    constexpr int k = decltype(K)::value, i = k - B;
-    const float cc = vw_step(du, c[i]);
-    c[i] = cc;
-    const unsigned cb = __float_as_uint(cc);
-    const bool rail = cc == du, near = !rail && cc <= bound;
-    old[i] = 0;  // "nothing changed" unless the atomic says otherwise
-    if (cb < seen[i] && cc < kInf)
-      old[i] = g_min(&a.rec[u + nb_offset<k>(a.d)].word,
-                         ((unsigned long long)cb << 32) | (near ? kRoadNear : rail ? kRoadRail : kRoadFar));
-  });
-  for_nb<B, E>([&](auto K) {
-    constexpr int k = decltype(K)::value, i = k - B;
-    const float cc = c[i];
-    const unsigned cb = __float_as_uint(cc);
-    const bool rail = cc == du, near = !rail && cc <= bound;
-    const unsigned long long nv = ((unsigned long long)cb << 32) | (near ? kRoadNear : rail ? kRoadRail : kRoadFar);
-    if (!(old[i] > nv)) return;
-    if ((unsigned)(old[i] >> 32) == 0xFFFFFFFFu) p.touched |= 1u << k;
-    if (rail) {
-      const unsigned long long key = ((unsigned long long)cb << 32) | (unsigned)(u + nb_offset<k>(a.d));
+// The lists of a railroad round.
+struct RoadLists {
+  Front nxt;
+  int n_nxt;
+  Far far;
+  int n_far;
+  int *touched;
+  int count;
+};
+
+// Front entries b .. of one railroad round over nc entries, at most 2P (the wave's batch): the
+// neighbours whose distance they improve go to the wave's stage.
+template <int P, bool Wide, class Flush>
+__device__ __forceinline__ void road_batch(const TraceArgs &a, const Lane<Wide> &ln, const Front &cur, int b, int nc,
+                                           unsigned bound, Stage &st, int &staged, Flush &&flush) {
+  int u[P];
+  const int ue = batch_entries<P>(ln, cur, b, nc, u);
+  unsigned long long q = 0, w[P];
+  unsigned me = 0;
+  if (ln.lane < min(2 * P, nc - b)) {  // lane e: entry e's distance by the dequeue, and its mask
+    q = g_or(a.road + ue, kNotQueued);
+    me = mask_of(a, ue);
+  }
+#pragma unroll
+  for (int p = 0; p < P; ++p) w[p] = g_ld(word_at(a.road0, ln.at(u[p])));
+  const unsigned de = road_dist(q);
+  if (de > bound) me = 0;
+  staged_pairs<P>([&](int p) {
+    const unsigned m = of_entry(ln, me, 2 * p), d = of_entry(ln, de, 2 * p);
+    const unsigned lo = unsigned(w[p]), hi = unsigned(w[p] >> 32);
+    const float cost = __uint_as_float(lo & kCostBits);
+    const bool rail = cost == 0.0f;
+    // The step d + cost, on the bits: one ulp up where a positive cost leaves d as it is (the rule of
+    // the reference's brook_vw_step, common.cuh:123-127), so distances increase strictly along every
+    // step and predecessor walks terminate.
+    const unsigned c = rail ? d : max(__float_as_uint(__uint_as_float(d) + cost), d + 1u);
+    const bool later = c > bound;  // never a rail: d <= bound
+    const unsigned nhi = (c << 1) | unsigned(later);
+    const unsigned nlo = (lo & kCostBits) | (rail | later ? unsigned(kNotQueued) : 0u);
+    // c below the distance: 2 * distance + far flag is above 2 * c + 1
+    stage_put(st, staged, ((m & ln.bit) != 0u) & ((nhi | 1u) < hi), u[p] + ln.off, ((unsigned long long)nhi << 32) | nlo);
+  }, flush);
+}
+
+// The staged improvements of a wave (full groups, or all of them).
+__device__ __forceinline__ void road_minima(const TraceArgs &a, Shared &sh, RoadMins &mins, Stage &st, int &staged, bool all,
+                                            const RoadLists &to) {
+  stage_take(st, staged, all, [&](bool on, int v, unsigned long long nv) {
+    unsigned long long old = 0;  // "nothing changed" unless the atomic says otherwise
+    if (on) old = g_min(a.road + v, nv);
+    const unsigned ohi = unsigned(old >> 32), cost = road_cost(nv);
+    const bool won = old > nv, later = nv & kFarListed, rail = cost == 0u;
+    if (won & rail) {
+      const unsigned long long key = ((unsigned long long)road_dist(nv) << 32) | unsigned(v);
       mins.rail = key < mins.rail ? key : mins.rail;
-    } else if (near) {
-      if (old[i] & 1ULL) p.near |= 1u << k;
-    } else {
-      const unsigned long long key = ((unsigned long long)cb << 32) | __float_as_uint(cc - du);
-      mins.far = key < mins.far ? key : mins.far;
-      if (!far_listed(old[i])) p.far |= 1u << k;
     }
+    if (won & later) {
+      const unsigned long long key = ((unsigned long long)road_dist(nv) << 32) | cost;
+      mins.far = key < mins.far ? key : mins.far;
+    }
+    Appends out;
+    if (!out.begin(sh.n, kTouched, ohi == unsigned(kUnreached >> 32), to.n_nxt, won & !later & !rail & (int(unsigned(old)) < 0),
+                   to.n_far, won & later & !(ohi & 1u)))
+      return;
+    // the far lists hold 2 * count entries: a wave whose appends would pass the end writes none
+    const int end = out.at[2] + out.count(2);
+    const bool full = end > 2 * to.count;
+    if (out.set[2] && end > to.count) atomicOr(&sh.flags[to.n_nxt], full ? kLong | kFull : kLong);
+    if (ohi == unsigned(kUnreached >> 32)) g_st(to.touched + out.place(0), v);
+    if (won & !later & !rail & (int(unsigned(old)) < 0)) to.nxt.put(out.place(1), v);
+    if (won & later & !(ohi & 1u) & !full) to.far.put(out.place(2), v);
   });
-}
-
-__device__ __forceinline__ void relax_all(const TraceArgs &a, RoadMins &mins, int u, unsigned m, float du, float bound,
-                                          Pushes &p) {
-  for_parts<kNbBatch>(m, [&](auto B, auto E) { relax_part<decltype(B)::value, decltype(E)::value>(a, mins, u, m, du, bound, p); });
-}
-
-// Dequeues front voxel u: marks it "not queued" and returns its distance, in one atomic.
-__device__ __forceinline__ float dequeue(const TraceArgs &a, int u) {
-  return __uint_as_float((unsigned)(g_or(&a.rec[u].word, 1ULL) >> 32));
-}
-
-// ---- fronts of up to a quarter workgroup: a group of lanes per entry (group_of) ----------------
-constexpr int kGroupFront = kBlock / 4;
-__device__ __forceinline__ Group group_of(int n) { return brook::group_of(n, kBlock); }
-
-// Neighbours kb..kb+cnt-1 (those set in m; cnt <= kSpan) of u: relax_part with a run-time span.
-__device__ __forceinline__ void relax_span(const TraceArgs &a, RoadMins &mins, int u, unsigned m, int kb, int cnt, float du,
-                                           float bound, const int *off, Pushes &p) {
-  constexpr int S = kSpan;
-  float c[S];
-  unsigned seen[S];
-  int v[S];
-#pragma unroll
-  for (int j = 0; j < S; ++j) {
-    const int k = kb + j;
-    const bool on = j < cnt && ((m >> k) & 1u);
-    v[j] = u + off[on ? k : 0];
-    const RecWords r = on ? rec_load(a.rec, v[j]) : RecWords{0x7f800000u, 0u, 0u, 0u};
-    c[j] = __uint_as_float(r.x);
-    seen[j] = r.w;
-  }
-  unsigned long long old[S];
-#pragma unroll
-  for (int j = 0; j < S; ++j) {
-    const float cc = vw_step(du, c[j]);
-    c[j] = cc;
-    const unsigned cb = __float_as_uint(cc);
-    const bool rail = cc == du, near = !rail && cc <= bound;
-    old[j] = 0;  // "nothing changed" unless the atomic says otherwise
-    if (cb < seen[j] && cc < kInf)
-      old[j] = g_min(&a.rec[v[j]].word, ((unsigned long long)cb << 32) | (near ? kRoadNear : rail ? kRoadRail : kRoadFar));
-  }
-#pragma unroll
-  for (int j = 0; j < S; ++j) {
-    const int k = kb + j;
-    const float cc = c[j];
-    const unsigned cb = __float_as_uint(cc);
-    const bool rail = cc == du, near = !rail && cc <= bound;
-    const unsigned long long nv = ((unsigned long long)cb << 32) | (near ? kRoadNear : rail ? kRoadRail : kRoadFar);
-    if (!(old[j] > nv)) continue;
-    if ((unsigned)(old[j] >> 32) == 0xFFFFFFFFu) p.touched |= 1u << k;
-    if (rail) {
-      const unsigned long long key = ((unsigned long long)cb << 32) | (unsigned)v[j];
-      mins.rail = key < mins.rail ? key : mins.rail;
-    } else if (near) {
-      if (old[j] & 1ULL) p.near |= 1u << k;
-    } else {
-      const unsigned long long key = ((unsigned long long)cb << 32) | __float_as_uint(cc - du);
-      mins.far = key < mins.far ? key : mins.far;
-      if (!far_listed(old[j])) p.far |= 1u << k;
-    }
-  }
-}
-
-// One railroad round over a front of at most kGroupFront entries, a group of lanes per entry: the
-// group's first lane dequeues the entry and shares it.
-__device__ __forceinline__ void relax_groups(const TraceArgs &a, Shared &sh, RoadMins &mins, const Front &cur, int nc,
-                                             float bound, const Front &nxt, int *n_nxt, int *far, int *touched) {
-  const Group q = group_of(nc);
-  int u = 0;
-  unsigned m = 0;
-  float du = kInf;
-  if (q.g == 0 && q.i < nc) {
-    u = front_get(cur, q.i);
-    m = rec_meta(a.rec, u) & kNbrBits;
-    du = dequeue(a, u);
-  }
-  u = __shfl(u, q.lead, 64);
-  m = __shfl(m, q.lead, 64);
-  du = __shfl(du, q.lead, 64);
-  Pushes p;
-  if (q.i < nc && du <= bound) relax_span(a, mins, u, m, q.kb, q.cnt, du, bound, sh.off, p);
-  emit_neighbours(touched, &sh.n_touched, p.touched, u, sh.off);
-  emit_front(nxt, n_nxt, p.near, u, sh.off);
-  emit_capped(far, &sh.n_far, p.far, u, sh.off, sh.far_cap, &sh.overflow);
-}
-
-// One railroad round over a larger front: a thread per entry, its neighbours in parts.
-__device__ __forceinline__ void relax_front(const TraceArgs &a, Shared &sh, RoadMins &mins, const Front &cur, int nc,
-                                            float bound, const Front &nxt, int *n_nxt, int *far, int *touched) {
-  for (int base = 0; base < nc; base += blockDim.x) {  // uniform: every lane reaches the appends
-    const int i = base + threadIdx.x;
-    Pushes p;
-    int u = 0;
-    if (i < nc) {
-      u = front_get(cur, i);
-      const unsigned m = (rec_meta(a.rec, u) & kNbrBits);
-      const float du = dequeue(a, u);
-      if (du <= bound) relax_all(a, mins, u, m, du, bound, p);
-    }
-    emit_neighbours(touched, &sh.n_touched, p.touched, u, sh.off);
-    emit_front(nxt, n_nxt, p.near, u, sh.off);
-    emit_capped(far, &sh.n_far, p.far, u, sh.off, sh.far_cap, &sh.overflow);
-  }
 }
 
 // Far-list compaction between rounds. A voxel can hold several entries: its entry goes stale when
-// a near improvement clears its far bit, and it is far-listed anew when a later, smaller bound
+// a near improvement clears its far flag, and it is far-listed anew when a later, smaller bound
 // (a closer rail) leaves its next improvement beyond the band. Within one round the bound is fixed,
 // so a round appends at most one entry per voxel (at most `count`); a list that holds more than
 // `count` entries after a round keeps one entry per far-listed voxel (the one whose atomic clears
-// the far bit, restored after a barrier), so 2 * count entries always suffice.
-__device__ __forceinline__ void far_compact(const TraceArgs &a, Shared &sh, int *&fcur, int *&fnxt) {
-  const int nf = sh.n_far;
+// the far flag, restored after a barrier), so 2 * count entries always suffice.
+__device__ __forceinline__ void far_compact(const TraceArgs &a, Shared &sh, const Far &from, int n_from, const Far &to,
+                                            int n_to) {
+  const int nf = sh.n[n_from];
   for (int i = threadIdx.x; i < nf; i += blockDim.x) {
-    const int w = lp_i(fcur + i);
-    if (far_listed(g_and(&a.rec[w].word, ~2ULL))) g_st(fnxt + wave_slot(&sh.n_farnxt), w);
+    const int w = from.get(i);
+    if (g_and(a.road + w, ~kFarListed) & kFarListed) to.put(wave_slot(&sh.n[n_to]), w);
   }
   __syncthreads();
-  const int kept = sh.n_farnxt;
-  for (int i = threadIdx.x; i < kept; i += blockDim.x) g_or(&a.rec[lp_i(fnxt + i)].word, 2ULL);
-  __syncthreads();
-  if (threadIdx.x == 0) { sh.n_far = kept; sh.n_farnxt = 0; }
-  int *tmp = fcur; fcur = fnxt; fnxt = tmp;
+  const int kept = sh.n[n_to];
+  for (int i = threadIdx.x; i < kept; i += blockDim.x) g_or(a.road + to.get(i), kFarListed);
+  if (threadIdx.x == 0) sh.n[n_from] = 0;
   __syncthreads();
 }
 
@@ -356,57 +260,77 @@ __device__ __forceinline__ float rail_bound(const Shared &sh) {
 // `source` run never takes t itself for a rail: with no rails in the label it settles every voxel
 // reachable from t (the vertex-weighted distances of the fix_branching=False field). The far lists
 // hold 2 * count entries.
-__device__ __forceinline__ int railroad(const TraceArgs &a, Shared &sh, int t, int count, const Front &near_a,
-                                        const Front &near_b, int *far_a, int *far_b, int *touched, bool source = false) {
+template <bool Wide>
+__device__ __forceinline__ int railroad(const TraceArgs &a, Shared &sh, const Lane<Wide> &ln, int t, int count, const Lists &l,
+                                        bool source = false) {
   if (threadIdx.x == 0) {
-    g_st(touched, t);
-    sh.n_touched = 1;
-    sh.cnt[0] = sh.cnt[1] = sh.cnt[2] = sh.n_far = sh.n_farnxt = 0;
-    sh.far_cap = 2 * count;
-    sh.overflow = 0;
+    g_st(l.touched, t);
+    for (int j = 0; j < kCounters; ++j) sh.n[j] = 0;
+    for (int j = 0; j < 3; ++j) sh.flags[j] = 0;
+    sh.n[kTouched] = 1;
     sh.minfar = kMinfarNone;
-    float ft = rec_pdrf(a.rec, t);
+    const unsigned cost = road_cost(lp_u64(a.road + t));
+    const float ft = __uint_as_float(cost);
     if (ft == 0.0f && !source) {
-      sp_u64(&a.rec[t].word, 1ULL);  // distance 0, not queued
+      sp_u64(a.road + t, road_word(0u, kNotQueued, cost));
       sh.rail_best = (unsigned)t;
       sh.done = kRailFound;
     } else {
-      sp_u64(&a.rec[t].word, 0ULL);  // distance 0, queued
+      sp_u64(a.road + t, road_word(0u, 0ULL, cost));  // queued
       sh.rail_best = kMaxKey;
       sh.done = 0;
-      front_put(near_a, 0, t);
-      sh.cnt[0] = 1;
+      l.near[0].put(0, t);
+      sh.n[0] = 1;
       sh.T = fmaxf(2.0f * ft, 1e-30f);
     }
   }
   __syncthreads();
   RoadMins mins;
-  Front cur = near_a, nxt = near_b;
-  int *fcur = far_a, *fnxt = far_b;
-  int r = 0;  // the near list's length is sh.cnt[r]
-  long long rounds = 0;  // rounds and phases so far (the same in every thread)
+  Stage &st = sh.stage[ln.wave];
+  Front cur = l.near[0], nxt = l.near[1];
+  Far fcur = l.far[0], fnxt = l.far[1];
+  int fc = kFar, fn = kFar + 1;  // their lengths are sh.n[fc], sh.n[fn]
+  int r = 0;                     // the near list's length is sh.n[r]
+  long long rounds = 0;          // rounds and phases so far (the same in every thread)
   const long long budget = round_budget(count);
-  while (sh.done == 0) {
-    bool stop = false;
+  auto swap_far = [&] {
+    const Far f = fcur; fcur = fnxt; fnxt = f;
+    const int n = fc; fc = fn; fn = n;
+  };
+  int done = sh.done;  // read after a barrier, written again only after the next one
+  while (done == 0) {
+    int stop = 0;
     for (;;) {  // settle the near band
-      const int nc = sh.cnt[r];
+      const int nc = __builtin_amdgcn_readfirstlane(sh.n[r]);
       if (nc == 0) break;
       const int rn = rot_next(r);
-      if (threadIdx.x == 0) { sh.cnt[rot_prev(r)] = 0; sh.prof[5] += 1; sh.prof[10] += nc; }
-      const float bound = rail_bound(sh);
-      if (nc <= kGroupFront) relax_groups(a, sh, mins, cur, nc, bound, nxt, &sh.cnt[rn], fcur, touched);
-      else relax_front(a, sh, mins, cur, nc, bound, nxt, &sh.cnt[rn], fcur, touched);
+      if (threadIdx.x == 0) {
+        sh.n[rot_prev(r)] = sh.flags[rot_prev(r)] = 0;
+        sh.prof[5] += 1;
+        sh.prof[10] += nc;
+      }
+      const unsigned bound = unsigned(__builtin_amdgcn_readfirstlane(__float_as_int(rail_bound(sh))));
+      const RoadLists to{nxt, rn, fcur, fc, l.touched, count};
+      int staged = 0;
+      with_pairs<kMaxPairs>(nc, kWaves, [&](auto Pairs) {
+        constexpr int P = decltype(Pairs)::value;
+        for (int b = ln.wave * 2 * P; b < nc; b += kWaves * 2 * P)
+          road_batch<P>(a, ln, cur, b, nc, bound, st, staged, [&] { road_minima(a, sh, mins, st, staged, false, to); });
+      });
+      road_minima(a, sh, mins, st, staged, true, to);
       road_fold(sh, mins);
       __syncthreads();
       r = rn;
-      const Front tmp = cur; cur = nxt; nxt = tmp;
-      if (sh.overflow || ++rounds > budget) { stop = true; break; }
-      if (sh.n_far > count) far_compact(a, sh, fcur, fnxt);
+      const Front f = cur; cur = nxt; nxt = f;
+      const int flags = sh.flags[r];
+      if ((flags & kFull) || ++rounds > budget) { stop = (flags & kFull) ? kOverflowed : kStalled; break; }
+      if (flags & kLong) {
+        far_compact(a, sh, fcur, fc, fnxt, fn);
+        swap_far();
+      }
     }
-    if (stop) {  // uniform: every thread read the same flags after the round's barrier
-      __syncthreads();
-      if (threadIdx.x == 0) sh.done = sh.overflow ? kOverflowed : kStalled;
-      __syncthreads();
+    if (stop) {  // uniform: every thread read the same flags
+      done = stop;
       break;
     }
     if (threadIdx.x == 0) {  // phase end: nearest rail final? else advance the band
@@ -416,75 +340,83 @@ __device__ __forceinline__ int railroad(const TraceArgs &a, Shared &sh, int t, i
       else if (rounds + 1 > budget) sh.done = kStalled;
       else {
         float dmin = __uint_as_float((unsigned)(mf >> 32)), f = __uint_as_float((unsigned)mf);
-        float w = 2.0f * f, lo = 5e-4f * dmin;
+        float w = BROOK_ROAD_BAND * f, lo = 5e-4f * dmin;
         if (!(w > lo)) w = lo;
         sh.T = dmin + w;
         sh.minfar = kMinfarNone;
       }
       sh.prof[8] += 1;
-      sh.prof[9] += sh.n_far;
+      sh.prof[9] += sh.n[fc];
     }
     ++rounds;
     __syncthreads();
-    if (sh.done) break;
-    const int nf = sh.n_far;
+    done = sh.done;
+    if (done) break;
+    const int nf = sh.n[fc];
     const float bound = rail_bound(sh);
-    // Promote far voxels inside the new band. Entries whose far bit is clear are stale (the voxel
-    // went near); of several entries of one voxel, the one whose atomic clears the far bit acts.
+    // Promote far voxels inside the new band. Entries whose far flag is clear are stale (the voxel
+    // went near); of several entries of one voxel, the one whose atomic clears the far flag acts.
     // A far-listed word is never queued, so the claim also queues it; a voxel still beyond the
-    // band gets both bits back. Each voxel lands in at most one list (at most count entries).
+    // band gets both flags back. Each voxel lands in at most one list (at most count entries).
     for (int i = threadIdx.x; i < nf; i += blockDim.x) {
-      const int w = lp_i(fcur + i);
-      if (!far_listed(lp_u64(&a.rec[w].word))) continue;
-      const unsigned long long was = g_and(&a.rec[w].word, ~3ULL);
-      if (!far_listed(was)) continue;
-      const float dw = __uint_as_float((unsigned)(was >> 32));
+      const int w = fcur.get(i);
+      if (!(lp_u64(a.road + w) & kFarListed)) continue;
+      const unsigned long long was = g_and(a.road + w, ~(kFarListed | kNotQueued));
+      if (!(was & kFarListed)) continue;
+      const float dw = __uint_as_float(road_dist(was));
       if (dw <= bound) {
-        front_put(cur, wave_slot(&sh.cnt[r]), w);
+        cur.put(wave_slot(&sh.n[r]), w);
       } else {
-        g_or(&a.rec[w].word, kRoadFar);
-        const unsigned long long key = ((unsigned long long)__float_as_uint(dw) << 32) | __float_as_uint(rec_pdrf(a.rec, w));
+        g_or(a.road + w, kFarListed | kNotQueued);
+        const unsigned long long key = ((unsigned long long)road_dist(was) << 32) | road_cost(was);
         mins.far = key < mins.far ? key : mins.far;
-        g_st(fnxt + wave_slot(&sh.n_farnxt), w);
+        fnxt.put(wave_slot(&sh.n[fn]), w);
       }
     }
     road_fold(sh, mins);
     __syncthreads();
-    if (threadIdx.x == 0) { sh.n_far = sh.n_farnxt; sh.n_farnxt = 0; }
-    int *tmp = fcur; fcur = fnxt; fnxt = tmp;
-    __syncthreads();
+    if (threadIdx.x == 0) sh.n[fc] = 0;  // read above; appended to again after the next phase end's barrier
+    swap_far();
   }
-  return sh.done;
+  return done;
+}
+
+// The railroad's words back to unreached, costs kept.
+__device__ __forceinline__ void road_restore(const TraceArgs &a, const Shared &sh, const int *touched) {
+  const int nt = sh.n[kTouched];
+  for (int j = threadIdx.x; j < nt; j += blockDim.x) {
+    const int v = g_ld(touched + j);
+    sp_u64(a.road + v, kUnreached | road_cost(lp_u64(a.road + v)));
+  }
 }
 
 // ---- backtrace (wave 0) ---------------------------------------------------------------------
+// Lane k probes neighbour k: its word beside the voxel's mask, one memory step per path vertex.
 __device__ __forceinline__ void backtrace(const TraceArgs &a, Shared &sh, int t, int count, int *walk) {
   if (threadIdx.x >= 64) return;
   const int lane = threadIdx.x;
-  const int ok_lane = lane < 26 ? lane : 0;
+  const bool on = lane < 26;
+  const int off = on ? nb_offset(on ? lane : 0, a.d) : 0;
+  const unsigned rank = on ? unsigned(kD3Rank[on ? lane : 0]) : 64u;
   int cur = (int)(unsigned)(sh.rail_best & 0xFFFFFFFFULL);
   int kept = 0;
   bool first = true;
   for (;;) {
     int kb = -1;
-    const unsigned m = in_mask(a, cur);  // the predecessor's step to cur must be permitted
     if (cur != t) {
-      float du = kInf;
-      if (lane < 26 && ((m >> lane) & 1u)) {
-        int u = cur + nb_offset(ok_lane, a.d);
-        if (rec_pdrf(a.rec, u) != 0.0f) du = __uint_as_float(word_dist_bits(lp_u64(&a.rec[u].word)));
-      }
-      int db = __float_as_int(du);
-      int mb = wave_min(db);
-      if (mb < 0x7f800000) kb = wave_min(db == mb ? lane : 64);
+      const unsigned m = in_mask(a, cur);  // the predecessor's step to cur must be permitted
+      const unsigned long long w = lp_u64(a.road + (long long)cur + off);  // padded: readable whatever the mask
+      unsigned db = kInfBits;
+      if (on && ((m >> lane) & 1u) && road_cost(w) != 0u) db = road_dist(w);
+      const unsigned mb = wave_min_u32(db);
+      if (mb < kInfBits) kb = __ffsll((long long)ballot(db == mb)) - 1;
     }
     if (first && kb >= 0) {  // the join at u = cur + N[kb]: u's first rail in dijkstra3d order
       const int u = cur + nb_offset(kb, a.d);
-      const unsigned mu = (rec_meta(a.rec, u) & kNbrBits);
-      int key = 64;
-      if (lane < 26 && ((mu >> lane) & 1u) && rec_pdrf(a.rec, u + nb_offset(ok_lane, a.d)) == 0.0f) key = kD3Rank[lane];
-      int r = wave_min(key);
-      if (r < 26) {
+      const unsigned mu = mask_of(a, u);
+      const unsigned long long w = lp_u64(a.road + (long long)u + off);
+      const unsigned r = wave_min_u32(on && ((mu >> lane) & 1u) && road_cost(w) == 0u ? rank : 64u);
+      if (r < 26u) {
         int ks = kD3Inv[r];
         cur = u + nb_offset(ks, a.d);
         kb = kOpp[ks];
@@ -505,34 +437,41 @@ __device__ __forceinline__ void backtrace(const TraceArgs &a, Shared &sh, int t,
 // bands of flood_lab_nf, batched_coop.inc:125-267) gives every voxel of the label its
 // vertex-weighted distance over the PDRF; parents_lab (batched_regular.inc:113-134) then takes
 // the same-label neighbour of smallest distance, first k on ties (-1 at the root and at voxels the
-// run does not reach, as a label that filled holes split has), and the words go back to ~0.
+// run does not reach, as a label that filled holes split has), and the words go back to unreached.
 // Returns the railroad's status: kNoRail is the complete field; kRailFound means the run met a
 // voxel of PDRF 0 besides the root (it would stop there as at a rail; PDRF underflows to 0 only for
 // extreme exponents), and the label is ejected; kStalled / kOverflowed end the label as failed.
-__device__ __forceinline__ int parent_field(const TraceArgs &a, Shared &sh, int root, const int *voxels, int count,
-                                            const Front &na, const Front &nb, int *l2, int *l3, int *touched) {
+template <bool Wide>
+__device__ __forceinline__ int parent_field(const TraceArgs &a, Shared &sh, const Lane<Wide> &ln, int root, const int *voxels,
+                                            int count, const Lists &l) {
   for (int j = threadIdx.x; j < count; j += blockDim.x) g_st(a.parent + g_ld(voxels + j), -1);  // unreached: no parent
   __syncthreads();
-  const int status = railroad(a, sh, root, count, na, nb, l2, l3, touched, true);
-  const int nt = sh.n_touched;
-  for (int j = threadIdx.x; j < nt; j += blockDim.x) {
-    const int v = g_ld(touched + j);
-    const unsigned dv = word_dist_bits(lp_u64(&a.rec[v].word));
-    int p = -1;
-    if (v != root && dv != 0u && dv < 0x7f800000u) {
-      unsigned m = in_mask(a, v), best = 0x7f800000u;
-      while (m) {  // ascending k: the first of equal distances stays
-        const int k = __ffs(m) - 1;
-        m &= m - 1;
-        const int u = v + sh.off[k];
-        const unsigned du = word_dist_bits(lp_u64(&a.rec[u].word));
-        if (du < best) { best = du; p = u; }
-      }
+  const int status = railroad(a, sh, ln, root, count, l, true);
+  const int nt = sh.n[kTouched];
+  constexpr int P = kMaxPairs;
+  for (int b = ln.wave * 2 * P; b < nt; b += kWaves * 2 * P) {  // half a wave per voxel, a lane per neighbour
+    int v[P];
+    unsigned long long w[P];
+    unsigned m[P];
+#pragma unroll
+    for (int p = 0; p < P; ++p) v[p] = g_ld(l.touched + min(b + 2 * p + ln.half, nt - 1));
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      m[p] = in_mask(a, v[p]);
+      w[p] = g_ld(word_at(a.road0, ln.at(v[p])));
     }
-    g_st(a.parent + v, p);
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const unsigned dv = unsigned(__shfl(int(road_dist(w[p])), ln.half * 32 + kCentre, 64));
+      const unsigned du = m[p] & ln.bit ? road_dist(w[p]) : kInfBits;
+      const unsigned best = half_min(du);
+      const unsigned k = half_min(du == best && ln.bit ? unsigned(ln.k) : 64u);  // the first k of equal distances
+      const bool has = v[p] != root && dv != 0u && dv < kInfBits && best < kInfBits;
+      if (ln.slot == 0) g_st(a.parent + v[p], has ? v[p] + nb_offset(int(k), a.d) : -1);  // (the last voxel repeats past the end)
+    }
   }
   __syncthreads();
-  for (int j = threadIdx.x; j < nt; j += blockDim.x) sp_u64(&a.rec[g_ld(touched + j)].word, kMaxKey);
+  road_restore(a, sh, l.touched);
   __syncthreads();
   return status;
 }
@@ -556,14 +495,27 @@ __device__ __forceinline__ void parent_walk(const TraceArgs &a, Shared &sh, int 
 }
 
 // ---- invalidation ---------------------------------------------------------------------------
-// A claim word is (bottleneck bits << 32) | (source << 1) | queued: claims order by (bottleneck,
-// source), and the improving atomicMin returns whether the voxel is already queued for the next
+// A claim word is (bottleneck bits << 32) | (source + 1) << 1 | queued: claims order by (bottleneck,
+// source), and the improving atomic minimum returns whether the voxel is already queued for the next
 // round (an equal claim never re-queues). A round's snapshot clears the queued bit with the atomic
-// that reads the claim. ~0 is unclaimed (and not queued).
+// that reads the claim. kFree is unclaimed, kDead invalidated.
+//
+// An offer whose bottleneck lies beyond the band [.., hi) takes the same atomic minimum: a word at or
+// above hi is then a waiting voxel's best offer so far, which no claim of the band depends on. Its
+// first offer (old word free) lists the voxel; at the band's end the waiting voxels whose word fell
+// into the next band are its first front, already queued. The reference pulls instead: at the band's end
+// every waiting voxel takes the smallest (max(bottleneck, distance), source) over its claimed
+// neighbours' final claims. Both are the same minimum, because every claimed voxel offers its final
+// claim to all its neighbours, with one exception: a voxel whose claim improves after it offered
+// (0.2 % of the claims of the 512^3 workload) leaves offers of the old claim behind. Those voxels
+// are noted (kStale), and before the band ends their waiting neighbours' words are replaced by
+// exact pulls. Measured on that workload's slowest label: 711 k pulls of 26 neighbours each became as
+// many single word reads.
+__device__ __forceinline__ unsigned claim_low(unsigned su) { return (su + 1u) << 1 | 1u; }
 __device__ __forceinline__ unsigned long long claim_word(unsigned mb, unsigned su) {
-  return ((unsigned long long)mb << 32) | ((unsigned long long)su << 1) | 1ULL;
+  return ((unsigned long long)mb << 32) | claim_low(su);
 }
-__device__ __forceinline__ unsigned claim_source(unsigned long long w) { return (unsigned)w >> 1; }
+__device__ __forceinline__ unsigned claim_source(unsigned long long w) { return ((unsigned)w >> 1) - 1u; }
 
 // The invalidation ball around source s: scale * DBF(s) + constant. Every source of an
 // invalidation is a voxel of its path, so the radii are staged once in an LDS table of (source,
@@ -578,248 +530,210 @@ __device__ __forceinline__ float source_radius(const TraceArgs &a, const Ball &b
   const unsigned long long e = tab[radius_slot(s)];
   return (unsigned)(e >> 32) == s ? __uint_as_float((unsigned)e) : ball_radius(ball, g_ld(a.dbf + s));
 }
-// An improving claim whose old word says the voxel still has to be queued.
-__device__ __forceinline__ bool needs_queue(unsigned long long old) { return old == kMaxKey || !(old & 1ULL); }
 
-__device__ __forceinline__ float offer_distance(const TraceArgs &a, int x, int y, int z, int qx, int qy, int qz) {
-  float dx = a.wx * (float)(x - qx), dy = a.wy * (float)(y - qy), dz = a.wz * (float)(z - qz);
+// Distance over voxel offsets (whole numbers, exact as floats).
+__device__ __forceinline__ float offset_distance(const TraceArgs &a, float ox, float oy, float oz) {
+  float dx = a.wx * ox, dy = a.wy * oy, dz = a.wz * oz;
   return sqrtf(dx * dx + dy * dy + dz * dz);
 }
 
-// A neighbour whose offer is beyond the band waits for it: if its record showed it unclaimed and
-// not yet waiting, one atomic sets the waiting flag and its winner reports it in p.far, to be
-// pulled at the band boundary. (A voxel claimed meanwhile may be listed too: the boundary skips
-// claimed entries; a claimed voxel keeps the flag until the claimed set dies.)
-__device__ __forceinline__ bool may_wait(const RecWords &r) { return r.w == 0xFFFFFFFFu && !(r.y & kWaiting); }
-
-// Masked neighbours B..E-1 of u at once: alive and key loads, then the claim and waiting atomics,
-// in flight together. Only the key's high word (the bottleneck) is pre-loaded: a claim whose
-// bottleneck is above it cannot win and issues no atomic. The outcome is a set of bit masks.
-template <int B, int E>
-__device__ __forceinline__ void offer_part(const TraceArgs &a, const int *off, int u, unsigned m, int x, int y, int z,
-                                           int qx, int qy, int qz, unsigned su, unsigned mu, float maxd, unsigned hi,
-                                           Pushes &p) {
-  bool al[E - B];
-  unsigned kh[E - B], fresh = 0;
-  for_nb<B, E>([&](auto K) {
-    constexpr int k = decltype(K)::value, i = k - B;
-    const bool on = (m >> k) & 1u;
-    const RecWords r = on ? rec_load(a.rec, u + nb_offset<k>(a.d)) : RecWords{0u, 0u, 0u, 0u};
-    al[i] = r.y & kAlive;
-    kh[i] = r.w;
-    if (may_wait(r)) fresh |= 1u << k;
-  });
-  unsigned mbs[E - B];
-  unsigned wait = 0;
-  unsigned long long old[E - B];
-  for_nb<B, E>([&](auto K) {
-    constexpr int k = decltype(K)::value, i = k - B;
-    const float d = offer_distance(a, x + kDX[k], y + kDY[k], z + kDZ[k], qx, qy, qz);
-    const unsigned mb = max(__float_as_uint(d), mu);  // M = max(M[u], d)
-    mbs[i] = mb;
-    old[i] = 0;  // "no improvement" unless the atomic says otherwise
-    if (al[i] && d < maxd) {
-      if (mb >= hi) {
-        if ((fresh >> k) & 1u) {
-          wait |= 1u << k;
-          old[i] = g_or(&a.rec[u + nb_offset<k>(a.d)].meta, kWaiting);
-        }
-      } else if (kh[i] >= mb) {
-        old[i] = g_min(&a.rec[u + nb_offset<k>(a.d)].word, claim_word(mb, su));
-      }
-    }
-  });
-  for_nb<B, E>([&](auto K) {
-    constexpr int k = decltype(K)::value, i = k - B;
-    if ((wait >> k) & 1u) {  // old: the meta before the waiting flag
-      if (!(old[i] & kWaiting)) p.far |= 1u << k;
-    } else if (old[i] > claim_word(mbs[i], su)) {  // won (old is 0 where no atomic was issued)
-      if (old[i] == kMaxKey) p.touched |= 1u << k;
-      if (needs_queue(old[i])) p.near |= 1u << k;
-    }
-  });
-}
-
-// Neighbours kb..kb+cnt-1 (those set in m; cnt <= kSpan) of u: offer_part with a run-time span.
-__device__ __forceinline__ void offer_span(const TraceArgs &a, const int *off, int u, unsigned m, int kb, int cnt, int x,
-                                           int y, int z, int qx, int qy, int qz, unsigned su, unsigned mu, float maxd,
-                                           unsigned hi, Pushes &p) {
-  constexpr int S = kSpan;
-  bool al[S];
-  unsigned kh[S], fresh = 0;
-  int v[S];
-#pragma unroll
-  for (int j = 0; j < S; ++j) {
-    const int k = kb + j;
-    const bool on = j < cnt && ((m >> k) & 1u);
-    v[j] = u + off[on ? k : 0];
-    const RecWords r = on ? rec_load(a.rec, v[j]) : RecWords{0u, 0u, 0u, 0u};
-    al[j] = r.y & kAlive;
-    kh[j] = r.w;
-    if (may_wait(r)) fresh |= 1u << j;
-  }
-  unsigned mbs[S];
-  unsigned wait = 0;  // bit j: slot j's atomic set the waiting flag
-  unsigned long long old[S];
-#pragma unroll
-  for (int j = 0; j < S; ++j) {
-    const int k = j < cnt ? kb + j : 0;  // slots past the span are off (al[j] false)
-    const float d = offer_distance(a, x + nb_dx(k), y + nb_dy(k), z + nb_dz(k), qx, qy, qz);
-    const unsigned mb = max(__float_as_uint(d), mu);  // M = max(M[u], d)
-    mbs[j] = mb;
-    old[j] = 0;  // "no improvement" unless the atomic says otherwise
-    if (al[j] && d < maxd) {
-      if (mb >= hi) {
-        if ((fresh >> j) & 1u) {
-          wait |= 1u << j;
-          old[j] = g_or(&a.rec[v[j]].meta, kWaiting);
-        }
-      } else if (kh[j] >= mb) {
-        old[j] = g_min(&a.rec[v[j]].word, claim_word(mb, su));
-      }
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < S; ++j) {
-    const int k = kb + j;
-    if ((wait >> j) & 1u) {  // old: the meta before the waiting flag
-      if (!(old[j] & kWaiting)) p.far |= 1u << k;
-    } else if (old[j] > claim_word(mbs[j], su)) {  // won
-      if (old[j] == kMaxKey) p.touched |= 1u << k;
-      if (needs_queue(old[j])) p.near |= 1u << k;
-    }
-  }
-}
-
-// One invalidation round over a front of at most kGroupFront entries, a group of lanes per entry.
-// The group's first lane takes the entry's snapshot (re-arming it) and its ball radius before the
-// barrier that separates the round's snapshots from its offers; the values stay in registers.
-__device__ __forceinline__ void offer_groups(const TraceArgs &a, const Ball &ball, Shared &sh, const Front &cur, int nc, unsigned hi,
-                                             const Front &nxt, int *n_nxt, int *far, int *touched) {
-  const Group q = group_of(nc);
+// A front entry's snapshot, in the lane that took it.
+struct Offer {
   int u = 0;
-  unsigned m = 0;
-  unsigned long long ku = kMaxKey;
-  float maxd = 0.0f;
-  if (q.i < nc) {
-    u = front_get(cur, q.i);
-    m = rec_meta(a.rec, u) & kNbrBits;
-    if (q.g == 0) {
-      ku = g_and(&a.rec[u].word, ~1ULL);
-      maxd = source_radius(a, ball, sh.radius, claim_source(ku));
-    }
-  }
-  __syncthreads();
-  ku = __shfl(ku, q.lead, 64);
-  maxd = __shfl(maxd, q.lead, 64);
-  Pushes p;
-  if (q.i < nc) {
-    const unsigned su = claim_source(ku), mu = (unsigned)(ku >> 32);
+  unsigned m = 0;                          // neighbours it offers to
+  unsigned mu = 0, low = 0;                // its claim's bottleneck; its source as an offer's low half
+  float maxd = 0.0f;                       // the source's ball
+  float ox = 0.0f, oy = 0.0f, oz = 0.0f;   // its place relative to the source
+  __device__ __forceinline__ void set(const TraceArgs &a, const Ball &ball, const Shared &sh, unsigned long long ku) {
+    const unsigned su = claim_source(ku);
+    mu = unsigned(ku >> 32);
+    low = claim_low(su);
+    maxd = source_radius(a, ball, sh.radius, su);
     int x, y, z, qx, qy, qz;
-    unravel(u, a.d, x, y, z);
-    unravel(int(su), a.d, qx, qy, qz);
-    offer_span(a, sh.off, u, m, q.kb, q.cnt, x, y, z, qx, qy, qz, su, mu, maxd, hi, p);
+    place(a, u, x, y, z);
+    place(a, int(su), qx, qy, qz);
+    ox = float(x - qx);
+    oy = float(y - qy);
+    oz = float(z - qz);
   }
-  emit_neighbours(touched, &sh.n_touched, p.touched, u, sh.off);
-  emit_front(nxt, n_nxt, p.near, u, sh.off);
-  emit_neighbours(far, &sh.n_far, p.far, u, sh.off);
+};
+
+// Where a round's offers go.
+struct OfferLists {
+  Front nxt;
+  int n_nxt;  // claimed and to be queued
+  Far far;
+  int n_far;  // waiting
+  int *touched, *stale;
+  int stale_cap;
+  unsigned hi;  // the band's end
+};
+
+// Offers of the entries held by lanes from .. from + 2P - 1 (their masks 0 beyond the wave's batch) to
+// their neighbours, u the entries and w the neighbours' words, loaded at any time of the round: an
+// offer whose bottleneck is above the word's cannot win. The others go to the wave's stage.
+template <int P, bool Wide, class Flush>
+__device__ __forceinline__ void offer_batch(const TraceArgs &a, const Lane<Wide> &ln, const Offer &e, int from, const int (&u)[P],
+                                            const unsigned long long (&w)[P], Stage &st, int &staged, Flush &&flush) {
+  staged_pairs<P>([&](int p) {
+    const int at = from + 2 * p;
+    const unsigned m = of_entry(ln, e.m, at), mu = of_entry(ln, e.mu, at), low = of_entry(ln, e.low, at);
+    const float maxd = of_entry(ln, e.maxd, at);
+    const float d = offset_distance(a, of_entry(ln, e.ox, at) + ln.dx, of_entry(ln, e.oy, at) + ln.dy, of_entry(ln, e.oz, at) + ln.dz);
+    const unsigned mb = max(__float_as_uint(d), mu);  // M = max(M[u], d)
+    stage_put(st, staged, ((m & ln.bit) != 0u) & (unsigned(w[p]) != 0u) & (d < maxd) & (unsigned(w[p] >> 32) >= mb),
+              u[p] + ln.off, ((unsigned long long)mb << 32) | low);
+  }, flush);
 }
 
-__device__ __forceinline__ void offer_all(const TraceArgs &a, const int *off, int u, unsigned m, unsigned su, unsigned mu,
-                                          float maxd, unsigned hi, Pushes &p) {
-  int x, y, z, qx, qy, qz;
-  unravel(u, a.d, x, y, z);
-  unravel(int(su), a.d, qx, qy, qz);
-  for_parts<kNbBatch>(m, [&](auto B, auto E) {
-    offer_part<decltype(B)::value, decltype(E)::value>(a, off, u, m, x, y, z, qx, qy, qz, su, mu, maxd, hi, p);
-  });
-}
-
-// The best claim waiting voxel c (at x, y, z) can pull from its claimed neighbours B..E-1: the
-// smallest (max(bottleneck, distance to the neighbour's source), source) among those whose source's
-// ball holds c. Claim loads, then the sources' DBF loads, each issued together.
-template <int B, int E>
-__device__ __forceinline__ void pull_part(const TraceArgs &a, const Ball &ball, const unsigned long long *tab, int c,
-                                          unsigned mc, int x, int y, int z, unsigned long long &best) {
-  unsigned long long ku[E - B];
-  for_nb<B, E>([&](auto K) {
-    constexpr int k = decltype(K)::value, i = k - B;
-    ku[i] = (mc >> k) & 1u ? lp_u64(&a.rec[c + nb_offset<k>(a.d)].word) : kMaxKey;
-  });
-  float r[E - B];
-  for_nb<B, E>([&](auto K) {
-    constexpr int k = decltype(K)::value, i = k - B;
-    r[i] = ku[i] != kMaxKey ? source_radius(a, ball, tab, claim_source(ku[i])) : 0.0f;
-  });
-  for_nb<B, E>([&](auto K) {
-    constexpr int k = decltype(K)::value, i = k - B;
-    if (ku[i] == kMaxKey) return;
-    const unsigned su = claim_source(ku[i]);
-    int qx, qy, qz;
-    unravel(int(su), a.d, qx, qy, qz);
-    const float d = offer_distance(a, x, y, z, qx, qy, qz);
-    if (d >= r[i]) return;
-    const unsigned mb = max(__float_as_uint(d), (unsigned)(ku[i] >> 32));
-    const unsigned long long cand = ((unsigned long long)mb << 32) | su;
-    if (cand < best) best = cand;
-  });
-}
-
-// Neighbours kb..kb+cnt-1 (those set in mc; cnt <= kSpan) of waiting voxel c: pull_part with a
-// run-time span.
-__device__ __forceinline__ void pull_span(const TraceArgs &a, const Ball &ball, const unsigned long long *tab, const int *off, int c,
-                                          unsigned mc, int kb, int cnt, int x, int y, int z, unsigned long long &best) {
-  constexpr int S = kSpan;
-  unsigned long long ku[S];
-#pragma unroll
-  for (int j = 0; j < S; ++j) {
-    const int k = kb + j;
-    ku[j] = j < cnt && ((mc >> k) & 1u) ? lp_u64(&a.rec[c + off[k]].word) : kMaxKey;
-  }
-  float r[S];
-#pragma unroll
-  for (int j = 0; j < S; ++j) r[j] = ku[j] != kMaxKey ? source_radius(a, ball, tab, claim_source(ku[j])) : 0.0f;
-#pragma unroll
-  for (int j = 0; j < S; ++j) {
-    if (ku[j] == kMaxKey) continue;
-    const unsigned su = claim_source(ku[j]);
-    int qx, qy, qz;
-    unravel(int(su), a.d, qx, qy, qz);
-    const float d = offer_distance(a, x, y, z, qx, qy, qz);
-    if (d >= r[j]) continue;
-    const unsigned mb = max(__float_as_uint(d), (unsigned)(ku[j] >> 32));
-    const unsigned long long cand = ((unsigned long long)mb << 32) | su;
-    if (cand < best) best = cand;
-  }
-}
-
-// Band-boundary pulls of at most kGroupFront waiting entries, a group of lanes per entry, the
-// group's minimum folded by shuffles: pull[i] = kClaimed (claimed meanwhile), the best claim, or
-// kMaxKey.
-__device__ __forceinline__ void pull_groups(const TraceArgs &a, const Ball &ball, Shared &sh, const int *far, int nf,
-                                            unsigned long long *pull) {
-  const Group q = group_of(nf);
-  unsigned long long best = kMaxKey;
-  bool claimed = false;
-  if (q.i < nf) {
-    const int c = lp_i(far + q.i);
-    const unsigned long long w = lp_u64(&a.rec[c].word);
-    const unsigned mc = in_mask(a, c);
-    claimed = w != kMaxKey;
-    if (!claimed) {
-      int x, y, z;
-      unravel(c, a.d, x, y, z);
-      pull_span(a, ball, sh.radius, sh.off, c, mc, q.kb, q.cnt, x, y, z, best);
+// The staged offers of a wave (full groups, or all of them). lowest: this thread's least waiting one.
+__device__ __forceinline__ void offer_minima(const TraceArgs &a, Shared &sh, Stage &st, int &staged, bool all,
+                                             const OfferLists &to, unsigned &lowest) {
+  stage_take(st, staged, all, [&](bool on, int v, unsigned long long nv) {
+    unsigned long long old = 0;  // "no improvement" unless the atomic says otherwise
+    if (on) old = g_min(a.claim + v, nv);
+    const unsigned ohi = unsigned(old >> 32), mb = unsigned(nv >> 32);
+    const bool won = old > nv, now = mb < to.hi, fresh = ohi >= to.hi;
+    const bool claimed = won & now & fresh, waits = won & !now & (ohi == ~0u);
+    const bool again = won & now & !fresh & !(unsigned(old) & 1u);  // it had offered its old claim already
+    if (won & !now) lowest = min(lowest, mb);
+    if (again) {
+      const int at = wave_slot(&sh.n[kStale]);
+      if (at < to.stale_cap) g_st(to.stale + at, v);
     }
+    Appends out;
+    if (!out.begin(sh.n, kTouched, claimed, to.n_nxt, claimed | again, to.n_far, waits)) return;
+    if (claimed) g_st(to.touched + out.place(0), v);
+    if (claimed | again) to.nxt.put(out.place(1), v);
+    if (waits) to.far.put(out.place(2), v);
+  });
+}
+
+// One invalidation round over nc entries: every snapshot before any offer. A wave's entries stay in
+// its registers (up to one per lane) for fronts of up to a workgroup; longer fronts keep their
+// snapshots in device memory. Fronts that fit one batch per wave load their neighbours' words before
+// the barrier.
+template <bool Wide>
+__device__ __forceinline__ void offer_round(const TraceArgs &a, const Ball &ball, Shared &sh, const Lane<Wide> &ln,
+                                            const Front &cur, int nc, const OfferLists &to, unsigned long long *snap,
+                                            unsigned &lowest) {
+  Stage &st = sh.stage[ln.wave];
+  int staged = 0;
+  auto flush = [&] { offer_minima(a, sh, st, staged, false, to, lowest); };
+  if (nc <= kWaves * 2 * kMaxPairs) {
+    with_pairs<kMaxPairs>(nc, kWaves, [&](auto Pairs) {
+      constexpr int P = decltype(Pairs)::value;
+      const int b = ln.wave * 2 * P;
+      Offer e;
+      int u[P];
+      unsigned long long w[P];
+      if (b < nc) {
+        e.u = batch_entries<P>(ln, cur, b, nc, u);
+        const bool mine = ln.lane < min(2 * P, nc - b);
+        unsigned long long ku = 0;
+        if (mine) {
+          ku = g_and(a.claim + e.u, ~1ULL);
+          e.m = mask_of(a, e.u);
+        }
+#pragma unroll
+        for (int p = 0; p < P; ++p) w[p] = g_ld(word_at(a.claim0, ln.at(u[p])));
+        if (mine) e.set(a, ball, sh, ku);
+      }
+      __syncthreads();
+      if (b < nc) offer_batch<P>(a, ln, e, 0, u, w, st, staged, flush);
+    });
+    offer_minima(a, sh, st, staged, true, to, lowest);
+    return;
   }
-  for (int o = 1; o < q.G; o <<= 1) {
-    const unsigned long long other = __shfl_xor(best, o, 64);
-    best = other < best ? other : best;
+  constexpr int P = kMaxPairs;
+  int u[P];
+  unsigned long long w[P];
+  if (nc <= kBlock) {
+    const int per = (nc + kWaves - 1) / kWaves, b = ln.wave * per, n = min(per, nc - b);
+    Offer e;
+    if (ln.lane < n) {
+      e.u = cur.get(b + ln.lane);
+      e.m = mask_of(a, e.u);
+      e.set(a, ball, sh, g_and(a.claim + e.u, ~1ULL));
+    }
+    __syncthreads();
+    for (int from = 0; from < n; from += 2 * P) {
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        u[p] = int(of_entry(ln, unsigned(e.u), from + 2 * p));
+        w[p] = g_ld(word_at(a.claim0, ln.at(u[p])));
+      }
+      offer_batch<P>(a, ln, e, from, u, w, st, staged, flush);
+    }
+    offer_minima(a, sh, st, staged, true, to, lowest);
+    return;
   }
-  if (q.g == 0 && q.i < nf) {
-    g_st(pull + q.i, claimed ? kClaimed : best);
-    if (!claimed && best != kMaxKey) atomicMin(&sh.lowest, (unsigned)(best >> 32));
+  for (int i = threadIdx.x; i < nc; i += blockDim.x) g_st(snap + i, g_and(a.claim + cur.get(i), ~1ULL));
+  __syncthreads();
+  for (int b = ln.wave * 2 * P; b < nc; b += kWaves * 2 * P) {
+    Offer e;
+    e.u = batch_entries<P>(ln, cur, b, nc, u);
+#pragma unroll
+    for (int p = 0; p < P; ++p) w[p] = g_ld(word_at(a.claim0, ln.at(u[p])));
+    if (ln.lane < min(2 * P, nc - b)) {
+      e.m = mask_of(a, e.u);
+      e.set(a, ball, sh, g_ld(snap + b + ln.lane));
+    }
+    offer_batch<P>(a, ln, e, 0, u, w, st, staged, flush);
   }
+  offer_minima(a, sh, st, staged, true, to, lowest);
+}
+
+// The exact pulls of list entries b .. b + 1 (n of them), a half each: the entry's word, when it waits,
+// becomes the smallest (max(bottleneck, distance to the neighbour's source), source) among its
+// claimed neighbours whose source's ball holds it, or free. An entry may occur twice: claimed
+// words do not change here, so both write the same.
+template <bool Wide>
+__device__ __forceinline__ void pull_pair(const TraceArgs &a, const Ball &ball, const Shared &sh, const Lane<Wide> &ln, int c,
+                                          bool on, unsigned hi) {
+  const unsigned m = in_mask(a, c);
+  const unsigned long long w = lp_u64(word_at(a.claim0, ln.at(c)));
+  unsigned long long best = kMaxKey;
+  if ((m & ln.bit) && unsigned(w) != 0u && unsigned(w >> 32) < hi) {
+    const unsigned su = claim_source(w);
+    int x, y, z, qx, qy, qz;
+    place(a, c, x, y, z);
+    place(a, int(su), qx, qy, qz);
+    const float d = offset_distance(a, float(x - qx), float(y - qy), float(z - qz));
+    if (d < source_radius(a, ball, sh.radius, su)) best = claim_word(max(__float_as_uint(d), unsigned(w >> 32)), su);
+  }
+  best = half_min_u64(best);
+  if (on && ln.slot == kCentre && unsigned(w >> 32) >= hi && w != kFree) sp_u64(a.claim + c, best);
+}
+
+// The waiting words that stale offers may have set, made exact: those of the noted voxels' neighbours,
+// or every waiting one when the notes overflowed. Ends with a barrier.
+template <bool Wide>
+__device__ __forceinline__ void pull_stale(const TraceArgs &a, const Ball &ball, Shared &sh, const Lane<Wide> &ln, const Far &far,
+                                           int nf, int ns, const OfferLists &to, int *dirty) {
+  const bool all = ns > to.stale_cap;
+  if (!all) {
+    for (int i = ln.wave * 2; i < ns; i += kWaves * 2) {
+      const int u = g_ld(to.stale + min(i + ln.half, ns - 1));
+      const unsigned m = i + ln.half < ns ? mask_of(a, u) : 0u;
+      const unsigned long long w = lp_u64(word_at(a.claim0, ln.at(u)));
+      if ((m & ln.bit) && unsigned(w >> 32) >= to.hi && w != kFree) {
+        const int at = wave_slot(&sh.n[kDirty]);
+        if (at < to.stale_cap) g_st(dirty + at, u + ln.off);
+      }
+    }
+    __syncthreads();
+  }
+  const int nd = sh.n[kDirty];
+  const bool listed = !all && nd <= to.stale_cap;
+  const int n = listed ? nd : nf;
+  for (int i = ln.wave * 2; i < n; i += kWaves * 2) {
+    const int j = min(i + ln.half, n - 1);
+    pull_pair(a, ball, sh, ln, listed ? g_ld(dirty + j) : far.get(j), i + ln.half < n, to.hi);
+  }
+  if (threadIdx.x == 0) sh.prof[14] += n;
+  __syncthreads();
+  if (threadIdx.x == 0) sh.n[kStale] = sh.n[kDirty] = 0;  // appended to again after the promotion's barrier
 }
 
 __device__ __forceinline__ int band_of(unsigned mbits, float delta, int kmin) {
@@ -830,121 +744,100 @@ __device__ __forceinline__ int band_of(unsigned mbits, float delta, int kmin) {
   return k < kmin ? kmin : k;
 }
 
+__device__ __forceinline__ void fold_lowest(unsigned *slot, unsigned &lowest) {
+  if (any_lane(lowest != kInfBits)) {
+    lowest = wave_min_u32(lowest);
+    if (__lane_id() == 0) atomicMin(slot, lowest);
+  }
+  lowest = kInfBits;
+}
+
 // Returns false when the rounds did not converge within the budget (the label is then given up;
 // the claimed set still dies).
-__device__ __forceinline__ bool invalidate(const TraceArgs &a, const Ball &ball, Shared &sh, const int *path, int len,
-                                           int count, const Front &la, const Front &lb, int *lfar, int *lkeep,
-                                           int *touched, unsigned long long *snap, unsigned long long *pull) {
+template <bool Wide>
+__device__ __forceinline__ bool invalidate(const TraceArgs &a, const Ball &ball, Shared &sh, const Lane<Wide> &ln,
+                                           const int *path, int len, int count, const Lists &l) {
   if (threadIdx.x == 0) {
-    sh.cnt[0] = sh.cnt[1] = sh.cnt[2] = sh.n_far = sh.n_keep = sh.n_touched = 0;
-    sh.band = 0;
+    for (int j = 0; j < kCounters; ++j) sh.n[j] = 0;
+    for (int j = 0; j < 3; ++j) sh.lowest[j] = kInfBits;
   }
   for (int j = threadIdx.x; j < kRadiusSlots; j += blockDim.x) sh.radius[j] = kMaxKey;
   __syncthreads();
-  Front cur = la, nxt = lb;
-  int *far = lfar, *keep = lkeep;
-  int r = 0;  // the current list's length is sh.cnt[r]
+  OfferLists to{l.near[1], 1, l.far[0], kFar, l.touched, l.stale, 2 * count, 0u};
+  Front cur = l.near[0];
+  Far keep = l.far[1];
+  int r = 0;   // the current front's length is sh.n[r]
+  int bt = 0;  // bands so far mod 3: the waiting list's length is sh.n[kFar + bt], its minimum sh.lowest[bt]
   for (int j = threadIdx.x; j < len; j += blockDim.x) {  // sources: path voxels still alive
     int p = g_ld(path + j);
     atomicMin(&sh.radius[radius_slot(unsigned(p))],
               ((unsigned long long)unsigned(p) << 32) | __float_as_uint(ball_radius(ball, g_ld(a.dbf + p))));
-    if (!(rec_meta(a.rec, p) & kAlive)) continue;
-    if (g_cas(&a.rec[p].word, kMaxKey, claim_word(0u, unsigned(p))) == kMaxKey) {
-      front_put(cur, wave_slot(&sh.cnt[0]), p);
-      g_st(touched + wave_slot(&sh.n_touched), p);
+    if (g_cas(a.claim + p, kFree, claim_word(0u, unsigned(p))) == kFree) {
+      cur.put(wave_slot(&sh.n[0]), p);
+      g_st(l.touched + wave_slot(&sh.n[kTouched]), p);
     }
   }
   __syncthreads();
   long long rounds = 0;  // rounds and bands so far (the same in every thread)
   const long long budget = round_budget(count);
   bool converged = true;
+  int band = 0;  // the same in every thread
+  unsigned lowest = kInfBits;
   for (;;) {
-    unsigned hi = __float_as_uint((float)(sh.band + 1) * a.delta);
+    to.hi = unsigned(__builtin_amdgcn_readfirstlane(__float_as_int((float)(band + 1) * a.delta)));
+    to.n_far = kFar + bt;
     for (;;) {  // synchronous rounds inside the band
-      const int nc = sh.cnt[r];
+      const int nc = __builtin_amdgcn_readfirstlane(sh.n[r]);
       if (nc == 0) break;
       if (++rounds > budget) { converged = false; break; }
-      const int rn = rot_next(r);
-      if (threadIdx.x == 0) { sh.cnt[rot_prev(r)] = 0; sh.prof[6] += 1; sh.prof[11] += nc; }
-      if (nc <= kGroupFront) {
-        offer_groups(a, ball, sh, cur, nc, hi, nxt, &sh.cnt[rn], far, touched);
-      } else {
-        for (int i = threadIdx.x; i < nc; i += blockDim.x)  // snapshot and re-arm in one atomic
-          g_st(snap + i, g_and(&a.rec[front_get(cur, i)].word, ~1ULL));
-        __syncthreads();
-        for (int base = 0; base < nc; base += blockDim.x) {  // uniform: every lane reaches the appends
-          const int i = base + threadIdx.x;
-          Pushes p;
-          int u = 0;
-          if (i < nc) {
-            u = front_get(cur, i);
-            const unsigned m = (rec_meta(a.rec, u) & kNbrBits);
-            const unsigned long long ku = g_ld(snap + i);
-            const unsigned su = claim_source(ku), mu = (unsigned)(ku >> 32);
-            offer_all(a, sh.off, u, m, su, mu, source_radius(a, ball, sh.radius, su), hi, p);
-          }
-          emit_neighbours(touched, &sh.n_touched, p.touched, u, sh.off);
-          emit_front(nxt, &sh.cnt[rn], p.near, u, sh.off);
-          emit_neighbours(far, &sh.n_far, p.far, u, sh.off);
-        }
-      }
+      to.n_nxt = rot_next(r);
+      if (threadIdx.x == 0) { sh.n[rot_prev(r)] = 0; sh.prof[6] += 1; sh.prof[11] += nc; }
+      offer_round(a, ball, sh, ln, cur, nc, to, l.snap, lowest);
+      fold_lowest(&sh.lowest[bt], lowest);
       __syncthreads();
-      r = rn;
-      const Front tmp = cur; cur = nxt; nxt = tmp;
+      r = to.n_nxt;
+      const Front f = cur; cur = to.nxt; to.nxt = f;
     }
-    const int nf = sh.n_far;
+    const int nf = sh.n[kFar + bt];
     if (nf == 0 || !converged || ++rounds > budget) { converged = converged && nf == 0; break; }
-    if (threadIdx.x == 0) { sh.lowest = 0x7f800000u; sh.prof[12] += nf; sh.prof[13] += 1; }
-    __syncthreads();
-    if (nf <= kGroupFront) {  // band boundary: exact pulls
-      pull_groups(a, ball, sh, far, nf, pull);
-    } else {
-      for (int i = threadIdx.x; i < nf; i += blockDim.x) {
-        int c = lp_i(far + i);
-        if (lp_u64(&a.rec[c].word) != kMaxKey) { g_st(pull + i, kClaimed); continue; }
-        const unsigned mc = in_mask(a, c);
-        int x, y, z;
-        unravel(c, a.d, x, y, z);
-        unsigned long long best = kMaxKey;
-        for_parts<kNbBatch>(mc, [&](auto B, auto E) { pull_part<decltype(B)::value, decltype(E)::value>(a, ball, sh.radius, c, mc, x, y, z, best); });
-        g_st(pull + i, best);
-        if (best != kMaxKey) atomicMin(&sh.lowest, (unsigned)(best >> 32));
-      }
-    }
-    __syncthreads();
-    if (threadIdx.x == 0 && sh.lowest != 0x7f800000u) sh.band = band_of(sh.lowest, a.delta, sh.band + 1);
-    __syncthreads();
-    hi = __float_as_uint((float)(sh.band + 1) * a.delta);
+    if (threadIdx.x == 0) { sh.prof[12] += nf; sh.prof[13] += 1; }
+    const int ns = sh.n[kStale];
+    if (ns) pull_stale(a, ball, sh, ln, to.far, nf, ns, to, reinterpret_cast<int *>(l.snap));
+    // The next band: the one that holds the least waiting offer (an offer replaced since leaves it
+    // too low at worst: an empty band).
+    const unsigned least = sh.lowest[bt];
+    if (least != kInfBits) band = band_of(least, a.delta, band + 1);
+    const unsigned next_hi = __float_as_uint((float)(band + 1) * a.delta);
+    const int bn = rot_next(bt);
     for (int i = threadIdx.x; i < nf; i += blockDim.x) {  // promote / keep waiting / drop
-      int c = lp_i(far + i);
-      unsigned long long p = g_ld(pull + i);
-      if (p == kClaimed) continue;
-      if (p == kMaxKey) { g_and(&a.rec[c].meta, ~kWaiting); continue; }
-      if ((unsigned)(p >> 32) < hi) {
-        sp_u64(&a.rec[c].word, claim_word((unsigned)(p >> 32), (unsigned)p));
-        g_st(touched + wave_slot(&sh.n_touched), c);
-        front_put(cur, wave_slot(&sh.cnt[r]), c);
-        g_and(&a.rec[c].meta, ~kWaiting);
+      const int c = to.far.get(i);
+      const unsigned long long w = lp_u64(a.claim + c);
+      const unsigned mb = unsigned(w >> 32);
+      if (mb < to.hi || w == kFree) continue;  // claimed in the band; its offer was stale
+      if (mb < next_hi) {                      // its word is the claim, queued
+        g_st(l.touched + wave_slot(&sh.n[kTouched]), c);
+        cur.put(wave_slot(&sh.n[r]), c);
       } else {
-        g_st(keep + wave_slot(&sh.n_keep), c);
+        keep.put(wave_slot(&sh.n[kFar + bn]), c);
+        lowest = min(lowest, mb);
       }
     }
+    fold_lowest(&sh.lowest[bn], lowest);
+    if (threadIdx.x == 0) {  // the third slots: last read a band ago, next written a band on
+      sh.n[kFar + rot_next(bn)] = 0;
+      sh.lowest[rot_next(bn)] = kInfBits;
+    }
     __syncthreads();
-    if (threadIdx.x == 0) { sh.n_far = sh.n_keep; sh.n_keep = 0; }
-    int *tmp = far; far = keep; keep = tmp;
-    __syncthreads();
+    const Far f = to.far; to.far = keep; keep = f;
+    bt = bn;
   }
   __syncthreads();
-  const int nt = sh.n_touched;
+  const int nt = sh.n[kTouched];
   if (threadIdx.x == 0) {
     g_add(reinterpret_cast<unsigned long long *>(a.counters + 6), (unsigned long long)nt);
     if (!converged) report_failure(a, kStalled);
   }
-  for (int j = threadIdx.x; j < nt; j += blockDim.x) {  // the claimed set dies
-    int v = g_ld(touched + j);
-    sp_u64(&a.rec[v].word, kMaxKey);
-    g_and(&a.rec[v].meta, ~(kAlive | kWaiting));
-  }
+  for (int j = threadIdx.x; j < nt; j += blockDim.x) sp_u64(a.claim + g_ld(l.touched + j), kDead);  // the claimed set dies
   __syncthreads();
   return converged;
 }
@@ -983,7 +876,7 @@ __device__ __forceinline__ int next_target(const TraceArgs &a, Shared &sh, int L
       long long j = c + r * blockDim.x + threadIdx.x;
       if (j < e) {
         int v = g_ld(a.order + j);
-        if ((rec_meta(a.rec, v) & kAlive)) atomicMin(&sh.found, int(j - c));
+        if (lp_u64(a.claim + v) != kDead) atomicMin(&sh.found, int(j - c));
       }
     }
     __syncthreads();
@@ -1038,28 +931,27 @@ __device__ __forceinline__ void soma_trim(const TraceArgs &a, Shared &sh, int *w
 // The somata's own balls (lockstep.cu:197-206), one workgroup per soma label, before the trace:
 // the ball of the soma parameters around the root dies, and the label's path budget becomes its
 // voxel count minus what the ball took (or max_paths), none when the manual targets reach it.
+template <bool Wide>
 __global__ void __launch_bounds__(kBlock) soma_balls(const TraceArgs *__restrict__ all, const int2 *__restrict__ queue,
                                                     int nqueue) {
   __shared__ Shared sh;
   const int2 q = queue[blockIdx.x];
   const TraceArgs a = all[__builtin_amdgcn_readfirstlane(q.x)];
   const int L = __builtin_amdgcn_readfirstlane(q.y);
-  if (threadIdx.x < 26) sh.off[threadIdx.x] = nb_offset(int(threadIdx.x), a.d);
-  const int seg = g_ld(a.seg_start + L), count = g_ld(a.seg_count + L);
-  // lists 2 and 3 (the far lists) hold two entries per voxel: segment 2 * seg
-  int *l2 = a.lists[2] + 2LL * seg, *l3 = a.lists[3] + 2LL * seg, *l4 = a.lists[4] + seg, *walk = a.lists[5] + seg;
-  const Front na{a.lists[0] + seg, sh.front[0]}, nb{a.lists[1] + seg, sh.front[1]};
-  unsigned long long *s0 = a.snaps[0] + seg, *s1 = a.snaps[1] + seg;
+  const Lane<Wide> ln = lane_of<Wide>(a.d, kBlock);
+  const int seg = __builtin_amdgcn_readfirstlane(g_ld(a.seg_start + L));  // uniform: scalar registers
+    const int count = __builtin_amdgcn_readfirstlane(g_ld(a.seg_count + L));
+  const Lists l = lists_of(a, sh, seg);
   const SomaLabel *soma = a.soma + L;
   if (threadIdx.x == 0) {
     for (int j = 0; j < kProf; ++j) sh.prof[j] = 0;
-    g_st(walk, int(g_ld(a.root + L)));
+    g_st(l.walk, int(g_ld(a.root + L)));
   }
   __syncthreads();
-  invalidate(a, soma->ball, sh, walk, 1, count, na, nb, l2, l3, l4, s0, s1);
+  invalidate(a, soma->ball, sh, ln, l.walk, 1, count, l);
   if (threadIdx.x == 0) {
     const long long limit = g_ld(&soma->max_paths);
-    const long long budget = limit >= 0 ? limit : (long long)count - sh.n_touched;
+    const long long budget = limit >= 0 ? limit : (long long)count - sh.n[kTouched];
     const int manual = g_ld(a.mcount + L) + (a.acount ? g_ld(a.acount + L) : 0);
     g_st(a.maxp + L, manual >= budget ? 0 : int(budget < INT32_MAX ? budget : INT32_MAX));
   }
@@ -1070,6 +962,7 @@ __global__ void __launch_bounds__(kBlock) soma_balls(const TraceArgs *__restrict
 // from item nfixed on. Workgroups go to the XCDs in turn (w mod 8), so the largest labels start on
 // different XCDs instead of wherever the first atomics land, and no XCD's L2 carries more than
 // its share of them.
+template <bool Wide>
 __global__ void __launch_bounds__(kBlock) trace_labels(const TraceArgs *__restrict__ all, const int2 *__restrict__ queue,
                                                       int nqueue, int nfixed, int *next) {
   __shared__ Shared sh;
@@ -1083,12 +976,11 @@ __global__ void __launch_bounds__(kBlock) trace_labels(const TraceArgs *__restri
     const int sample = __builtin_amdgcn_readfirstlane(q.x);
     const TraceArgs a = all[sample];  // uniform: scalar registers
     const int L = __builtin_amdgcn_readfirstlane(q.y);
-    if (threadIdx.x < 26) sh.off[threadIdx.x] = nb_offset(int(threadIdx.x), a.d);
-    const int seg = g_ld(a.seg_start + L), count = g_ld(a.seg_count + L);
-    // lists 2 and 3 (the far lists) hold two entries per voxel: segment 2 * seg
-    int *l2 = a.lists[2] + 2LL * seg, *l3 = a.lists[3] + 2LL * seg, *l4 = a.lists[4] + seg, *walk = a.lists[5] + seg;
-    const Front na{a.lists[0] + seg, sh.front[0]}, nb{a.lists[1] + seg, sh.front[1]};
-    unsigned long long *s0 = a.snaps[0] + seg, *s1 = a.snaps[1] + seg;
+    const Lane<Wide> ln = lane_of<Wide>(a.d, kBlock);
+    const int seg = __builtin_amdgcn_readfirstlane(g_ld(a.seg_start + L));  // uniform: scalar registers
+    const int count = __builtin_amdgcn_readfirstlane(g_ld(a.seg_count + L));
+    const Lists l = lists_of(a, sh, seg);
+    int *walk = l.walk;
     if (threadIdx.x == 0) {
       sh.cursor = seg;
       sh.seg_end = (long long)seg + count;
@@ -1101,7 +993,7 @@ __global__ void __launch_bounds__(kBlock) trace_labels(const TraceArgs *__restri
     __syncthreads();
     bool traceable = true;
     if (a.parent) {
-      const int field = parent_field(a, sh, int(g_ld(a.root + L)), a.order + seg, count, na, nb, l2, l3, l4);
+      const int field = parent_field(a, sh, ln, int(g_ld(a.root + L)), a.order + seg, count, l);
       lap(sh, 2);
       traceable = field == kNoRail;
       if (field == kRailFound && threadIdx.x == 0) g_st(a.ejected + g_add(a.counters + 2, 1) % a.ejected_cap, L);
@@ -1116,18 +1008,16 @@ __global__ void __launch_bounds__(kBlock) trace_labels(const TraceArgs *__restri
       int status = kRailFound;
       if (a.parent) {
         parent_walk(a, sh, t, count, walk);
-        if (threadIdx.x == 0) sh.n_touched = 0;
+        if (threadIdx.x == 0) sh.n[kTouched] = 0;
       } else {
-        status = railroad(a, sh, t, count, na, nb, l2, l3, l4);
+        status = railroad(a, sh, ln, t, count, l);
         lap(sh, 2);
         if (status == kRailFound) backtrace(a, sh, t, count, walk);
       }
       __syncthreads();
       lap(sh, 3);
-      const int nt = sh.n_touched;
-      for (int j = threadIdx.x; j < nt; j += blockDim.x) {  // restore the railroad state
-        sp_u64(&a.rec[g_ld(l4 + j)].word, kMaxKey);
-      }
+      const int nt = sh.n[kTouched];
+      road_restore(a, sh, l.touched);
       if (status == kStalled || status == kOverflowed) {  // given up: the host raises
         if (threadIdx.x == 0) report_failure(a, status);
         __syncthreads();
@@ -1170,10 +1060,10 @@ __global__ void __launch_bounds__(kBlock) trace_labels(const TraceArgs *__restri
         if (a.parent) {
           if (!soma) g_st(a.parent + v, -2);  // STOP: later walks end on this vertex (not for somata)
         }
-        else sp_f(&a.rec[v].pdrf, 0.0f);       // the path becomes rail
+        else sp_u64(a.road + v, kUnreached);    // the path becomes rail (cost 0)
       }
       __syncthreads();
-      const bool converged = invalidate(a, a.ball, sh, walk, len, count, na, nb, l2, l3, l4, s0, s1);
+      const bool converged = invalidate(a, a.ball, sh, ln, walk, len, count, l);
       lap(sh, 4);
       if (!converged) break;  // reported by invalidate; the host raises
       if (threadIdx.x == 0) { sh.pcount += 1; sh.prof[7] += 1; }
@@ -1200,6 +1090,8 @@ void trace_all(Context &ctx, const std::vector<TraceArgs> &args, const std::vect
   Buffer<int> next(ctx, 1);  // queue cursor
   next.clear(ctx);
   const int nq = int(q.size());
+  bool wide = false;  // one launch serves every sample of the group
+  for (const TraceArgs &t : args) wide |= !narrow_words(t.d);
   // every workgroup takes labels from the queue until it is spent, so any grid drains it
   const int grid = std::min(nq, BROOK_TRACE_GRID > 0 ? BROOK_TRACE_GRID : ctx.compute_units() * 2);
   if (!somata.empty()) {
@@ -1208,12 +1100,12 @@ void trace_all(Context &ctx, const std::vector<TraceArgs> &args, const std::vect
     Buffer<int2> soma_queue(ctx, sq.size());
     soma_queue.upload(ctx, sq.data(), sq.size());
     KernelTimer kt(ctx, "soma_balls");
-    soma_balls<<<unsigned(sq.size()), kBlock, 0, ctx.stream()>>>(args_dev.data(), soma_queue.data(), int(sq.size()));
+    (wide ? soma_balls<true> : soma_balls<false>)<<<unsigned(sq.size()), kBlock, 0, ctx.stream()>>>(args_dev.data(), soma_queue.data(), int(sq.size()));
     BROOK_LAUNCHED();
   }
   {
     KernelTimer kt(ctx, "trace_labels");
-    trace_labels<<<grid, kBlock, 0, ctx.stream()>>>(args_dev.data(), queue.data(), nq,
+    (wide ? trace_labels<true> : trace_labels<false>)<<<grid, kBlock, 0, ctx.stream()>>>(args_dev.data(), queue.data(), nq,
                                                     std::min(grid, ctx.compute_units()), next.data());
     BROOK_LAUNCHED();
   }

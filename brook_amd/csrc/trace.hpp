@@ -15,7 +15,11 @@ struct Ball {
 
 struct TraceArgs {
   Dims d{0, 0, 0};
-  VoxelRec *rec = nullptr;  // voxel records: PDRF (rails become 0 in place), flags, words (~0 between uses)
+  FastDiv by_row, by_plane;     // divisions by d.sx and d.sx * d.sy
+  const unsigned *mask = nullptr;       // neighbour masks
+  // word arrays (common.hpp; road0, claim0: their first pad words)
+  unsigned long long *road = nullptr, *road0 = nullptr;    // the PDRF (rails become 0 in place), unreached between uses
+  unsigned long long *claim = nullptr, *claim0 = nullptr;  // free (alive) or dead between uses
   const float *dbf = nullptr;
   const int *seg_start = nullptr, *seg_count = nullptr;
   const int *order = nullptr;  // per-label target order (voxels) in segment layout
@@ -37,7 +41,8 @@ struct TraceArgs {
   int *counters = nullptr;
   // per label (kTraceProfileSlots u64): wall-clock ticks total / target / railroad / backtrace /
   // invalidation, railroad rounds, invalidation rounds, paths, railroad phases, far entries
-  // scanned, near entries expanded, invalidation entries expanded, waiting entries pulled, bands
+  // scanned, near entries expanded, invalidation entries expanded, waiting entries scanned, bands,
+  // entries pulled
   // (null: not recorded)
   unsigned long long *label_stats = nullptr;
   int *ejected = nullptr;
@@ -52,8 +57,8 @@ struct TraceArgs {
   // Somata, per label (null: none in the sample).
   const struct SomaLabel *soma = nullptr;
   // With a voxel graph, the pull masks (bit k of v: neighbour v + N[k] is of v's id and its word
-  // permits the step to v) for backtraces, band-boundary pulls and parents; the records' masks are
-  // then the push masks. Null: no graph (pulls read the records' masks).
+  // permits the step to v) for backtraces, band-boundary pulls and parents; `mask` is then the push
+  // masks. Null: no graph (pulls read `mask`).
   const unsigned *inmask = nullptr;
 };
 

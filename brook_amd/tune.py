@@ -1,9 +1,9 @@
 """Autotuner for the launch shapes and frontier chunk sizes of the persistent label kernels.
 
 The flood (`prepare_labels`) and trace (`trace_labels`) kernels take six compile-time shapes:
-threads per label workgroup for each, how many of a voxel's 26 neighbours one thread keeps in
-flight together (`for_parts` chunks: 9, 13 or 26; more in flight hides more latency and costs
-registers), and how many label workgroups are resident at once (fewer: less contention for the
+threads per label workgroup for each, how many neighbour words one lane keeps in flight in a long
+front (9, 13 or 26: that many pairs of front entries per wave and batch; more in flight hides more
+latency and costs registers), and how many label workgroups are resident at once (fewer: less contention for the
 labels on the critical path, later starts for the rest). They set speed only: every value gives bit-identical skeletons. This tuner searches
 them by coordinate descent from the current values in `csrc/tuned.hpp`: for each parameter in
 turn it builds the library with each candidate value (the others at their best so far), times it

@@ -1,0 +1,51 @@
+// CPU check of the frontier kernels' word and index arithmetic (common.hpp, front.hpp): divisions by
+// a high product for divisors and dividends at the edges of their ranges, the lane slots in address
+// order, the order of road words of one voxel, the padded words' byte offsets. Prints "ok" or the
+// first violation.
+#include <cstdio>
+#include <initializer_list>
+
+#include "../../brook_amd/csrc/front.hpp"
+
+using namespace brook;
+
+int main() {
+  for (unsigned d : {1u, 2u, 3u, 5u, 7u, 48u, 64u, 127u, 128u, 129u, 512u, 641u, 1000u, 4095u, 65535u, 65536u, 65537u, 262144u,
+                     1000003u, (1u << 30) - 1u, 1u << 30, (1u << 30) + 1u, (1u << 31) - 1u}) {
+    const FastDiv f = fast_div(d);
+    auto check = [&](unsigned n) { return fast_quotient(n, f) == n / d; };
+    const unsigned top = (1u << 31) - 1u;
+    for (unsigned i = 0; i < 3000; ++i)
+      for (unsigned n : {i, top - i, unsigned((unsigned long long)i * 715827ull % (1ull << 31))})
+        if (!check(n)) { std::printf("%u / %u\n", n, d); return 1; }
+    for (unsigned long long q = 1; q * d <= top; q = q * 3 / 2 + 1)  // around multiples of d
+      for (int e = -1; e <= 1; ++e)
+        if (q * d + e <= top && !check(unsigned(q * d + e))) { std::printf("%llu * %u + %d\n", q, d, e); return 1; }
+  }
+  const SlotTable t = slot_table();
+  bool seen[26] = {};
+  for (int s = 0; s < 26; ++s) {
+    seen[t.k[s]] = true;
+    auto key = [&](int k) { return (kDZ[k] * 1000 + kDY[k]) * 1000 + kDX[k]; };
+    if (s && key(t.k[s - 1]) >= key(t.k[s])) { std::printf("slot %d out of order\n", s); return 1; }
+  }
+  for (bool b : seen)
+    if (!b) { std::printf("a neighbour has no slot\n"); return 1; }
+  // one voxel's words: by distance, then queued, rail, far-listed; unreached above every finite one
+  const unsigned cost = 0x3f800000u, d0 = 0x3f000000u, d1 = d0 + 1u, most = kInfBits - 1u;
+  const unsigned long long order[] = {road_word(d0, 0, cost), road_word(d0, kNotQueued, cost),
+                                      road_word(d0, kFarListed | kNotQueued, cost), road_word(d1, 0, cost),
+                                      road_word(most, kFarListed | kNotQueued, cost), kUnreached | cost};
+  for (int i = 1; i < 6; ++i)
+    if (order[i - 1] >= order[i]) { std::printf("word %d out of order\n", i); return 1; }
+  for (unsigned long long w : order)
+    if (road_cost(w) != cost) { std::printf("cost lost\n"); return 1; }
+  if (road_dist(kUnreached) != kInfBits || road_dist(order[1]) != d0) { std::printf("distance lost\n"); return 1; }
+  // the last padded byte of a narrow volume lies within 32 bits, and the limit is where it has to be
+  for (Dims d : {Dims{1, 1, 1}, Dims{512, 512, 512}, Dims{1024, 1024, 509}, Dims{1024, 1024, 510}, Dims{9000, 9000, 5}}) {
+    const long long words = (long long)d.sx * d.sy * d.sz + 2 * word_pad(d);
+    if (narrow_words(d) != (words * 8 <= (1LL << 32))) { std::printf("narrow %d %d %d\n", d.sx, d.sy, d.sz); return 1; }
+  }
+  std::printf("ok\n");
+  return 0;
+}
