@@ -5,10 +5,15 @@
 // Whole-result passes are wide: union-find components over every edge, per-edge lengths, keep
 // masks and prefix sums, radix sorts of edge keys and of join candidates, a 27-cell grid search
 // for join candidates. The rules that are sequential by nature (one component's cycle loop, one
-// tree's tick loop, one label's greedy fusion) run one lane per component or label over scratch
-// slices sized from the component: rows, neighbour lists (doubly linked in insertion order, with
-// a free list), search stack and path for the loops; a CSR neighbour table, chain records, end
-// slots and a binary heap keyed (length, lower end, higher end) for the ticks.
+// tree's tick loop, one label's greedy fusion) are chains of dependent accesses: rows, neighbour lists
+// (doubly linked in insertion order, with a free list), search stack and path for the loops; a CSR
+// neighbour table, chain records, end slots and a binary heap keyed (length, lower end, higher end) for
+// the ticks. A component (a tree) is one wave's: all lanes take the same steps on the same
+// addresses, so no step diverges, scans over its vertices, rows or cycle use all of them, and its
+// state, in 16-bit indices, lies in LDS up to kLdsPiece bytes (about 2700 vertices) and in device
+// memory beyond. One lane per component of a 64-lane wave, state in device memory, took 11.5 ms for
+// the loops and 5.1 ms for the ticks of 150 skeletons of 1100 vertices each; a wave each with its
+// state in LDS takes 1.7 and 0.7 ms.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
@@ -37,11 +42,52 @@ template <class Op> void with_scratch(Context &ctx, Buffer<unsigned char> &scrat
   BROOK_HIP(op(scratch.data(), bytes));
 }
 
+// Bits of the keys 0 .. n.
+int bits_for(long long n) {
+  int bits = 1;
+  while ((1LL << bits) <= n) ++bits;
+  return bits;
+}
+
 template <class T> T read_one(Context &ctx, const T *p) {
   T v{};
   BROOK_HIP(hipMemcpyAsync(&v, p, sizeof(T), hipMemcpyDeviceToHost, ctx.stream()));
   ctx.synchronize();
   return v;
+}
+
+// ---------------------------------------------------------------------------------------------
+// one wave per component: LDS address space, wave-wide steps
+
+template <class T> using InLds = __attribute__((address_space(3))) T;
+template <class T> using InGlobal = __attribute__((address_space(1))) T;
+constexpr size_t kLdsPiece = 150 * 1024;
+
+// Lanes see what other lanes of the wave wrote (blocks of one wave).
+__device__ __forceinline__ void wave_sync() { __syncthreads(); }
+
+// The greater (Sign 1) or smaller (Sign -1) value over the lanes that have one (index >= 0), the
+// lower index on ties; every lane gets the index, -1 if none has.
+template <int Sign> __device__ __forceinline__ int wave_extreme(float d, int index) {
+  for (int off = 32; off > 0; off >>= 1) {
+    const float od = __shfl_xor(d, off, 64);
+    const int oi = __shfl_xor(index, off, 64);
+    const bool better = oi >= 0 && (index < 0 || (Sign > 0 ? od > d : od < d) || (od == d && oi < index));
+    if (better) { d = od; index = oi; }
+  }
+  return index;
+}
+__device__ __forceinline__ int wave_total(int v) {
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  return v;
+}
+__device__ __forceinline__ int wave_before(int v) {  // exclusive sum over the lanes
+  int x = v;
+  for (int off = 1; off < 64; off <<= 1) {
+    const int y = __shfl_up(x, off, 64);
+    if (int(threadIdx.x) >= off) x += y;
+  }
+  return x - v;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -90,6 +136,7 @@ __global__ void graph_vertices(const long long *voff, int k, int n, int *vlabel,
   degree[i] = 0;
 }
 
+// root: null when the components are not asked for.
 __global__ void graph_edges(const unsigned *local, int m, const long long *voff, const long long *eoff, int k, int *elabel,
                             int2 *e, int *root, int *degree, int *bad) {
   const int i = blockIdx.x * kThreads + threadIdx.x;
@@ -107,7 +154,7 @@ __global__ void graph_edges(const unsigned *local, int m, const long long *voff,
   e[i] = make_int2(ga, gb);
   atomicAdd(degree + ga, 1);
   atomicAdd(degree + gb, 1);
-  uf_join(root, ga, gb);
+  if (root) uf_join(root, ga, gb);
 }
 
 __global__ void graph_flatten(int *root, int n) {
@@ -125,7 +172,8 @@ struct Graph {
   Buffer<int2> e;
 };
 
-Graph build_graph(Context &ctx, const DevicePacked &p) {
+// components: false leaves g.root as it is (each vertex its own).
+Graph build_graph(Context &ctx, const DevicePacked &p, bool components = true) {
   const size_t k = p.labels.size();
   const bool ok = p.voff.size() == k + 1 && p.eoff.size() == k + 1 && p.voff.front() == 0 && p.eoff.front() == 0 &&
                   std::is_sorted(p.voff.begin(), p.voff.end()) && std::is_sorted(p.eoff.begin(), p.eoff.end()) &&
@@ -153,8 +201,8 @@ Graph build_graph(Context &ctx, const DevicePacked &p) {
   if (g.n) graph_vertices<<<grid(g.n), kThreads, 0, s>>>(g.voff.data(), g.k, g.n, g.vlabel.data(), g.root.data(), g.degree.data());
   if (g.m)
     graph_edges<<<grid(g.m), kThreads, 0, s>>>(p.edges.data(), g.m, g.voff.data(), g.eoff.data(), g.k, g.elabel.data(),
-                                               g.e.data(), g.root.data(), g.degree.data(), bad.data());
-  if (g.n) graph_flatten<<<grid(g.n), kThreads, 0, s>>>(g.root.data(), g.n);
+                                               g.e.data(), components ? g.root.data() : nullptr, g.degree.data(), bad.data());
+  if (g.n && components) graph_flatten<<<grid(g.n), kThreads, 0, s>>>(g.root.data(), g.n);
   BROOK_LAUNCHED();
   if (read_one(ctx, bad.data())) throw std::invalid_argument("packed edge is out of bounds");
   return g;
@@ -329,7 +377,7 @@ __global__ void nonzero(const int *degree, int n, int *keep, int *zero) {
 }
 
 DevicePacked prune_unused(Context &ctx, DevicePacked p) {
-  Graph g = build_graph(ctx, p);
+  Graph g = build_graph(ctx, p, false);
   if (!g.n) return p;
   Buffer<int> keep(ctx, g.n), zero(ctx, 1);
   zero.clear(ctx);
@@ -512,14 +560,26 @@ DevicePacked remove_dust(Context &ctx, DevicePacked p, double threshold) {
 // Components taking part in a sequential rule: their vertices (ascending index) and edges (edge
 // order) as contiguous segments in slot order, local ids = position in the segment.
 
-__global__ void component_sizes(const int *root, const int *degree, int n, const int2 *e, int m, int *nv, int *ne,
-                                int *branch) {
+// Adds 1 to count[slot] for every lane with `on` (all lanes of the wave here): lanes of consecutive
+// equal slots add together, so a long run of one component is one atomic per wave.
+__device__ __forceinline__ void count_runs(int *count, int slot, bool on) {
+  const int lane = int(threadIdx.x) & 63;
+  const int key = on ? slot : -1, before = __shfl_up(key, 1, 64);
+  const unsigned long long heads = __builtin_amdgcn_ballot_w64(lane == 0 || key != before);
+  if (!on || !((heads >> lane) & 1ULL)) return;
+  const unsigned long long after = lane == 63 ? 0ULL : heads >> (lane + 1);
+  atomicAdd(count + slot, after ? __ffsll((long long)after) : 64 - lane);
+}
+
+// critical: vertices of degree 1 or at least 3; branch: a vertex of degree at least 3.
+__global__ void component_sizes(const int *root, const int *degree, int n, const int2 *e, int m, int *nv, int *ne, int *branch,
+                                int *critical) {
   const int i = blockIdx.x * kThreads + threadIdx.x;
-  if (i < n) {
-    atomicAdd(nv + root[i], 1);
-    if (degree[i] >= 3) branch[root[i]] = 1;
-  }
-  if (i < m) atomicAdd(ne + root[e[i].x], 1);
+  const int r = i < n ? root[i] : 0, d = i < n ? degree[i] : 0;
+  count_runs(nv, r, i < n);
+  count_runs(critical, r, d == 1 || d >= 3);
+  if (d >= 3) branch[r] = 1;
+  count_runs(ne, i < m ? root[e[i].x] : 0, i < m);
 }
 
 __global__ void pick_components(const int *nv, const int *ne, const int *branch, int n, bool trees, int *flag) {
@@ -528,14 +588,13 @@ __global__ void pick_components(const int *nv, const int *ne, const int *branch,
   flag[r] = trees ? (branch[r] && ne[r] == nv[r] - 1) : (ne[r] > 0 && ne[r] - nv[r] + 1 > 0);
 }
 
-__global__ void component_slots(const int *flag, const int *pos, const int *nv, const int *ne, int n, int *slot,
-                                int *slot_nv, int *slot_ne) {
+__global__ void component_slots(const int *flag, const int *pos, const int *nv, const int *ne, const int *critical, int n,
+                                int *slot, int3 *sizes) {
   const int r = blockIdx.x * kThreads + threadIdx.x;
   if (r >= n) return;
   slot[r] = flag[r] ? pos[r] : -1;
   if (flag[r]) {
-    slot_nv[pos[r]] = nv[r];
-    slot_ne[pos[r]] = ne[r];
+    sizes[pos[r]] = make_int3(nv[r], ne[r], critical[r]);
   }
 }
 
@@ -575,36 +634,67 @@ struct Pieces {
   Buffer<int> vlist, elist;       // global ids in slot order
   Buffer<long long> vs, es;       // per slot: segment starts (count + 1)
   std::vector<long long> vs_host, es_host;
+  std::vector<int> critical;      // per slot: vertices of degree 1 or at least 3
   Buffer<int> local;              // per vertex of a piece: local id
   Buffer<int2> rows;              // per edge of a piece: local (x, y) as stored
+  Buffer<int> comp_of_edge;       // per edge of a piece: its component
 };
+
+// The components (of `count`) whose state fits LDS and the others, as lists on the device;
+// lds: the largest fitting state.
+struct Split {
+  Buffer<int> small, large;
+  int nsmall = 0, nlarge = 0;
+  size_t lds = 0;
+};
+template <class Bytes> Split split_pieces(Context &ctx, const Pieces &pc, Bytes &&bytes) {
+  Split sp;
+  std::vector<int> small, large;
+  for (int c = 0; c < pc.count; ++c) {
+    const long long nv = pc.vs_host[size_t(c) + 1] - pc.vs_host[size_t(c)], E = pc.es_host[size_t(c) + 1] - pc.es_host[size_t(c)];
+    const size_t need = bytes(size_t(c), size_t(nv), size_t(E));
+    // 16-bit indices: entries are numbered up to 2 E + 4
+    if (need <= kLdsPiece && 2 * E + 4 < 32768 && nv < 32768) {
+      small.push_back(c);
+      sp.lds = std::max(sp.lds, need);
+    } else {
+      large.push_back(c);
+    }
+  }
+  sp.nsmall = int(small.size());
+  sp.nlarge = int(large.size());
+  sp.small = Buffer<int>(ctx, std::max<size_t>(small.size(), 1));
+  sp.large = Buffer<int>(ctx, std::max<size_t>(large.size(), 1));
+  if (sp.nsmall) sp.small.upload(ctx, small.data(), small.size());
+  if (sp.nlarge) sp.large.upload(ctx, large.data(), large.size());
+  return sp;
+}
 
 Pieces pieces_of(Context &ctx, const Graph &g, bool trees) {
   Pieces pc;
   auto s = ctx.stream();
-  Buffer<int> nv(ctx, g.n), ne(ctx, g.n), branch(ctx, g.n), flag(ctx, g.n + 1), pos(ctx, g.n + 1);
-  nv.clear(ctx);
-  ne.clear(ctx);
-  branch.clear(ctx);
-  component_sizes<<<grid(std::max(g.n, g.m)), kThreads, 0, s>>>(g.root.data(), g.degree.data(), g.n, g.e.data(), g.m, nv.data(),
-                                                               ne.data(), branch.data());
-  pick_components<<<grid(g.n), kThreads, 0, s>>>(nv.data(), ne.data(), branch.data(), g.n, trees, flag.data());
+  Buffer<int> sums(ctx, size_t(4) * g.n), flag(ctx, g.n + 1), pos(ctx, g.n + 1);
+  sums.clear(ctx);
+  int *nv = sums.data(), *ne = nv + g.n, *branch = ne + g.n, *critical = branch + g.n;
+  component_sizes<<<grid(std::max(g.n, g.m)), kThreads, 0, s>>>(g.root.data(), g.degree.data(), g.n, g.e.data(), g.m, nv, ne,
+                                                               branch, critical);
+  pick_components<<<grid(g.n), kThreads, 0, s>>>(nv, ne, branch, g.n, trees, flag.data());
   BROOK_LAUNCHED();
   BROOK_HIP(hipMemsetAsync(flag.data() + g.n, 0, 4, s));
   exclusive_sum(ctx, flag.data(), pos.data(), g.n + 1);
   pc.count = read_one(ctx, pos.data() + g.n);
   if (!pc.count) return pc;
   pc.slot = Buffer<int>(ctx, g.n);
-  Buffer<int> snv(ctx, pc.count), sne(ctx, pc.count);
-  component_slots<<<grid(g.n), kThreads, 0, s>>>(flag.data(), pos.data(), nv.data(), ne.data(), g.n, pc.slot.data(), snv.data(),
-                                                 sne.data());
+  Buffer<int3> sizes(ctx, pc.count);
+  component_slots<<<grid(g.n), kThreads, 0, s>>>(flag.data(), pos.data(), nv, ne, critical, g.n, pc.slot.data(), sizes.data());
   BROOK_LAUNCHED();
-  const std::vector<int> hv = snv.download(ctx), he = sne.download(ctx);
+  const std::vector<int3> h = sizes.download(ctx);
   pc.vs_host.assign(1, 0);
   pc.es_host.assign(1, 0);
-  for (int c = 0; c < pc.count; ++c) {
-    pc.vs_host.push_back(pc.vs_host.back() + hv[c]);
-    pc.es_host.push_back(pc.es_host.back() + he[c]);
+  for (const int3 &c : h) {
+    pc.vs_host.push_back(pc.vs_host.back() + c.x);
+    pc.es_host.push_back(pc.es_host.back() + c.y);
+    pc.critical.push_back(c.z);
   }
   pc.nv = int(pc.vs_host.back());
   pc.ne = int(pc.es_host.back());
@@ -625,13 +715,14 @@ Pieces pieces_of(Context &ctx, const Graph &g, bool trees) {
     });
   }
   {
-    Buffer<int> key(ctx, g.m), key_sorted(ctx, g.m), index(ctx, g.m);
+    Buffer<int> key(ctx, g.m), index(ctx, g.m);
     pc.elist = Buffer<int>(ctx, g.m);
+    pc.comp_of_edge = Buffer<int>(ctx, g.m);  // the sorted keys
     slot_keys_edges<<<grid(g.m), kThreads, 0, s>>>(g.e.data(), g.root.data(), pc.slot.data(), g.m, pc.count, key.data(),
                                                    index.data());
     BROOK_LAUNCHED();
     with_scratch(ctx, scratch, [&](void *t, size_t &b) {
-      return hipcub::DeviceRadixSort::SortPairs(t, b, key.data(), key_sorted.data(), index.data(), pc.elist.data(), g.m, 0, bits, s);
+      return hipcub::DeviceRadixSort::SortPairs(t, b, key.data(), pc.comp_of_edge.data(), index.data(), pc.elist.data(), g.m, 0, bits, s);
     });
   }
   pc.local = Buffer<int>(ctx, g.n);
@@ -643,20 +734,16 @@ Pieces pieces_of(Context &ctx, const Graph &g, bool trees) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// remove_loops: one lane per cyclic component (post_kernels.cuh:22-199)
+// remove_loops: one wave per cyclic component (post_kernels.cuh:22-199)
 
-struct LoopArena {
-  int2 *rows;                            // 2 * E + 2 per component: (x, y), x = -1 once dead
-  int *nbr, *nxt, *prv, *rid, *mul;      // 2 * E + 4 entries per component
-  int *head, *tail, *cnt, *seen, *order;  // nv + 1 per component
-  int *branch, *path;                    // nv + 1 per component
-  unsigned char *drop;                   // nv + 1 per component
-  int3 *stack;                           // 2 * E + 2 per component: (node, parent, depth)
-};
-
-struct LoopLocal {
-  int2 *rows;
-  int *nbr, *nxt, *prv, *rid, *mul, *head, *tail, *cnt;
+// A component's state: I indexes (pointer to short in LDS, int in device memory), B bytes.
+template <class I, class B> struct LoopState {
+  I rx, ry;                       // 2 E + 2 rows: (x, y), x = -1 once dead
+  I nbr, nxt, prv, rid, mul;      // 2 E + 4 list entries
+  I head, tail, cnt, seen, order;  // nv + 1
+  I branch, path;                 // nv + 1
+  I node, parent, depth;          // 2 E + 2: the search stack
+  B drop;                         // nv + 1
   int freelist, bump, entry_cap;
   int nrows;
   long long nlive;
@@ -693,14 +780,16 @@ struct LoopLocal {
   }
   __device__ void add_row(int x, int y) {
     const int r = nrows++;
-    rows[r] = make_int2(x, y);
+    rx[r] = x;
+    ry[r] = y;
     nlive++;
-    cnt[x]++;
-    cnt[y]++;
+    cnt[x] += 1;
+    cnt[y] += 1;
     const int f = find(x, y);
     if (f >= 0) {  // a repeated pair: the first match of each list counts it
-      mul[f]++;
-      mul[find(y, x)]++;
+      mul[f] += 1;
+      const int back = find(y, x);
+      mul[back] += 1;
     } else {
       link(x, y, r);
       link(y, x, r);
@@ -708,96 +797,197 @@ struct LoopLocal {
   }
 };
 
-__device__ __forceinline__ float sq_dist(const float *P, int v, float x, float y, float z) {
-  const float dx = P[3 * v] - x, dy = P[3 * v + 1] - y, dz = P[3 * v + 2] - z;
+// The arrays of a component laid out one after another: index arrays of T, then bytes.
+template <class T> size_t loop_bytes(size_t nv, size_t E) {
+  return sizeof(T) * (2 * (2 * E + 2) + 5 * (2 * E + 4) + 7 * (nv + 1) + 3 * (2 * E + 2)) + (nv + 1);
+}
+template <class I, class B> __device__ LoopState<I, B> loop_state(I at, int nv, int E) {
+  LoopState<I, B> s;
+  auto take = [&](int n) { I p = at; at += n; return p; };
+  s.node = take(2 * E + 2);  // first: the list build counts in its place, in 32 bits
+  s.parent = take(2 * E + 2);
+  s.depth = take(2 * E + 2);
+  s.rx = take(2 * E + 2);
+  s.ry = take(2 * E + 2);
+  s.nbr = take(2 * E + 4);
+  s.nxt = take(2 * E + 4);
+  s.prv = take(2 * E + 4);
+  s.rid = take(2 * E + 4);
+  s.mul = take(2 * E + 4);
+  s.head = take(nv + 1);
+  s.tail = take(nv + 1);
+  s.cnt = take(nv + 1);
+  s.seen = take(nv + 1);
+  s.order = take(nv + 1);
+  s.branch = take(nv + 1);
+  s.path = take(nv + 1);
+  s.drop = (B)at;
+  s.freelist = -1;
+  s.bump = 2 * E;
+  s.entry_cap = 2 * E + 4;
+  s.nrows = E;
+  s.nlive = E;
+  s.overflow = false;
+  return s;
+}
+
+// The neighbour lists of the input rows, as add_row row by row gives them: counted, given out and put
+// in row order per vertex by lanes of their own. W: 32-bit counters (the stack's place: a cyclic
+// component has at least as many rows as vertices, so 6 E + 6 16-bit slots hold nv of them).
+template <class W, class I, class B>
+__device__ void loop_lists(LoopState<I, B> &s, W counter, int nv, int E, const int2 *rows_in) {
+  const int lane = threadIdx.x;
+  for (int v = lane; v < nv; v += 64) counter[v] = 0;
+  wave_sync();
+  for (int r = lane; r < E; r += 64) {
+    const int2 x = rows_in[r];
+    s.rx[r] = x.x;
+    s.ry[r] = x.y;
+    __hip_atomic_fetch_add(counter + x.x, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __hip_atomic_fetch_add(counter + x.y, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  wave_sync();
+  int base = 0;
+  for (int v0 = 0; v0 < nv; v0 += 64) {  // segment starts: head for now
+    const int v = v0 + lane, c = v < nv ? counter[v] : 0, before = wave_before(c);
+    if (v < nv) {
+      s.cnt[v] = c;
+      s.head[v] = base + before;
+      s.seen[v] = 0;
+      counter[v] = base + before;
+    }
+    base += wave_total(c);
+  }
+  wave_sync();
+  for (int r = lane; r < E; r += 64) {
+    const int x = s.rx[r], y = s.ry[r];
+    const int a = __hip_atomic_fetch_add(counter + x, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    s.rid[a] = r;
+    const int b = __hip_atomic_fetch_add(counter + y, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    s.rid[b] = r;
+  }
+  wave_sync();
+  bool dropped = false;
+  for (int v = lane; v < nv; v += 64) {
+    const int e0 = s.head[v], e1 = e0 + s.cnt[v];
+    for (int i = e0 + 1; i < e1; ++i) {  // by row
+      const int r = s.rid[i];
+      int j = i - 1;
+      while (j >= e0 && s.rid[j] > r) { s.rid[j + 1] = s.rid[j]; --j; }
+      s.rid[j + 1] = r;
+    }
+    int head = -1, tail = -1;
+    for (int i = e0; i < e1; ++i) {
+      const int r = s.rid[i], x = s.rx[r], y = s.ry[r], other = x == v ? y : x;
+      int first = -1;  // an earlier row's entry of the same pair
+      for (int f = head; f >= 0; f = s.nxt[f])
+        if (s.nbr[f] == other && s.rid[f] != r) { first = f; break; }
+      if (first >= 0) {
+        s.mul[first] += 1;
+        s.rid[i] = -2;  // a free entry
+        dropped = true;
+        continue;
+      }
+      s.nbr[i] = other;
+      s.mul[i] = 1;
+      s.nxt[i] = -1;
+      s.prv[i] = tail;
+      if (tail >= 0) s.nxt[tail] = i;
+      else head = i;
+      tail = i;
+    }
+    s.head[v] = head;
+    s.tail[v] = tail;
+  }
+  wave_sync();
+  if (__builtin_amdgcn_ballot_w64(dropped))
+    for (int i = 0; i < 2 * E; ++i)
+      if (s.rid[i] == -2) { s.nxt[i] = s.freelist; s.freelist = i; }
+}
+
+__device__ __forceinline__ float sq_dist(const float *P, float x, float y, float z) {
+  const float dx = P[0] - x, dy = P[1] - y, dz = P[2] - z;
   return (dx * dx + dy * dy) + dz * dz;
 }
 
-__global__ void loops_kernel(int count, const long long *vs, const long long *es, const int2 *rows_in, const int *vlist,
-                             const float *vertices, const float *radii, LoopArena ar, int2 *rows_out, int *ne_out, int *failed) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= count) return;
-  const long long v0 = vs[c], e0 = es[c];
-  const int nv = int(vs[c + 1] - v0), E = int(es[c + 1] - e0);
+template <class I, class B>
+__device__ void loops_component(LoopState<I, B> &s, int nv, int E, const int *vl, const float *vertices, const float *radii,
+                                int2 *rows_out, int *ne_out, int *failed) {
+  const int lane = threadIdx.x;
   const int row_cap = 2 * E + 2;
-  const long long rbase = 2 * e0 + 2LL * c, ebase = 2 * e0 + 4LL * c, nbase = v0 + c;
-  LoopLocal s;
-  s.rows = ar.rows + rbase;
-  s.nbr = ar.nbr + ebase;
-  s.nxt = ar.nxt + ebase;
-  s.prv = ar.prv + ebase;
-  s.rid = ar.rid + ebase;
-  s.mul = ar.mul + ebase;
-  s.head = ar.head + nbase;
-  s.tail = ar.tail + nbase;
-  s.cnt = ar.cnt + nbase;
-  int *seen = ar.seen + nbase, *order = ar.order + nbase, *branch = ar.branch + nbase, *path = ar.path + nbase;
-  unsigned char *drop = ar.drop + nbase;
-  int3 *stack = ar.stack + rbase;
-  const int *vl = vlist + v0;
   auto P = [&](int v) { return vertices + 3LL * vl[v]; };
-  s.freelist = -1;
-  s.bump = 0;
-  s.entry_cap = 2 * E + 4;
-  s.nrows = 0;
-  s.nlive = 0;
-  s.overflow = false;
-  for (int v = 0; v < nv; ++v) { s.head[v] = s.tail[v] = -1; s.cnt[v] = 0; seen[v] = 0; }
-  for (int i = 0; i < E; ++i) s.add_row(rows_in[e0 + i].x, rows_in[e0 + i].y);
+  auto fail = [&](int bit) { if (lane == 0) atomicOr(failed, bit); };
   int app0 = s.nrows, app1 = s.nrows;  // rows appended by the previous iteration
+  int first = 0;                       // no row before it lives
   const long long budget = 64LL * (E + nv) + 64;
   for (long long iteration = 0;; ++iteration) {
-    if (iteration > budget) { atomicOr(failed, 1); break; }
-    if (s.overflow) { atomicOr(failed, 2); break; }
+    if (iteration > budget) { fail(1); break; }
+    if (s.overflow) { fail(2); break; }
     if (s.nlive == 0) break;
-    int first = 0;
-    while (s.rows[first].x < 0) first++;
+    while (s.rx[first] < 0) first++;
     // depth-first search from the first live row's first end
     int sp = 0, plen = 0, node = -1, nseen = 0;
     bool found = false;
-    stack[sp++] = make_int3(s.rows[first].x, -1, 0);
+    s.node[sp] = s.rx[first];
+    s.parent[sp] = -1;
+    s.depth[sp++] = 0;
     while (sp) {
-      const int3 f = stack[--sp];
-      node = f.x;
-      if (plen > f.z) plen = f.z;
-      path[plen++] = node;
-      if (seen[node]) { found = true; break; }
-      seen[node] = 1;
-      order[nseen++] = node;
-      for (int e = s.head[node]; e >= 0; e = s.nxt[e])
-        if (s.nbr[e] != f.y) stack[sp++] = make_int3(s.nbr[e], node, f.z + 1);
+      --sp;
+      node = s.node[sp];
+      const int parent = s.parent[sp], depth = s.depth[sp];
+      if (plen > depth) plen = depth;
+      s.path[plen++] = node;
+      if (s.seen[node]) { found = true; break; }
+      s.seen[node] = 1;
+      s.order[nseen++] = node;
+      for (int e = s.head[node]; e >= 0; e = s.nxt[e]) {
+        const int to = s.nbr[e];
+        if (to == parent) continue;
+        s.node[sp] = to;
+        s.parent[sp] = node;
+        s.depth[sp++] = depth + 1;
+      }
     }
-    for (int j = 0; j < nseen; ++j) seen[order[j]] = 0;
+    wave_sync();
+    for (int j = lane; j < nseen; j += 64) s.seen[s.order[j]] = 0;
+    wave_sync();
     if (!found || plen <= 1) break;
     int i0 = 0;
-    while (i0 < plen - 1 && path[i0] != node) i0++;
+    while (i0 < plen - 1 && s.path[i0] != node) i0++;
     if (plen - i0 < 3) break;
-    const int *cy = path + i0;
+    const I cy = s.path + i0;
     const int cl = plen - i0;
     int nb = 0;
     for (int j = 0; j + 1 < cl; ++j)
-      if (s.cnt[cy[j]] >= 3) branch[nb++] = cy[j];
+      if (s.cnt[cy[j]] >= 3) s.branch[nb++] = cy[j];
     for (int i = 1; i < nb; ++i) {  // ascending (few)
-      const int x = branch[i];
+      const int x = s.branch[i];
       int j = i - 1;
-      while (j >= 0 && branch[j] > x) { branch[j + 1] = branch[j]; --j; }
-      branch[j + 1] = x;
+      while (j >= 0 && s.branch[j] > x) { s.branch[j + 1] = s.branch[j]; --j; }
+      s.branch[j + 1] = x;
     }
-    for (int j = 0; j < cl; ++j) drop[j] = 0;
+    wave_sync();
+    for (int j = lane; j < cl; j += 64) s.drop[j] = 0;
+    wave_sync();
     int add_a = -1, add_b = -1, hub = -1;
-    bool star = false;
+    bool star = false, whole = false;  // whole: every edge of the cycle goes
     if (nb == 0) {
-      for (int j = 0; j + 1 < cl; ++j) drop[j] = 1;
+      whole = true;
     } else if (nb == 1) {
-      const int bn = branch[0];
+      // the farthest cycle node, the lower one on ties; a first node at a NaN distance stays
+      const int bn = s.branch[0];
+      const float bx = P(bn)[0], by = P(bn)[1], bz = P(bn)[2];
+      float best = 0.0f;
       int end = -1;
-      float best = -1.0f;
-      for (int j = 0; j + 1 < cl; ++j) {
+      for (int j = lane; j + 1 < cl; j += 64) {
         const int v = cy[j];
-        const float d = sq_dist(P(v), 0, P(bn)[0], P(bn)[1], P(bn)[2]);
-        if (end < 0 || d > best || (d == best && v < end)) { best = d; end = v; }
+        const float d = sq_dist(P(v), bx, by, bz);
+        if (d == d && (end < 0 || d > best || (d == best && v < end))) { best = d; end = v; }
       }
-      for (int j = 0; j + 1 < cl; ++j) drop[j] = 1;
+      end = wave_extreme<1>(best, end);
+      const float d0 = sq_dist(P(cy[0]), bx, by, bz);
+      if (d0 != d0) end = cy[0];
+      whole = true;
       add_a = bn;
       add_b = end;
     } else if (nb == 2) {
@@ -809,47 +999,53 @@ __global__ void loops_kernel(int count, const long long *vs, const long long *es
           else p1 = j;
         }
       const bool inner = double(p1 - p0) < double(L) / 2.0;
-      for (int j = 0; j + 1 < cl; ++j) {
+      for (int j = lane; j + 1 < cl; j += 64) {
         const bool on_inner = j - 1 >= 0 && j - 1 >= p0 && j <= p1;
-        if (!(inner ? on_inner : !on_inner)) drop[j] = 1;
+        if (!(inner ? on_inner : !on_inner)) s.drop[j] = 1;
       }
     } else {
       float cx = 0.0f, cyy = 0.0f, cz = 0.0f;
-      for (int i = 0; i < nb; ++i) { cx += P(branch[i])[0]; cyy += P(branch[i])[1]; cz += P(branch[i])[2]; }
+      for (int i = 0; i < nb; ++i) { const float *q = P(s.branch[i]); cx += q[0]; cyy += q[1]; cz += q[2]; }
       cx /= float(nb);
       cyy /= float(nb);
       cz /= float(nb);
+      // the nearest vertex, the lowest on ties; a first vertex at a NaN distance stays
       float best = 0.0f;
-      for (int v = 0; v < nv; ++v) {
-        const float d = sq_dist(P(v), 0, cx, cyy, cz);
-        if (hub < 0 || d < best) { best = d; hub = v; }
+      for (int v = lane; v < nv; v += 64) {
+        const float d = sq_dist(P(v), cx, cyy, cz);
+        if (d == d && (hub < 0 || d < best)) { best = d; hub = v; }
       }
+      hub = wave_extreme<-1>(best, hub);
+      const float d0 = sq_dist(P(0), cx, cyy, cz);
+      if (d0 != d0) hub = 0;
       float far = 0.0f;
       for (int i = 0; i < nb; ++i) {
-        const float d = sq_dist(P(branch[i]), 0, P(hub)[0], P(hub)[1], P(hub)[2]);
+        const float d = sq_dist(P(s.branch[i]), P(hub)[0], P(hub)[1], P(hub)[2]);
         if (i == 0 || d > far) far = d;
       }
       if (sqrtf(far) > radii[vl[hub]]) {
-        drop[0] = 1;
+        s.drop[0] = 1;
       } else {
-        for (int j = 0; j + 1 < cl; ++j) drop[j] = 1;
-        star = true;
+        whole = star = true;
       }
     }
-    for (int r = app0; r < app1; ++r)
-      if (s.rows[r].x > s.rows[r].y) s.rows[r] = make_int2(s.rows[r].y, s.rows[r].x);
+    wave_sync();
+    for (int r = app0; r < app1; ++r) {
+      const int x = s.rx[r], y = s.ry[r];
+      if (x > y) { s.rx[r] = y; s.ry[r] = x; }
+    }
     for (int j = 0; j + 1 < cl; ++j) {
-      if (!drop[j]) continue;
+      if (!whole && !s.drop[j]) continue;
       const int a = cy[j], b = cy[j + 1];
       const int e = s.find(a, b);
       if (e < 0) continue;
       const int m = s.mul[e];
       if (m == 1) {
-        s.rows[s.rid[e]].x = -1;
+        s.rx[s.rid[e]] = -1;
       } else {
         const int lo = min(a, b), hi = max(a, b);
         for (int r = first; r < s.nrows; ++r)
-          if (s.rows[r].x == lo && s.rows[r].y == hi) s.rows[r].x = -1;
+          if (s.rx[r] == lo && s.ry[r] == hi) s.rx[r] = -1;
       }
       s.nlive -= m;
       s.cnt[a] -= m;
@@ -861,36 +1057,78 @@ __global__ void loops_kernel(int count, const long long *vs, const long long *es
     const int adds = add_b >= 0 ? 1 : (star ? nb : 0);
     if (s.nrows + adds > row_cap) {  // squeeze out the dead rows, keeping the order of the live ones
       int w = 0;
-      for (int r = 0; r < s.nrows; ++r)
-        if (s.rows[r].x >= 0) s.rows[w++] = s.rows[r];
+      for (int r = 0; r < s.nrows; ++r) {
+        const int x = s.rx[r], y = s.ry[r];
+        if (x >= 0) { s.rx[w] = x; s.ry[w++] = y; }
+      }
       s.nrows = w;
+      first = 0;
       for (int v = 0; v < nv; ++v)
         for (int e = s.head[v]; e >= 0; e = s.nxt[e]) s.rid[e] = -1;
       for (int r = 0; r < s.nrows; ++r) {
-        const int f = s.find(s.rows[r].x, s.rows[r].y);
+        const int x = s.rx[r], y = s.ry[r];
+        const int f = s.find(x, y);
         if (f >= 0 && s.rid[f] < 0) {  // (a row whose pair lost its entry has none)
           s.rid[f] = r;
-          s.rid[s.find(s.rows[r].y, s.rows[r].x)] = r;
+          s.rid[s.find(y, x)] = r;
         }
       }
     }
-    if (s.nrows + adds > row_cap) { atomicOr(failed, 2); break; }  // live rows outgrew the input's count
+    if (s.nrows + adds > row_cap) { fail(2); break; }  // live rows outgrew the input's count
     app0 = s.nrows;
     if (add_b >= 0) s.add_row(add_a, add_b);
     if (star)
-      for (int i = 0; i < nb; ++i)
-        if (branch[i] != hub) s.add_row(branch[i], hub);
+      for (int i = 0; i < nb; ++i) {
+        const int x = s.branch[i];
+        if (x != hub) s.add_row(x, hub);
+      }
     app1 = s.nrows;
   }
-  int w = 0;
-  for (int r = 0; r < s.nrows; ++r) w += s.rows[r].x >= 0;
+  wave_sync();
+  int live = 0;
+  for (int r = lane; r < s.nrows; r += 64) live += s.rx[r] >= 0;
+  int w = wave_total(live);
   if (w > E) {  // more live rows than the component had (rows repeated in both orientations)
-    atomicOr(failed, 2);
+    fail(2);
     w = 0;
   }
-  for (int r = 0, k = 0; r < s.nrows && k < w; ++r)
-    if (s.rows[r].x >= 0) rows_out[e0 + k++] = s.rows[r];
-  ne_out[c] = w;
+  int done = 0;
+  for (int r0 = 0; r0 < s.nrows && done < w; r0 += 64) {
+    const int r = r0 + lane;
+    const bool on = r < s.nrows && s.rx[r] >= 0;
+    const unsigned long long m = __builtin_amdgcn_ballot_w64(on);
+    if (on) rows_out[done + __popcll(m & ((1ULL << lane) - 1ULL))] = make_int2(s.rx[r], s.ry[r]);
+    done += __popcll(m);
+  }
+  if (lane == 0) *ne_out = w;
+}
+
+extern __shared__ int post_lds[];
+
+// Block b: component list[b], its state in LDS.
+__global__ void __launch_bounds__(64) loops_small(const int *list, const long long *vs, const long long *es, const int2 *rows_in,
+                                                  const int *vlist, const float *vertices, const float *radii, int2 *rows_out,
+                                                  int *ne_out, int *failed) {
+  const int c = list[blockIdx.x];
+  const long long v0 = vs[c], e0 = es[c];
+  const int nv = int(vs[c + 1] - v0), E = int(es[c + 1] - e0);
+  auto s = loop_state<InLds<short> *, InLds<unsigned char> *>((InLds<short> *)post_lds, nv, E);
+  loop_lists(s, (InLds<int> *)post_lds, nv, E, rows_in + e0);
+  loops_component(s, nv, E, vlist + v0, vertices, radii, rows_out + e0, ne_out + c, failed);
+}
+
+// Block b: component list[b], its state at slot starts[b] (ints) of `arena`.
+__global__ void __launch_bounds__(64) loops_large(const int *list, const long long *starts, int *arena, const long long *vs,
+                                                  const long long *es, const int2 *rows_in, const int *vlist,
+                                                  const float *vertices, const float *radii, int2 *rows_out, int *ne_out,
+                                                  int *failed) {
+  const int c = list[blockIdx.x];
+  const long long v0 = vs[c], e0 = es[c];
+  const int nv = int(vs[c + 1] - v0), E = int(es[c + 1] - e0);
+  InGlobal<int> *at = (InGlobal<int> *)(arena + starts[blockIdx.x]);
+  auto s = loop_state<InGlobal<int> *, InGlobal<unsigned char> *>(at, nv, E);
+  loop_lists(s, at, nv, E, rows_in + e0);
+  loops_component(s, nv, E, vlist + v0, vertices, radii, rows_out + e0, ne_out + c, failed);
 }
 
 __global__ void loop_keys_untouched(const int2 *e, const int *root, const int *slot, int m, unsigned long long *keys) {
@@ -912,12 +1150,6 @@ __global__ void loop_keys_kept(const int2 *rows, const int *ne_out, const long l
   if (a != b) keys[elist[j]] = ((unsigned long long)min(a, b) << 32) | (unsigned long long)max(a, b);
 }
 
-__global__ void edge_component(const long long *es, int count, int *comp_of_edge) {
-  const int c = blockIdx.x * kThreads + threadIdx.x;
-  if (c >= count) return;
-  for (long long j = es[c]; j < es[c + 1]; ++j) comp_of_edge[j] = c;
-}
-
 __global__ void keep_unemptied(const int *root, const int *slot, const int *ne_out, int n, int *keep) {
   const int i = blockIdx.x * kThreads + threadIdx.x;
   if (i >= n) return;
@@ -931,32 +1163,46 @@ DevicePacked remove_loops(Context &ctx, DevicePacked p) {
   Pieces pc = pieces_of(ctx, g, false);
   if (!pc.count) return p;
   auto s = ctx.stream();
-  const long long A = pc.count, N = pc.nv, M = pc.ne;
-  Buffer<int2> rows(ctx, size_t(2 * M + 2 * A)), rows_out(ctx, size_t(std::max<long long>(M, 1)));
-  Buffer<int3> frames(ctx, size_t(2 * M + 2 * A));
-  const size_t entries = size_t(2 * M + 4 * A), nodes = size_t(N + A);
-  Buffer<int> nbr(ctx, entries), nxt(ctx, entries), prv(ctx, entries), rid(ctx, entries), mul(ctx, entries);
-  Buffer<int> head(ctx, nodes), tail(ctx, nodes), cnt(ctx, nodes), seen(ctx, nodes), order(ctx, nodes), branch(ctx, nodes),
-      path(ctx, nodes);
-  Buffer<unsigned char> drop(ctx, nodes);
+  const long long A = pc.count, M = pc.ne;
+  Buffer<int2> rows_out(ctx, size_t(std::max<long long>(M, 1)));
   Buffer<int> ne_out(ctx, A), failed(ctx, 1);
   failed.clear(ctx);
-  LoopArena ar{rows.data(), nbr.data(), nxt.data(), prv.data(), rid.data(), mul.data(), head.data(), tail.data(), cnt.data(),
-               seen.data(), order.data(), branch.data(), path.data(), drop.data(), frames.data()};
-  loops_kernel<<<unsigned((A + 63) / 64), 64, 0, s>>>(pc.count, pc.vs.data(), pc.es.data(), pc.rows.data(), pc.vlist.data(),
-                                                     p.vertices.data(), p.radii.data(), ar, rows_out.data(), ne_out.data(),
-                                                     failed.data());
-  BROOK_LAUNCHED();
+  const Split sp = split_pieces(ctx, pc, [](size_t, size_t nv, size_t E) { return loop_bytes<short>(nv, E); });
+  if (sp.nsmall) {
+    BROOK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(loops_small), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  int(kLdsPiece)));
+    loops_small<<<unsigned(sp.nsmall), 64, sp.lds, s>>>(sp.small.data(), pc.vs.data(), pc.es.data(), pc.rows.data(),
+                                                       pc.vlist.data(), p.vertices.data(), p.radii.data(), rows_out.data(),
+                                                       ne_out.data(), failed.data());
+    BROOK_LAUNCHED();
+  }
+  Buffer<int> arena;
+  Buffer<long long> starts_dev;
+  if (sp.nlarge) {
+    std::vector<int> large = sp.large.download(ctx);
+    std::vector<long long> starts;
+    long long ints = 0;
+    for (int c : large) {
+      starts.push_back(ints);
+      ints += (long long)((loop_bytes<int>(size_t(pc.vs_host[size_t(c) + 1] - pc.vs_host[size_t(c)]),
+                                           size_t(pc.es_host[size_t(c) + 1] - pc.es_host[size_t(c)])) + 3) / 4);
+    }
+    arena = Buffer<int>(ctx, size_t(ints));
+    starts_dev = Buffer<long long>(ctx, starts.size());
+    starts_dev.upload(ctx, starts.data(), starts.size());
+    loops_large<<<unsigned(sp.nlarge), 64, 0, s>>>(sp.large.data(), starts_dev.data(), arena.data(), pc.vs.data(), pc.es.data(),
+                                                  pc.rows.data(), pc.vlist.data(), p.vertices.data(), p.radii.data(),
+                                                  rows_out.data(), ne_out.data(), failed.data());
+    BROOK_LAUNCHED();
+  }
   const int failure = read_one(ctx, failed.data());
   if (failure & 1) throw std::runtime_error("remove_loops did not converge");
   if (failure & 2) throw std::runtime_error("remove_loops row capacity exceeded (rows repeated in both orientations)");
   Buffer<unsigned long long> keys(ctx, size_t(std::max(g.m, 1)));
-  Buffer<int> comp_of_edge(ctx, size_t(std::max<long long>(M, 1)));
   loop_keys_untouched<<<grid(g.m), kThreads, 0, s>>>(g.e.data(), g.root.data(), pc.slot.data(), g.m, keys.data());
-  edge_component<<<grid(A), kThreads, 0, s>>>(pc.es.data(), pc.count, comp_of_edge.data());
   if (M)
     loop_keys_kept<<<grid(M), kThreads, 0, s>>>(rows_out.data(), ne_out.data(), pc.es.data(), pc.vs.data(), pc.vlist.data(),
-                                                pc.elist.data(), comp_of_edge.data(), int(M), keys.data());
+                                                pc.elist.data(), pc.comp_of_edge.data(), int(M), keys.data());
   BROOK_LAUNCHED();
   const std::vector<int> kept = ne_out.download(ctx);
   DevicePacked out = edges_from_keys(ctx, std::move(p), g, keys, g.m);
@@ -964,12 +1210,12 @@ DevicePacked remove_loops(Context &ctx, DevicePacked p) {
   Buffer<int> keep(ctx, g.n);
   keep_unemptied<<<grid(g.n), kThreads, 0, s>>>(g.root.data(), pc.slot.data(), ne_out.data(), g.n, keep.data());
   BROOK_LAUNCHED();
-  Graph next = build_graph(ctx, out);
+  Graph next = build_graph(ctx, out, false);
   return select_vertices(ctx, out, keep, next);
 }
 
 // ---------------------------------------------------------------------------------------------
-// remove_ticks: one lane per tree with a branch point (post_kernels.cuh:309-405)
+// remove_ticks: one wave per tree with a branch point (post_kernels.cuh:309-405)
 
 // CSR neighbours of the pieces' vertices: a node's rows that start at it, then those that end at
 // it, each in row order (a stable sort of both directions by source).
@@ -986,30 +1232,27 @@ __global__ void csr_entries(const int2 *rows, const long long *vs, const long lo
   value[M + j] = ((unsigned long long)unsigned(x.x) << 32) | r;
 }
 
-__global__ void csr_degree(const unsigned *source_sorted, int total, int *deg) {
-  const int j = blockIdx.x * kThreads + threadIdx.x;
-  if (j < total) atomicAdd(deg + source_sorted[j], 1);
+// off[v]: the first entry whose source is at or past v.
+__global__ void csr_offsets(const unsigned *source_sorted, long long total, long long n, long long *off) {
+  const long long v = (long long)blockIdx.x * kThreads + threadIdx.x;
+  if (v > n) return;
+  long long lo = 0, hi = total;
+  while (lo < hi) {
+    const long long mid = (lo + hi) >> 1;
+    if ((long long)source_sorted[mid] < v) lo = mid + 1;
+    else hi = mid;
+  }
+  off[v] = lo;
 }
 
-struct TickArena {
-  int *bc, *slot_head;               // nv per component
-  int4 *stack;                       // (node, parent, root, chain), nv + 1 per component
-  float *stack_dist;
-  int *su, *sv, *ver, *chain_first, *chain_last, *chain_next;  // E + 1 per component (chain ids)
-  double *len;
-  unsigned char *alive, *eligible, *dead;
-  int *slot_next, *slot_owner;       // 2 (E + 1) per component
-  double *heap_len;                  // 2 (E + 1) + 2 per component
-  int *heap_lo, *heap_hi, *heap_id, *heap_ver;
-  int *chain_of;                     // E per component (row -> chain)
-};
-
-struct Heap {
-  double *len;
-  int *lo, *hi, *id, *ver;
+// A binary heap keyed (length, lower end, higher end).
+template <class I, class D> struct Heap {
+  D len;
+  I lo, hi, id, ver;
   int n = 0;
   __device__ bool less(int i, int j) const {
-    return len[i] < len[j] || (len[i] == len[j] && (lo[i] < lo[j] || (lo[i] == lo[j] && hi[i] < hi[j])));
+    const double a = len[i], b = len[j];
+    return a < b || (a == b && (lo[i] < lo[j] || (lo[i] == lo[j] && hi[i] < hi[j])));
   }
   __device__ void swap(int i, int j) {
     const double l = len[i]; len[i] = len[j]; len[j] = l;
@@ -1044,127 +1287,217 @@ struct Heap {
   }
 };
 
-__global__ void ticks_kernel(int count, const long long *vs, const long long *es, const int *vlist, const float *vertices,
-                             const long long *csr_off, const unsigned long long *csr, double threshold, TickArena ar,
-                             unsigned char *keep_rows) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= count) return;
-  const long long v0 = vs[c], e0 = es[c];
-  const int nv = int(vs[c + 1] - v0), E = int(es[c + 1] - e0);
-  const long long cbase = e0 + c, sbase = 2 * (e0 + c), hbase = 2 * (e0 + c) + 2LL * c;
-  int *bc = ar.bc + v0, *slot_head = ar.slot_head + v0;
-  int4 *stack = ar.stack + v0 + c;
-  float *sdist = ar.stack_dist + v0 + c;
-  int *su = ar.su + cbase, *sv = ar.sv + cbase, *ver = ar.ver + cbase;
-  int *cf = ar.chain_first + cbase, *cla = ar.chain_last + cbase, *cn = ar.chain_next + cbase;
-  double *len = ar.len + cbase;
-  unsigned char *alive = ar.alive + cbase, *eligible = ar.eligible + cbase, *dead = ar.dead + cbase;
-  int *snext = ar.slot_next + sbase, *sowner = ar.slot_owner + sbase;
-  int *chain_of = ar.chain_of + e0;
-  Heap heap{ar.heap_len + hbase, ar.heap_lo + hbase, ar.heap_hi + hbase, ar.heap_id + hbase, ar.heap_ver + hbase, 0};
-  const long long *off = csr_off + v0;
-  const int *vl = vlist + v0;
-  auto deg = [&](int v) { return int(off[v + 1] - off[v]); };
-  int start = -1;
-  for (int v = 0; v < nv; ++v) {
-    const int d = deg(v);
-    bc[v] = d >= 3 ? d : 0;
-    slot_head[v] = -1;
-    if (start < 0 && d == 1) start = v;
+// A tree's state: I indexes (pointer to short in LDS, int in device memory), D doubles, F floats, B
+// bytes. A tree of `critical` vertices of degree 1 or at least 3 has critical - 1 chains between them, at
+// most 2 of them ever enter the heap per chain (one at first, one per fusion), and its search stack
+// holds roots of subtrees not entered yet, each with a leaf of its own.
+template <class I, class D, class F, class B> struct TickState {
+  D len;                                   // chains
+  Heap<I, D> heap;                         // 2 per chain
+  F pos, sdist;                            // 3 nv; stack
+  I off, child, row;                       // nv + 1; 2 E: the neighbours
+  I bc, slot_head;                         // nv
+  I node, parent, root, chain;             // stack
+  I su, sv, ver, cf, cla, cn;              // chains
+  I snext, sowner;                         // 2 per chain
+  I chain_of;                              // E: row -> chain
+  B alive, eligible, dead;                 // chains
+};
+template <class T> size_t tick_bytes(size_t nv, size_t E, size_t critical) {
+  const size_t C = critical + 1, H = 2 * C + 2, S = critical + 2;
+  return 8 * (C + H) + 4 * (3 * nv + S) + sizeof(T) * (4 * H + nv + 1 + 4 * E + 2 * nv + 4 * S + 6 * C + 4 * C + E) + 3 * C;
+}
+template <class I, class D, class F, class B> __device__ TickState<I, D, F, B> tick_state(D at, int nv, int E, int critical) {
+  const int C = critical + 1, H = 2 * C + 2, S = critical + 2;
+  TickState<I, D, F, B> s;
+  s.len = at;
+  s.heap.len = at + C;
+  F f = (F)(at + C + H);
+  s.pos = f;
+  s.sdist = f + 3 * nv;
+  I i = (I)(f + 3 * nv + S);
+  auto take = [&](int n) { I p = i; i += n; return p; };
+  s.heap.lo = take(H);
+  s.heap.hi = take(H);
+  s.heap.id = take(H);
+  s.heap.ver = take(H);
+  s.off = take(nv + 1);
+  s.child = take(2 * E);
+  s.row = take(2 * E);
+  s.bc = take(nv);
+  s.slot_head = take(nv);
+  s.node = take(S);
+  s.parent = take(S);
+  s.root = take(S);
+  s.chain = take(S);
+  s.su = take(C);
+  s.sv = take(C);
+  s.ver = take(C);
+  s.cf = take(C);
+  s.cla = take(C);
+  s.cn = take(C);
+  s.snext = take(2 * C);
+  s.sowner = take(2 * C);
+  s.chain_of = take(E);
+  s.alive = (B)i;
+  s.eligible = s.alive + C;
+  s.dead = s.eligible + C;
+  return s;
+}
+
+// keep_rows[r]: row r of the tree stays. off, csr: the CSR from the tree's first vertex on.
+template <class I, class D, class F, class B>
+__device__ void ticks_component(TickState<I, D, F, B> &s, int nv, int E, const int *vl, const float *vertices, const long long *off,
+                                const unsigned long long *csr, double threshold, unsigned char *keep_rows) {
+  const int lane = threadIdx.x;
+  const long long base = off[0];
+  for (int v = lane; v <= nv; v += 64) s.off[v] = int(off[v] - base);
+  for (int q = lane; q < 2 * E; q += 64) {
+    const unsigned long long x = csr[base + q];
+    s.child[q] = int(x >> 32);
+    s.row[q] = int(unsigned(x));
   }
-  for (int r = 0; r < E; ++r) keep_rows[e0 + r] = 1;
-  if (start < 0) return;
+  for (int j = lane; j < 3 * nv; j += 64) s.pos[j] = vertices[3LL * vl[j / 3] + j % 3];
+  wave_sync();
+  auto deg = [&](int v) { return int(s.off[v + 1]) - int(s.off[v]); };
+  int start = INT_MAX;
+  for (int v = lane; v < nv; v += 64) {
+    const int d = deg(v);
+    s.bc[v] = d >= 3 ? d : 0;
+    s.slot_head[v] = -1;
+    if (d == 1) start = min(start, v);
+  }
+  for (int o = 32; o > 0; o >>= 1) start = min(start, __shfl_xor(start, o, 64));
+  wave_sync();
+  if (start == INT_MAX) {
+    for (int r = lane; r < E; r += 64) keep_rows[r] = 1;
+    return;
+  }
   int chains = 0, sp = 0;
-  stack[sp] = make_int4(start, -1, start, -1);
-  sdist[sp++] = 0.0f;
+  s.node[sp] = start;
+  s.parent[sp] = -1;
+  s.root[sp] = start;
+  s.chain[sp] = -1;
+  s.sdist[sp++] = 0.0f;
   while (sp) {
     --sp;
-    const int node = stack[sp].x, parent = stack[sp].y;
-    int root = stack[sp].z, chain = stack[sp].w;
-    float dist = sdist[sp];
-    const int d = deg(node);
+    const int node = s.node[sp], parent = s.parent[sp];
+    int root = s.root[sp], chain = s.chain[sp];
+    float dist = s.sdist[sp];
+    const int q0 = s.off[node], q1 = s.off[node + 1], d = q1 - q0;
     if ((d == 1 || d >= 3) && node != root) {  // a chain reaches a critical node: a super-edge
-      su[chain] = root;
-      sv[chain] = node;
-      len[chain] = double(dist);
-      ver[chain] = 0;
-      alive[chain] = 1;
-      eligible[chain] = deg(root) == 1 || d == 1;
-      snext[2 * chain] = slot_head[root];
-      slot_head[root] = 2 * chain;
-      snext[2 * chain + 1] = slot_head[node];
-      slot_head[node] = 2 * chain + 1;
-      sowner[2 * chain] = sowner[2 * chain + 1] = chain;
-      if (eligible[chain]) heap.push(len[chain], root, node, chain, 0);
+      s.su[chain] = root;
+      s.sv[chain] = node;
+      s.len[chain] = double(dist);
+      s.ver[chain] = 0;
+      s.alive[chain] = 1;
+      const bool el = deg(root) == 1 || d == 1;
+      s.eligible[chain] = el;
+      s.snext[2 * chain] = s.slot_head[root];
+      s.slot_head[root] = 2 * chain;
+      s.snext[2 * chain + 1] = s.slot_head[node];
+      s.slot_head[node] = 2 * chain + 1;
+      s.sowner[2 * chain] = s.sowner[2 * chain + 1] = chain;
+      if (el) s.heap.push(double(dist), root, node, chain, 0);
       dist = 0.0f;
       root = node;
     }
-    const float *pn = vertices + 3LL * vl[node];
-    for (long long q = off[node]; q < off[node + 1]; ++q) {
-      const int child = int(csr[q] >> 32), row = int(unsigned(csr[q]));
+    const float nx = s.pos[3 * node], ny = s.pos[3 * node + 1], nz = s.pos[3 * node + 2];
+    for (int q = q0; q < q1; ++q) {
+      const int child = s.child[q], row = s.row[q];
       if (child == parent) continue;
-      const float *pc = vertices + 3LL * vl[child];
-      float dx = pn[0] - pc[0], dy = pn[1] - pc[1], dz = pn[2] - pc[2];
+      float dx = nx - s.pos[3 * child], dy = ny - s.pos[3 * child + 1], dz = nz - s.pos[3 * child + 2];
       dx *= dx;
       dy *= dy;
       dz *= dz;
       int ch = chain;
       if (node == root) {  // a chain leaves a critical node
         ch = chains++;
-        cf[ch] = cla[ch] = ch;
-        cn[ch] = -1;
-        dead[ch] = 0;
-        alive[ch] = 0;
-        eligible[ch] = 0;
+        s.cf[ch] = s.cla[ch] = ch;
+        s.cn[ch] = -1;
+        s.dead[ch] = 0;
+        s.alive[ch] = 0;
+        s.eligible[ch] = 0;
       }
-      chain_of[row] = ch;
-      stack[sp] = make_int4(child, node, root, ch);
-      sdist[sp++] = dist + sqrtf((dx + dy) + dz);
+      s.chain_of[row] = ch;
+      s.node[sp] = child;
+      s.parent[sp] = node;
+      s.root[sp] = root;
+      s.chain[sp] = ch;
+      s.sdist[sp++] = dist + sqrtf((dx + dy) + dz);
     }
   }
   int nalive = 0;
-  for (int k = 0; k < chains; ++k) nalive += alive[k];
+  for (int k = 0; k < chains; ++k) nalive += s.alive[k];
   while (nalive > 1) {
-    while (heap.n > 0 && (!alive[heap.id[0]] || ver[heap.id[0]] != heap.ver[0])) heap.pop();
-    if (heap.n == 0) break;
-    const int best = heap.id[0];
-    const int e1 = su[best], e2 = sv[best];
-    if (bc[e1] == 1 && bc[e2] == 1) break;
-    if (len[best] >= threshold) break;
-    heap.pop();
-    for (int k = cf[best]; k >= 0; k = cn[k]) dead[k] = 1;
-    alive[best] = 0;
+    while (s.heap.n > 0 && (!s.alive[s.heap.id[0]] || s.ver[s.heap.id[0]] != s.heap.ver[0])) s.heap.pop();
+    if (s.heap.n == 0) break;
+    const int best = s.heap.id[0];
+    const int e1 = s.su[best], e2 = s.sv[best];
+    if (s.bc[e1] == 1 && s.bc[e2] == 1) break;
+    if (s.len[best] >= threshold) break;
+    s.heap.pop();
+    for (int k = s.cf[best]; k >= 0; k = s.cn[k]) s.dead[k] = 1;
+    s.alive[best] = 0;
     nalive--;
-    bc[e1] -= 1;
-    bc[e2] -= 1;
+    s.bc[e1] -= 1;
+    s.bc[e2] -= 1;
     for (int t = 0; t < 2; ++t) {
       const int v = t ? e2 : e1;
-      if (bc[v] != 2) continue;
+      if (s.bc[v] != 2) continue;
       int a = -1, b = -1;
-      for (int k = slot_head[v]; k >= 0; k = snext[k]) {
-        const int o = sowner[k];
-        if (!alive[o] || (su[o] != v && sv[o] != v) || o == a) continue;
+      for (int k = s.slot_head[v]; k >= 0; k = s.snext[k]) {
+        const int o = s.sowner[k];
+        if (!s.alive[o] || (s.su[o] != v && s.sv[o] != v) || o == a) continue;
         if (a < 0) a = o;
         else { b = o; break; }
       }
-      if (a < 0 || b < 0) { bc[v] = 0; continue; }
-      const int ea = su[a] == v ? sv[a] : su[a], eb = su[b] == v ? sv[b] : su[b];
-      len[a] = (0.0 + len[a]) + len[b];
-      su[a] = ea;
-      sv[a] = eb;
-      eligible[a] = 1;
-      cn[cla[a]] = cf[b];
-      cla[a] = cla[b];
-      alive[b] = 0;
+      if (a < 0 || b < 0) { s.bc[v] = 0; continue; }
+      const int ea = s.su[a] == v ? s.sv[a] : s.su[a], eb = s.su[b] == v ? s.sv[b] : s.su[b];
+      const double la = (0.0 + s.len[a]) + s.len[b];
+      s.len[a] = la;
+      s.su[a] = ea;
+      s.sv[a] = eb;
+      s.eligible[a] = 1;
+      s.cn[s.cla[a]] = s.cf[b];
+      s.cla[a] = s.cla[b];
+      s.alive[b] = 0;
       nalive--;
-      for (int k = slot_head[eb]; k >= 0; k = snext[k])
-        if (sowner[k] == b) sowner[k] = a;
-      ver[a] += 1;
-      heap.push(len[a], ea, eb, a, ver[a]);
-      bc[v] = 0;
+      for (int k = s.slot_head[eb]; k >= 0; k = s.snext[k])
+        if (s.sowner[k] == b) s.sowner[k] = a;
+      const int ver = s.ver[a] + 1;
+      s.ver[a] = ver;
+      s.heap.push(la, ea, eb, a, ver);
+      s.bc[v] = 0;
     }
   }
-  for (int r = 0; r < E; ++r) keep_rows[e0 + r] = !dead[chain_of[r]];
+  wave_sync();
+  for (int r = lane; r < E; r += 64) keep_rows[r] = !s.dead[s.chain_of[r]];
+}
+
+// Block b: tree list[b], its state in LDS.
+__global__ void __launch_bounds__(64) ticks_small(const int *list, const long long *vs, const long long *es, const int *critical,
+                                                  const int *vlist, const float *vertices, const long long *csr_off,
+                                                  const unsigned long long *csr, double threshold, unsigned char *keep_rows) {
+  const int c = list[blockIdx.x];
+  const long long v0 = vs[c], e0 = es[c];
+  const int nv = int(vs[c + 1] - v0), E = int(es[c + 1] - e0);
+  auto s = tick_state<InLds<short> *, InLds<double> *, InLds<float> *, InLds<unsigned char> *>((InLds<double> *)post_lds, nv, E,
+                                                                                             critical[c]);
+  ticks_component(s, nv, E, vlist + v0, vertices, csr_off + v0, csr, threshold, keep_rows + e0);
+}
+
+// Block b: tree list[b], its state at slot starts[b] (doubles) of `arena`.
+__global__ void __launch_bounds__(64) ticks_large(const int *list, const long long *starts, double *arena, const long long *vs,
+                                                  const long long *es, const int *critical, const int *vlist,
+                                                  const float *vertices, const long long *csr_off,
+                                                  const unsigned long long *csr, double threshold, unsigned char *keep_rows) {
+  const int c = list[blockIdx.x];
+  const long long v0 = vs[c], e0 = es[c];
+  const int nv = int(vs[c + 1] - v0), E = int(es[c + 1] - e0);
+  auto s = tick_state<InGlobal<int> *, InGlobal<double> *, InGlobal<float> *, InGlobal<unsigned char> *>(
+      (InGlobal<double> *)(arena + starts[blockIdx.x]), nv, E, critical[c]);
+  ticks_component(s, nv, E, vlist + v0, vertices, csr_off + v0, csr, threshold, keep_rows + e0);
 }
 
 __global__ void tick_keep(const int *elist, const unsigned char *keep_rows, int M, int *keep) {
@@ -1185,43 +1518,51 @@ DevicePacked remove_ticks(Context &ctx, DevicePacked p, double threshold) {
   auto s = ctx.stream();
   const long long A = pc.count, N = pc.nv, M = pc.ne;
   if (M > INT32_MAX / 2) throw std::invalid_argument("tick adjacency exceeds int32 capacity");
-  Buffer<int> comp_of_edge(ctx, size_t(M));
-  edge_component<<<grid(A), kThreads, 0, s>>>(pc.es.data(), pc.count, comp_of_edge.data());
   Buffer<unsigned> source(ctx, size_t(2 * M)), source_sorted(ctx, size_t(2 * M));
   Buffer<unsigned long long> value(ctx, size_t(2 * M)), csr(ctx, size_t(2 * M));
-  csr_entries<<<grid(M), kThreads, 0, s>>>(pc.rows.data(), pc.vs.data(), pc.es.data(), comp_of_edge.data(), int(M),
+  csr_entries<<<grid(M), kThreads, 0, s>>>(pc.rows.data(), pc.vs.data(), pc.es.data(), pc.comp_of_edge.data(), int(M),
                                            source.data(), value.data());
   BROOK_LAUNCHED();
   Buffer<unsigned char> scratch;
   with_scratch(ctx, scratch, [&](void *t, size_t &b) {
     return hipcub::DeviceRadixSort::SortPairs(t, b, source.data(), source_sorted.data(), value.data(), csr.data(), int(2 * M), 0,
-                                              32, s);
+                                              bits_for(N), s);
   });
-  Buffer<int> deg(ctx, size_t(N) + 1);
-  deg.clear(ctx);
-  csr_degree<<<grid(2 * M), kThreads, 0, s>>>(source_sorted.data(), int(2 * M), deg.data());
-  BROOK_LAUNCHED();
   Buffer<long long> off(ctx, size_t(N) + 1);
-  {
-    std::vector<int> h = deg.download(ctx);
-    std::vector<long long> o(size_t(N) + 1, 0);
-    for (long long v = 0; v < N; ++v) o[v + 1] = o[v] + h[v];
-    off.upload(ctx, o.data(), o.size());
+  csr_offsets<<<grid(N + 1), kThreads, 0, s>>>(source_sorted.data(), 2 * M, N, off.data());
+  BROOK_LAUNCHED();
+  Buffer<unsigned char> keep_rows(ctx, size_t(M));
+  Buffer<int> critical(ctx, size_t(A));
+  critical.upload(ctx, pc.critical.data(), size_t(A));
+  const Split sp = split_pieces(ctx, pc, [&](size_t c, size_t nv, size_t E) { return tick_bytes<short>(nv, E, size_t(pc.critical[c])); });
+  if (sp.nsmall) {
+    BROOK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(ticks_small), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  int(kLdsPiece)));
+    ticks_small<<<unsigned(sp.nsmall), 64, sp.lds, s>>>(sp.small.data(), pc.vs.data(), pc.es.data(), critical.data(),
+                                                       pc.vlist.data(), p.vertices.data(), off.data(), csr.data(), threshold,
+                                                       keep_rows.data());
+    BROOK_LAUNCHED();
   }
-  const size_t nodes = size_t(N), nodes1 = size_t(N + A), chains = size_t(M + A), slots = size_t(2 * (M + A)),
-               heapsz = size_t(2 * (M + A) + 2 * A);
-  Buffer<int> bc(ctx, nodes), slot_head(ctx, nodes), su(ctx, chains), sv(ctx, chains), ver(ctx, chains), cf(ctx, chains),
-      cl(ctx, chains), cn(ctx, chains), snext(ctx, slots), sowner(ctx, slots), hlo(ctx, heapsz), hhi(ctx, heapsz),
-      hid(ctx, heapsz), hver(ctx, heapsz), chain_of(ctx, size_t(M));
-  Buffer<int4> stack(ctx, nodes1);
-  Buffer<float> sdist(ctx, nodes1);
-  Buffer<double> len(ctx, chains), hlen(ctx, heapsz);
-  Buffer<unsigned char> alive(ctx, chains), eligible(ctx, chains), dead(ctx, chains), keep_rows(ctx, size_t(M));
-  TickArena ar{bc.data(), slot_head.data(), stack.data(), sdist.data(), su.data(), sv.data(), ver.data(), cf.data(), cl.data(),
-               cn.data(), len.data(), alive.data(), eligible.data(), dead.data(), snext.data(), sowner.data(), hlen.data(),
-               hlo.data(), hhi.data(), hid.data(), hver.data(), chain_of.data()};
-  ticks_kernel<<<unsigned((A + 63) / 64), 64, 0, s>>>(pc.count, pc.vs.data(), pc.es.data(), pc.vlist.data(), p.vertices.data(),
-                                                     off.data(), csr.data(), threshold, ar, keep_rows.data());
+  Buffer<double> arena;
+  Buffer<long long> starts_dev;
+  if (sp.nlarge) {
+    std::vector<int> large = sp.large.download(ctx);
+    std::vector<long long> starts;
+    long long doubles = 0;
+    for (int c : large) {
+      starts.push_back(doubles);
+      doubles += (long long)((tick_bytes<int>(size_t(pc.vs_host[size_t(c) + 1] - pc.vs_host[size_t(c)]),
+                                              size_t(pc.es_host[size_t(c) + 1] - pc.es_host[size_t(c)]),
+                                              size_t(pc.critical[size_t(c)])) + 7) / 8);
+    }
+    arena = Buffer<double>(ctx, size_t(doubles));
+    starts_dev = Buffer<long long>(ctx, starts.size());
+    starts_dev.upload(ctx, starts.data(), starts.size());
+    ticks_large<<<unsigned(sp.nlarge), 64, 0, s>>>(sp.large.data(), starts_dev.data(), arena.data(), pc.vs.data(), pc.es.data(),
+                                                  critical.data(), pc.vlist.data(), p.vertices.data(), off.data(), csr.data(),
+                                                  threshold, keep_rows.data());
+    BROOK_LAUNCHED();
+  }
   Buffer<int> keep(ctx, size_t(g.m));
   fill_ones<<<grid(g.m), kThreads, 0, s>>>(keep.data(), g.m);
   tick_keep<<<grid(M), kThreads, 0, s>>>(pc.elist.data(), keep_rows.data(), int(M), keep.data());
@@ -1234,31 +1575,49 @@ DevicePacked remove_ticks(Context &ctx, DevicePacked p, double threshold) {
 
 __global__ void join_statistics(const int *root, const int *vlabel, const float *radii, int n, int *ncomp, unsigned *rmax) {
   const int i = blockIdx.x * kThreads + threadIdx.x;
-  if (i >= n) return;
-  const int l = vlabel[i];
-  if (root[i] == i) atomicAdd(ncomp + l, 1);
-  const float r = radii[i];
-  if (r > 0) atomicMax(rmax + l, __float_as_uint(r));
+  const int l = i < n ? vlabel[i] : -1;
+  if (i < n && root[i] == i) atomicAdd(ncomp + l, 1);
+  const float r = i < n ? radii[i] : 0.0f;
+  unsigned top = r > 0 ? __float_as_uint(r) : 0u;
+  // vertices come label by label: a wave of one label sends one maximum
+  const int first = __shfl(l, 0, 64);
+  if (__all(l == first)) {
+    for (int o = 32; o > 0; o >>= 1) top = max(top, unsigned(__shfl_xor(int(top), o, 64)));
+    if ((threadIdx.x & 63) != 0) top = 0u;
+  }
+  if (top && l >= 0) atomicMax(rmax + l, top);
 }
 
-// Cell of a vertex of a label with several components: (rank, floor(coordinate / bound)).
+// Cell of a vertex of a label with several components: (rank, floor(coordinate / bound)); the others'
+// rank is LLONG_MAX. range: least and greatest rank, x, y, z over the members (LLONG_MAX, LLONG_MIN
+// before).
 __global__ void join_cells(const int *vlabel, const int *rank, const double *bound, const float *v, int n, long long *kl,
-                           long long *kx, long long *ky, long long *kz, int *index, int *member) {
+                           long long *kx, long long *ky, long long *kz, int *index, long long *range) {
   const int i = blockIdx.x * kThreads + threadIdx.x;
-  if (i >= n) return;
-  const int r = rank[vlabel[i]];
-  member[i] = r >= 0;
-  index[i] = i;
-  if (r < 0) {
-    kl[i] = LLONG_MAX;
-    kx[i] = ky[i] = kz[i] = 0;
-    return;
+  const int r = i < n ? rank[vlabel[i]] : -1;
+  long long k[3] = {0, 0, 0};
+  if (r >= 0) {
+    const double b = bound[r];
+    for (int a = 0; a < 3; ++a) k[a] = (long long)floor(double(v[3LL * i + a]) / b);
   }
-  const double b = bound[r];
-  kl[i] = r;
-  kx[i] = (long long)floor(double(v[3LL * i]) / b);
-  ky[i] = (long long)floor(double(v[3LL * i + 1]) / b);
-  kz[i] = (long long)floor(double(v[3LL * i + 2]) / b);
+  if (i < n) {
+    index[i] = i;
+    kl[i] = r < 0 ? LLONG_MAX : r;
+    kx[i] = k[0];
+    ky[i] = k[1];
+    kz[i] = k[2];
+  }
+  for (int a = 0; a < 3; ++a) {
+    long long lo = r < 0 ? LLONG_MAX : k[a], hi = r < 0 ? LLONG_MIN : k[a];
+    for (int o = 32; o > 0; o >>= 1) {
+      lo = min(lo, __shfl_xor(lo, o, 64));
+      hi = max(hi, __shfl_xor(hi, o, 64));
+    }
+    if ((threadIdx.x & 63) == 0 && lo <= hi) {
+      atomicMin(range + 2 * a, lo);
+      atomicMax(range + 2 * a + 1, hi);
+    }
+  }
 }
 
 __global__ void permute_key(const long long *key, const int *order, int n, long long *out) {
@@ -1266,80 +1625,170 @@ __global__ void permute_key(const long long *key, const int *order, int n, long 
   if (i < n) out[i] = key[order[i]];
 }
 
-struct Cells {
-  const int *order;  // sorted position -> vertex
+__global__ void iota(int *out, int n) {
+  const int i = blockIdx.x * kThreads + threadIdx.x;
+  if (i < n) out[i] = i;
+}
+
+// A vertex in cell order: what its neighbours' searches read.
+struct alignas(16) CellVertex {
+  float x, y, z;
+  int root;
+};
+__global__ void cell_vertices(const int *order, const float *v, const int *root, int n, CellVertex *out) {
+  const int p = blockIdx.x * kThreads + threadIdx.x;
+  if (p >= n) return;
+  const int i = order[p];
+  out[p] = CellVertex{v[3LL * i], v[3LL * i + 1], v[3LL * i + 2], root[i]};
+}
+
+// Cells whose four coordinates fit one 64-bit key (z in the low bits): the sorted keys.
+struct CellRange {
+  long long least[3];
+  int bits[3];
+  unsigned long long most[3];  // greatest coordinate, from the least
+};
+__global__ void pack_cells(const long long *kl, const long long *kx, const long long *ky, const long long *kz, int n, CellRange r,
+                           unsigned long long *key) {
+  const int i = blockIdx.x * kThreads + threadIdx.x;
+  if (i >= n) return;
+  if (kl[i] == LLONG_MAX) { key[i] = kNone; return; }
+  const unsigned long long x = (unsigned long long)(kx[i] - r.least[0]), y = (unsigned long long)(ky[i] - r.least[1]),
+                           z = (unsigned long long)(kz[i] - r.least[2]);
+  key[i] = ((((unsigned long long)kl[i] << r.bits[0] | x) << r.bits[1]) | y) << r.bits[2] | z;
+}
+struct PackedCells {
+  const unsigned long long *key;  // per position
+  int n;
+  CellRange r;
+  struct Cell { unsigned long long key; };
+  __device__ Cell at(int pos) const { return Cell{key[pos]}; }
+  __device__ static Cell from_lane(const Cell &c, int lane) { return Cell{__shfl(c.key, lane, 64)}; }
+  __device__ static bool same(const Cell &a, const Cell &b) { return a.key == b.key; }
+  __device__ bool member(const Cell &c) const { return c.key != kNone; }
+  __device__ int rank(const Cell &c) const { return int(c.key >> (r.bits[0] + r.bits[1] + r.bits[2])); }
+  // First position at or past cell (x + dx, y + dy, z - 1) (end false), or past (x + dx, y + dy, z + 1).
+  __device__ int bound(const Cell &c, int dx, int dy, bool end) const {
+    auto field = [&](int shift, int bits) { return (c.key >> shift) & ((1ULL << bits) - 1ULL); };
+    const unsigned long long x = field(r.bits[1] + r.bits[2], r.bits[0]), y = field(r.bits[2], r.bits[1]), z = field(0, r.bits[2]);
+    if ((dx < 0 && x == 0) || (dx > 0 && x == r.most[0]) || (dy < 0 && y == 0) || (dy > 0 && y == r.most[1])) return 0;  // no such column
+    const unsigned long long nz = end ? (z < r.most[2] ? z + 1 : z) : (z > 0 ? z - 1 : z);
+    unsigned long long k = c.key >> (r.bits[0] + r.bits[1] + r.bits[2]);
+    k = ((((k << r.bits[0]) | (x + dx)) << r.bits[1]) | (y + dy)) << r.bits[2] | nz;
+    int lo = 0, hi = n;
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (key[mid] < k || (end && key[mid] == k)) lo = mid + 1;
+      else hi = mid;
+    }
+    return lo;
+  }
+};
+
+// Cells of any coordinates (a label whose radii are all 0 has cells of a millionth): four keys per vertex.
+struct WideCells {
+  const int *order;  // position -> vertex
   const long long *kl, *kx, *ky, *kz;  // per vertex
   int n;
-  __device__ int cmp(int pos, long long l, long long x, long long y, long long z) const {
+  struct Cell { long long l, x, y, z; };
+  __device__ Cell at(int pos) const { const int v = order[pos]; return Cell{kl[v], kx[v], ky[v], kz[v]}; }
+  __device__ static Cell from_lane(const Cell &c, int lane) {
+    return Cell{__shfl(c.l, lane, 64), __shfl(c.x, lane, 64), __shfl(c.y, lane, 64), __shfl(c.z, lane, 64)};
+  }
+  __device__ static bool same(const Cell &a, const Cell &b) { return a.l == b.l && a.x == b.x && a.y == b.y && a.z == b.z; }
+  __device__ bool member(const Cell &c) const { return c.l != LLONG_MAX; }
+  __device__ int rank(const Cell &c) const { return int(c.l); }
+  __device__ int cmp(int pos, const Cell &c) const {
     const int v = order[pos];
-    if (kl[v] != l) return kl[v] < l ? -1 : 1;
-    if (kx[v] != x) return kx[v] < x ? -1 : 1;
-    if (ky[v] != y) return ky[v] < y ? -1 : 1;
-    if (kz[v] != z) return kz[v] < z ? -1 : 1;
+    if (kl[v] != c.l) return kl[v] < c.l ? -1 : 1;
+    if (kx[v] != c.x) return kx[v] < c.x ? -1 : 1;
+    if (ky[v] != c.y) return ky[v] < c.y ? -1 : 1;
+    if (kz[v] != c.z) return kz[v] < c.z ? -1 : 1;
     return 0;
+  }
+  __device__ int bound(const Cell &c, int dx, int dy, bool end) const {
+    if (c.x == (dx < 0 ? LLONG_MIN : LLONG_MAX) && dx) return 0;  // no such column
+    if (c.y == (dy < 0 ? LLONG_MIN : LLONG_MAX) && dy) return 0;
+    const Cell k{c.l, c.x + dx, c.y + dy, end ? (c.z < LLONG_MAX ? c.z + 1 : c.z) : (c.z > LLONG_MIN ? c.z - 1 : c.z)};
+    int lo = 0, hi = n;
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1, o = cmp(mid, k);
+      if (o < 0 || (end && o == 0)) lo = mid + 1;
+      else hi = mid;
+    }
+    return lo;
   }
 };
 
 constexpr int kJoinTable = 16;
 
-// Per vertex i of a joinable label: for each component above its own within reach, the nearest
-// vertex (ties by the lower index); a vertex meeting more components than its table holds sends
-// the excess straight out. mode 0 counts, mode 1 writes from offs[i].
-__global__ void join_candidates(int n, int mode, Cells cells, const int *member, const int *vlabel, const int *rank,
-                                const double *bound, const float *v, const int *root, long long *counts, const long long *offs,
-                                int *oa, int *ob, double *od, int *ov, int *ou) {
-  const int i = blockIdx.x * kThreads + threadIdx.x;
-  if (i >= n || !member[i]) return;
-  const int r = rank[vlabel[i]];
-  const double bnd = bound[r];
-  float b32 = float(bnd);
-  b32 = b32 * b32 * 1.0001f + 1e-30f;
-  const float px = v[3LL * i], py = v[3LL * i + 1], pz = v[3LL * i + 2];
-  const long long cx = cells.kx[i], cy = cells.ky[i], cz = cells.kz[i];
+// Per vertex of a joinable label: for each component above its own within reach, the nearest vertex
+// (ties by the lower index); a vertex meeting more components than its table holds sends the excess
+// straight out. Candidates go to the places *count gives out, in no order (they are sorted by all
+// their fields), none at or past `cap` (*count then says how many there are).
+// A thread per vertex in cell order, so that a wave's vertices lie in one or a few cells: per cell, lanes
+// find the bounds of its 9 columns of three cells (contiguous positions), then the cell's lanes
+// walk the same positions together, from one array in that order. (166 k vertices of 150 skeletons:
+// 0.33 ms; a search of 27 cells per vertex through the sort order, once to count and once to write,
+// took 2.3 ms.)
+template <class Cells>
+__global__ void __launch_bounds__(kThreads) join_candidates(Cells cells, const CellVertex *cv, const int *order,
+                                                           const double *bound, unsigned long long *count, unsigned long long cap,
+                                                           int *oa, int *ob,
+                                                           double *od, int *ov, int *ou) {
+  const int p = blockIdx.x * kThreads + threadIdx.x, lane = int(threadIdx.x) & 63;
+  const int at = p < cells.n ? p : cells.n - 1;
+  const typename Cells::Cell mine = cells.at(at);
+  const CellVertex me = cv[at];
+  const int i = order[at];
   int tb[kJoinTable], tu[kJoinTable];
   double td[kJoinTable];
   int nt = 0;
-  long long emitted = 0;
-  const long long base = mode ? offs[i] : 0;
-  const int ci = root[i];
-  for (int dz = -1; dz <= 1; ++dz)
-    for (int dy = -1; dy <= 1; ++dy)
-      for (int dx = -1; dx <= 1; ++dx) {
-        const long long x = cx + dx, y = cy + dy, z = cz + dz;
-        int lo = 0, hi = cells.n;
-        while (lo < hi) {
-          const int mid = (lo + hi) >> 1;
-          if (cells.cmp(mid, r, x, y, z) < 0) lo = mid + 1;
-          else hi = mid;
-        }
-        for (int q = lo; q < cells.n && cells.cmp(q, r, x, y, z) == 0; ++q) {
-          const int j = cells.order[q];
-          const int cj = root[j];
-          if (cj <= ci) continue;
-          const float fx = v[3LL * j] - px, fy = v[3LL * j + 1] - py, fz = v[3LL * j + 2] - pz;
-          if ((fx * fx + fy * fy) + fz * fz > b32) continue;
-          const double ex = double(v[3LL * j]) - double(px), ey = double(v[3LL * j + 1]) - double(py),
-                       ez = double(v[3LL * j + 2]) - double(pz);
-          const double d = sqrt((ex * ex + ey * ey) + ez * ez);
-          if (!(d < bnd)) continue;
-          int t = -1;
-          for (int k = 0; k < nt; ++k)
-            if (tb[k] == cj) { t = k; break; }
-          if (t >= 0) {
-            if (d < td[t] || (d == td[t] && j < tu[t])) { td[t] = d; tu[t] = j; }
-          } else if (nt < kJoinTable) {
-            tb[nt] = cj; td[nt] = d; tu[nt] = j; nt++;
-          } else {
-            if (mode) { const long long o = base + emitted; oa[o] = ci; ob[o] = cj; od[o] = d; ov[o] = i; ou[o] = j; }
-            emitted++;
-          }
+  auto emit = [&](int cj, double d, int j) {
+    const unsigned long long o = atomicAdd(count, 1ULL);
+    if (o >= cap) return;
+    oa[o] = me.root;
+    ob[o] = cj;
+    od[o] = d;
+    ov[o] = i;
+    ou[o] = j;
+  };
+  unsigned long long left = __builtin_amdgcn_ballot_w64(p < cells.n && cells.member(mine));
+  while (left) {
+    const int leader = __ffsll((long long)left) - 1;
+    const typename Cells::Cell cell = Cells::from_lane(mine, leader);
+    const int col = lane >> 1;  // lanes 2c, 2c + 1: column c's begin and end
+    const int b = lane < 18 ? cells.bound(cell, col % 3 - 1, col / 3 - 1, lane & 1) : 0;
+    const bool here = ((left >> lane) & 1ULL) && Cells::same(mine, cell);
+    left &= ~__builtin_amdgcn_ballot_w64(here);
+    const double bnd = bound[cells.rank(cell)];
+    float b32 = float(bnd);
+    b32 = b32 * b32 * 1.0001f + 1e-30f;
+    for (int c = 0; c < 9; ++c) {
+      const int q0 = __shfl(b, 2 * c, 64), q1 = __shfl(b, 2 * c + 1, 64);
+      for (int q = q0; q < q1; ++q) {
+        const CellVertex o = cv[q];
+        if (!here || o.root <= me.root) continue;
+        const float fx = o.x - me.x, fy = o.y - me.y, fz = o.z - me.z;
+        if ((fx * fx + fy * fy) + fz * fz > b32) continue;
+        const double ex = double(o.x) - double(me.x), ey = double(o.y) - double(me.y), ez = double(o.z) - double(me.z);
+        const double d = sqrt((ex * ex + ey * ey) + ez * ez);
+        if (!(d < bnd)) continue;
+        const int j = order[q];
+        int t = -1;
+        for (int k = 0; k < nt; ++k)
+          if (tb[k] == o.root) { t = k; break; }
+        if (t >= 0) {
+          if (d < td[t] || (d == td[t] && j < tu[t])) { td[t] = d; tu[t] = j; }
+        } else if (nt < kJoinTable) {
+          tb[nt] = o.root; td[nt] = d; tu[nt] = j; nt++;
+        } else {
+          emit(o.root, d, j);
         }
       }
-  for (int k = 0; k < nt; ++k) {
-    if (mode) { const long long o = base + emitted; oa[o] = ci; ob[o] = tb[k]; od[o] = td[k]; ov[o] = i; ou[o] = tu[k]; }
-    emitted++;
+    }
   }
-  if (!mode) counts[i] = emitted;
+  for (int k = 0; k < nt; ++k) emit(tb[k], td[k], tu[k]);
 }
 
 __global__ void candidate_key(const int *order, int n, const int *a, const int *b, const double *d, const int *va, const int *vb,
@@ -1501,52 +1950,83 @@ DevicePacked join_components(Context &ctx, DevicePacked input) {
   bound_dev.upload(ctx, bound.data(), labels);
   Buffer<long long> cs_dev(ctx, cs.size());
   cs_dev.upload(ctx, cs.data(), cs.size());
-  // cells: a stable multi-key sort by (rank, x, y, z) cell, least significant key first
-  Buffer<long long> kl(ctx, g.n), kx(ctx, g.n), ky(ctx, g.n), kz(ctx, g.n), key(ctx, g.n), key_sorted(ctx, g.n);
-  Buffer<int> order(ctx, g.n), order_sorted(ctx, g.n), member(ctx, g.n);
+  // cells, sorted by (rank, x, y, z): one key where the coordinates' ranges fit 64 bits, else a stable
+  // sort per coordinate, least significant first
+  Buffer<long long> kl(ctx, g.n), kx(ctx, g.n), ky(ctx, g.n), kz(ctx, g.n), range_dev(ctx, 6);
+  Buffer<int> order(ctx, g.n), order_sorted(ctx, g.n);
+  long long range[6] = {LLONG_MAX, LLONG_MIN, LLONG_MAX, LLONG_MIN, LLONG_MAX, LLONG_MIN};
+  range_dev.upload(ctx, range, 6);
   join_cells<<<grid(g.n), kThreads, 0, s>>>(g.vlabel.data(), rank_dev.data(), bound_dev.data(), p.vertices.data(), g.n, kl.data(),
-                                            kx.data(), ky.data(), kz.data(), order.data(), member.data());
-  BROOK_LAUNCHED();
-  Buffer<unsigned char> scratch;
-  for (const Buffer<long long> *k : {&kz, &ky, &kx, &kl}) {
-    permute_key<<<grid(g.n), kThreads, 0, s>>>(k->data(), order.data(), g.n, key.data());
-    BROOK_LAUNCHED();
-    with_scratch(ctx, scratch, [&](void *t, size_t &b) {
-      return hipcub::DeviceRadixSort::SortPairs(t, b, key.data(), key_sorted.data(), order.data(), order_sorted.data(), g.n, 0, 64, s);
-    });
-    std::swap(order, order_sorted);
-  }
-  Cells cells{order.data(), kl.data(), kx.data(), ky.data(), kz.data(), g.n};
-  Buffer<long long> counts(ctx, g.n), offs(ctx, size_t(g.n) + 1);
-  counts.clear(ctx);
-  join_candidates<<<grid(g.n), kThreads, 0, s>>>(g.n, 0, cells, member.data(), g.vlabel.data(), rank_dev.data(), bound_dev.data(),
-                                                 p.vertices.data(), g.root.data(), counts.data(), nullptr, nullptr, nullptr,
-                                                 nullptr, nullptr, nullptr);
+                                            kx.data(), ky.data(), kz.data(), order.data(), range_dev.data());
   BROOK_LAUNCHED();
   {
-    Buffer<long long> padded(ctx, size_t(g.n) + 1);
-    BROOK_HIP(hipMemcpyAsync(padded.data(), counts.data(), size_t(g.n) * 8, hipMemcpyDeviceToDevice, s));
-    BROOK_HIP(hipMemsetAsync(padded.data() + g.n, 0, 8, s));
-    exclusive_sum(ctx, padded.data(), offs.data(), g.n + 1);
+    const std::vector<long long> h = range_dev.download(ctx);
+    std::copy(h.begin(), h.end(), range);
   }
-  const long long total = read_one(ctx, offs.data() + g.n);
-  if (!total) return p;
-  if (total > INT32_MAX) throw std::invalid_argument("join candidates exceed int32 capacity");
-  const int nt = int(total);
-  Buffer<int> ca(ctx, nt), cb(ctx, nt), cv(ctx, nt), cu(ctx, nt);
-  Buffer<double> cd(ctx, nt);
-  join_candidates<<<grid(g.n), kThreads, 0, s>>>(g.n, 1, cells, member.data(), g.vlabel.data(), rank_dev.data(), bound_dev.data(),
-                                                 p.vertices.data(), g.root.data(), counts.data(), offs.data(), ca.data(),
-                                                 cb.data(), cd.data(), cv.data(), cu.data());
+  CellRange cr{};
+  int key_bits = bits_for(labels);
+  for (int a = 0; a < 3; ++a) {
+    cr.least[a] = range[2 * a];
+    cr.most[a] = (unsigned long long)range[2 * a + 1] - (unsigned long long)range[2 * a];
+    while (cr.bits[a] < 64 && (cr.most[a] >> cr.bits[a])) ++cr.bits[a];
+    key_bits += cr.bits[a];
+  }
+  const bool packed = key_bits < 64;  // kNone, of the others, sorts last
+  Buffer<unsigned char> scratch;
+  Buffer<unsigned long long> cell_key(ctx, packed ? size_t(g.n) : 1);
+  if (packed) {
+    Buffer<unsigned long long> key(ctx, g.n);
+    pack_cells<<<grid(g.n), kThreads, 0, s>>>(kl.data(), kx.data(), ky.data(), kz.data(), g.n, cr, key.data());
+    BROOK_LAUNCHED();
+    with_scratch(ctx, scratch, [&](void *t, size_t &b) {
+      return hipcub::DeviceRadixSort::SortPairs(t, b, key.data(), cell_key.data(), order.data(), order_sorted.data(), g.n, 0,
+                                                key_bits + 1, s);
+    });
+    std::swap(order, order_sorted);
+  } else {
+    Buffer<long long> key(ctx, g.n), key_sorted(ctx, g.n);
+    for (const Buffer<long long> *k : {&kz, &ky, &kx, &kl}) {
+      permute_key<<<grid(g.n), kThreads, 0, s>>>(k->data(), order.data(), g.n, key.data());
+      BROOK_LAUNCHED();
+      with_scratch(ctx, scratch, [&](void *t, size_t &b) {
+        return hipcub::DeviceRadixSort::SortPairs(t, b, key.data(), key_sorted.data(), order.data(), order_sorted.data(), g.n, 0, 64, s);
+      });
+      std::swap(order, order_sorted);
+    }
+  }
+  Buffer<CellVertex> cell_verts(ctx, g.n);
+  cell_vertices<<<grid(g.n), kThreads, 0, s>>>(order.data(), p.vertices.data(), g.root.data(), g.n, cell_verts.data());
   BROOK_LAUNCHED();
+  Buffer<int> ca, cb, cv, cu;
+  Buffer<double> cd;
+  Buffer<unsigned long long> found(ctx, 1);
+  unsigned long long total = 0;
+  for (unsigned long long cap = std::max(g.n, 4096);; cap = total) {
+    ca = Buffer<int>(ctx, cap);
+    cb = Buffer<int>(ctx, cap);
+    cv = Buffer<int>(ctx, cap);
+    cu = Buffer<int>(ctx, cap);
+    cd = Buffer<double>(ctx, cap);
+    found.clear(ctx);
+    if (packed)
+      join_candidates<<<grid(g.n), kThreads, 0, s>>>(PackedCells{cell_key.data(), g.n, cr}, cell_verts.data(), order.data(),
+                                                     bound_dev.data(), found.data(), cap, ca.data(), cb.data(), cd.data(),
+                                                     cv.data(), cu.data());
+    else
+      join_candidates<<<grid(g.n), kThreads, 0, s>>>(WideCells{order.data(), kl.data(), kx.data(), ky.data(), kz.data(), g.n},
+                                                     cell_verts.data(), order.data(), bound_dev.data(), found.data(), cap, ca.data(),
+                                                     cb.data(), cd.data(), cv.data(), cu.data());
+    BROOK_LAUNCHED();
+    total = read_one(ctx, found.data());
+    if (total > (unsigned long long)INT32_MAX) throw std::invalid_argument("join candidates exceed int32 capacity");
+    if (total <= cap) break;
+  }
+  if (!total) return p;
+  const int nt = int(total);
   // candidates by (A, B, distance, lower vertex, higher vertex); the first of each (A, B) stays
   Buffer<int> porder(ctx, nt), porder_sorted(ctx, nt);
   Buffer<unsigned long long> pkey(ctx, nt), pkey_sorted(ctx, nt);
-  {
-    std::vector<int> iota(nt);
-    for (int i = 0; i < nt; ++i) iota[i] = i;
-    porder.upload(ctx, iota.data(), nt);
-  }
+  iota<<<grid(nt), kThreads, 0, s>>>(porder.data(), nt);
   for (int pass = 0; pass < 3; ++pass) {
     candidate_key<<<grid(nt), kThreads, 0, s>>>(porder.data(), nt, ca.data(), cb.data(), cd.data(), cv.data(), cu.data(), pass,
                                                 pkey.data());
