@@ -562,22 +562,17 @@ class Sample {
   // boxes, a component's box voids become the component; a component painted over, even in part,
   // fills nothing later; then the boxes and first voxels are recomputed.
   void fill_holes() {
-    std::vector<uint8_t> skip(k_, 0);
-    bool painted = false;
+    std::vector<int64_t> ids;
     for (size_t id = 1; id < k_; ++id) {
       const Box &b = boxes_[id];
-      if (!b.count || skip[id]) continue;
+      if (!b.count) continue;
       const int64_t ex = b.hi[0] - b.lo[0] + 1, ey = b.hi[1] - b.lo[1] + 1, ez = b.hi[2] - b.lo[2] + 1;
       if (ex <= 2 || ey <= 2 || ez <= 2 || ex * ey * ez == b.count) continue;  // no voxel can be enclosed
-      if (!enclosed_voids(*cx_, cc_.labels.data(), cc_.cc_bytes, d_, int64_t(id), b)) continue;
-      VoidFill fill(*cx_, cc_.labels.data(), cc_.cc_bytes, d_, int64_t(id), b, k_);
-      fill.paint(*cx_);
-      for (size_t o = 1; o < k_; ++o)
-        if (fill.taken()[o] && o != id) skip[o] = 1;
-      cx_->stats["hole_filled_voxels"] += double(fill.voids());
-      painted = true;
+      ids.push_back(int64_t(id));
     }
-    if (!painted) return;
+    const int64_t filled = fill_voids(*cx_, cc_.labels.data(), cc_.cc_bytes, d_, boxes_, ids);
+    if (!filled) return;
+    cx_->stats["hole_filled_voxels"] += double(filled);
     boxes_ = analyze(*cx_, cc_, d_);
     const std::vector<int64_t> first = first_voxels(*cx_, cc_.labels.data(), cc_.cc_bytes, n_, count_);
     for (size_t id = 1; id < k_; ++id) cc_.roots[id - 1] = first[id];

@@ -208,11 +208,195 @@ int64_t fill_of(Context &ctx, const CC *cc, Dims d, CC id, const Crop &c, size_t
   return int64_t(holes.download(ctx)[0]);
 }
 
+// The first lane of each stretch of one id in a wave looks at the id's minimum so far and sends its
+// voxel only if that is lower: of a million voxels of an id a few reach the atomic (with one atomic
+// per voxel, all of an id's on one word, 5.9 M voxels took 9.8 ms; 0.11 now).
 template <class CC> __global__ void first_of(const CC *cc, long long n, unsigned long long *first) {
   const long long i = (long long)blockIdx.x * kThreads + threadIdx.x;
-  if (i >= n) return;
-  const CC l = cc[i];
-  if (l != CC(0)) g_min(first + (unsigned long long)l, (unsigned long long)i);
+  const CC l = i < n ? cc[i] : CC(0);
+  const CC prev = shfl_up_any(l, 1);
+  if (l == CC(0) || ((threadIdx.x & 63) != 0 && prev == l)) return;
+  if (ld_u64(first + (unsigned long long)l) > (unsigned long long)i) g_min(first + (unsigned long long)l, (unsigned long long)i);
+}
+
+// ---- the voids of many boxes at once (hole filling) -------------------------------------------------
+// The same union-find over several components' boxes side by side: one launch per step for all of
+// them, a block of kBoxTile voxels finding its box by its number. A component's voids depend on its
+// own voxels alone, and a component that another one painted over fills nothing, so every component's
+// voids can be found before any is filled; the filling then goes component by component in stream
+// order, with the painted-over marks on the device. Found and filled one by one, with a host read
+// each, the 200^3 volume's 40 components took 8.3 ms; 1.3 now.
+constexpr int kBoxTile = 2048;
+struct BoxTask {
+  Crop c;
+  FastDiv by_row, by_plane;
+  long long first_block, start;  // its first block, its first voxel in the shared arrays
+  long long id;
+};
+constexpr uint8_t kReached = 1, kVoid = 2;  // of a root: it reaches a face; of a voxel: in a void
+
+__device__ __forceinline__ int box_of(const BoxTask *tasks, int count) {
+  int lo = 0, hi = count;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (tasks[mid].first_block <= (long long)blockIdx.x) lo = mid;
+    else hi = mid;
+  }
+  return lo;
+}
+__device__ __forceinline__ void box_place(const BoxTask &t, int i, int &x, int &y, int &z) {
+  z = int(fast_quotient(unsigned(i), t.by_plane));
+  const int r = i - z * (t.c.ext[0] * t.c.ext[1]);
+  y = int(fast_quotient(unsigned(r), t.by_row));
+  x = r - y * t.c.ext[0];
+}
+// Calls f(task, box voxel or -1, x, y, z) for the block's voxels, 64 consecutive ones per wave and
+// step; every lane calls it.
+template <class F> __device__ __forceinline__ void for_box(const BoxTask *tasks, int count, F &&f) {
+  const int k = box_of(tasks, count);
+  const BoxTask t = tasks[k];
+  const long long n = t.c.size(), base = ((long long)blockIdx.x - t.first_block) * kBoxTile;
+  for (int j = 0; j < kBoxTile; j += kThreads) {
+    const long long i = base + j + threadIdx.x;
+    int x = 0, y = 0, z = 0;
+    if (i < n) box_place(t, int(i), x, y, z);
+    f(t, k, i < n ? int(i) : -1, x, y, z);
+  }
+}
+
+template <class CC> __global__ void __launch_bounds__(kThreads) boxes_runs(const CC *cc, Dims d, const BoxTask *tasks, int count, int *parent) {
+  for_box(tasks, count, [&](const BoxTask &t, int, int i, int x, int y, int z) {
+    const int lane = threadIdx.x & 63;
+    const bool valid = i >= 0;
+    auto open_here = [&](int xx) { return !is_label(cc, d, t.c, xx, y, z, CC(t.id)); };
+    const bool open = valid && open_here(x);
+    int prev = shfl_up_any(int(open), 1);
+    if (lane == 0 && valid && x > 0) prev = int(open_here(x - 1));
+    const unsigned long long mask = __ballot(open && (x == 0 || !prev));
+    if (!valid) return;
+    int *p = parent + t.start;
+    if (!open) { p[i] = kOut; return; }
+    const unsigned long long below = mask & lanes_upto(lane);
+    const int base = i - lane;
+    p[i] = below ? base + (63 - __clzll((long long)below)) : base - 1;  // base - 1: same run
+  });
+}
+
+// Contacts as in box_union.
+__global__ void __launch_bounds__(kThreads) boxes_union(const BoxTask *tasks, int count, int *parent) {
+  for_box(tasks, count, [&](const BoxTask &t, int, int i, int x, int y, int z) {
+    int *p = parent + t.start;
+    if (i < 0 || ld_i(p + i) == kOut) return;
+    const int ex = t.c.ext[0], ey = t.c.ext[1];
+    const bool first = x == 0 || ld_i(p + i - 1) == kOut;
+    const int rows[2] = {y > 0 ? i - ex : -1, z > 0 ? i - ex * ey : -1};
+    for (int r = 0; r < 2; ++r) {
+      const int j = rows[r];
+      if (j < 0 || ld_i(p + j) == kOut) continue;
+      if (first || ld_i(p + j - 1) == kOut) box_unite(p, i, j);  // x > 0 when !first
+    }
+  });
+}
+
+__global__ void __launch_bounds__(kThreads) boxes_mark(const BoxTask *tasks, int count, int *parent, uint8_t *state) {
+  for_box(tasks, count, [&](const BoxTask &t, int, int i, int x, int y, int z) {
+    int *p = parent + t.start;
+    if (i < 0 || ld_i(p + i) == kOut) return;
+    const bool face = x == 0 || y == 0 || z == 0 || x == t.c.ext[0] - 1 || y == t.c.ext[1] - 1 || z == t.c.ext[2] - 1;
+    if (face) g_st(state + t.start + box_root(p, i), kReached);
+  });
+}
+
+__global__ void __launch_bounds__(kThreads) boxes_voids(const BoxTask *tasks, int count, int *parent, uint8_t *state,
+                                                        unsigned long long *voids) {
+  for_box(tasks, count, [&](const BoxTask &t, int k, int i, int, int, int) {
+    int *p = parent + t.start;
+    bool hole = false;
+    if (i >= 0 && ld_i(p + i) != kOut) {
+      hole = !(ld_u8(state + t.start + box_root(p, i)) & kReached);
+      if (hole) g_st(state + t.start + i, kVoid);  // an unreached root's own byte: its kReached stays clear
+    }
+    const int n = __popcll(__ballot(hole));
+    if ((threadIdx.x & 63) == 0 && n) g_add(voids + k, (unsigned long long)n);
+  });
+}
+
+// Task k's voids become its id, their owners painted over; nothing when it was painted over itself.
+template <class CC>
+__global__ void __launch_bounds__(kThreads) box_fill(CC *cc, Dims d, const BoxTask *tasks, int k, const uint8_t *state,
+                                                     uint8_t *painted_over, unsigned long long *filled) {
+  const BoxTask t = tasks[k];
+  if (painted_over[t.id]) return;
+  const long long n = t.c.size();
+  const long long i = (long long)blockIdx.x * kThreads + threadIdx.x;
+  const bool hole = i < n && state[t.start + i] == kVoid;
+  if (hole) {
+    int x, y, z;
+    box_place(t, int(i), x, y, z);
+    CC *at = cc + (t.c.lo[0] + x) + (long long)d.sx * ((t.c.lo[1] + y) + (long long)d.sy * (t.c.lo[2] + z));
+    const CC owner = *at;
+    if (owner != CC(0)) painted_over[owner] = 1;
+    *at = CC(t.id);
+  }
+  const int m = __popcll(__ballot(hole));
+  if ((threadIdx.x & 63) == 0 && m) g_add(filled, (unsigned long long)m);
+}
+
+template <class CC>
+int64_t fill_boxes(Context &ctx, CC *cc, Dims d, const std::vector<Box> &boxes, const std::vector<int64_t> &ids) {
+  auto s = ctx.stream();
+  Buffer<uint8_t> painted_over(ctx, boxes.size());
+  painted_over.clear(ctx);
+  Buffer<unsigned long long> filled(ctx, 1);
+  filled.clear(ctx);
+  // Boxes in groups of up to the volume's own size (at least one box), 5 bytes per voxel: less than
+  // the fields that the call allocates for the volume next.
+  const long long group = std::min((long long)d.sx * d.sy * d.sz, 1LL << 28);
+  for (size_t at = 0; at < ids.size();) {
+    std::vector<BoxTask> tasks;
+    long long voxels = 0, blocks = 0;
+    while (at < ids.size()) {
+      const Box &b = boxes[size_t(ids[at])];
+      BoxTask t;
+      for (int a = 0; a < 3; ++a) {
+        t.c.lo[a] = b.lo[a];
+        t.c.ext[a] = b.hi[a] - b.lo[a] + 1;
+      }
+      const long long n = t.c.size();
+      if (n > INT32_MAX) throw std::invalid_argument("label bounding box exceeds int32 capacity");
+      if (!tasks.empty() && voxels + n > group) break;
+      t.by_row = fast_div(unsigned(t.c.ext[0]));
+      t.by_plane = fast_div(unsigned(t.c.ext[0]) * unsigned(t.c.ext[1]));
+      t.first_block = blocks;
+      t.start = voxels;
+      t.id = ids[at];
+      tasks.push_back(t);
+      voxels += n;
+      blocks += (n + kBoxTile - 1) / kBoxTile;
+      ++at;
+    }
+    const int count = int(tasks.size());
+    Buffer<BoxTask> tasks_dev(ctx, tasks.size());
+    tasks_dev.upload(ctx, tasks.data(), tasks.size());
+    Buffer<int> parent(ctx, size_t(voxels));
+    Buffer<uint8_t> state(ctx, size_t(voxels));
+    Buffer<unsigned long long> voids(ctx, tasks.size());
+    state.clear(ctx);
+    voids.clear(ctx);
+    const unsigned grid = unsigned(blocks);
+    boxes_runs<CC><<<grid, kThreads, 0, s>>>(cc, d, tasks_dev.data(), count, parent.data());
+    boxes_union<<<grid, kThreads, 0, s>>>(tasks_dev.data(), count, parent.data());
+    boxes_mark<<<grid, kThreads, 0, s>>>(tasks_dev.data(), count, parent.data(), state.data());
+    boxes_voids<<<grid, kThreads, 0, s>>>(tasks_dev.data(), count, parent.data(), state.data(), voids.data());
+    BROOK_LAUNCHED();
+    const std::vector<unsigned long long> found = voids.download(ctx);
+    for (int k = 0; k < count; ++k)
+      if (found[size_t(k)])
+        box_fill<CC><<<blocks_for(tasks[size_t(k)].c.size()), kThreads, 0, s>>>(cc, d, tasks_dev.data(), k, state.data(),
+                                                                              painted_over.data(), filled.data());
+    BROOK_LAUNCHED();
+  }
+  return int64_t(filled.download(ctx)[0]);
 }
 
 template <class CC> struct AtMaximum {
@@ -254,6 +438,13 @@ std::vector<Maximum> maxima_of(Context &ctx, const CC *cc, long long n, const fl
 }
 
 }  // namespace
+
+int64_t fill_voids(Context &ctx, void *cc, int cc_bytes, Dims d, const std::vector<Box> &boxes, const std::vector<int64_t> &ids) {
+  if (ids.empty()) return 0;
+  if (cc_bytes == 1) return fill_boxes(ctx, static_cast<uint8_t *>(cc), d, boxes, ids);
+  if (cc_bytes == 2) return fill_boxes(ctx, static_cast<uint16_t *>(cc), d, boxes, ids);
+  return fill_boxes(ctx, static_cast<uint32_t *>(cc), d, boxes, ids);
+}
 
 int64_t enclosed_voids(Context &ctx, const void *cc, int cc_bytes, Dims d, int64_t id, const Box &box) {
   Crop c;

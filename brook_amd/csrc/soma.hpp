@@ -45,6 +45,11 @@ class VoidFill {
   Buffer<uint8_t> mask_;  // per box voxel: 1 = id or void
 };
 
+// In the order of `ids`, the voids of each id's box (`boxes`, per id) become the id; an id some of
+// whose voxels were painted over so fills nothing. Returns the voxels painted.
+int64_t fill_voids(Context &ctx, void *cc, int cc_bytes, Dims d, const std::vector<Box> &boxes,
+                   const std::vector<int64_t> &ids);
+
 // Per id (count + 1 entries): its smallest flat index (-1: no voxel).
 std::vector<int64_t> first_voxels(Context &ctx, const void *cc, int cc_bytes, long long n, int64_t count);
 
