@@ -3,10 +3,10 @@
 // table, y/z lower envelopes with float64 intersections, sqrtf at the end.
 //
 // Layout for HBM: the x pass gives each row to one wave (64 consecutive voxels per load, run
-// boundaries from two ballots, no atomics); the y and z passes first list the label runs of every
-// line (one thread per line, coalesced across neighbouring x) and then give each run its own
-// thread. Background runs are never evaluated (their values are discarded by the finish rule) and
-// the last pass fuses sqrt, the background zero and the per-label maximum.
+// boundaries from two ballots, no atomics); the y and z passes take whole lines into LDS, a block a
+// stretch of neighbouring ones, and halve for each voxel's nearest vertex. Background runs are never
+// evaluated (their values are discarded by the finish rule) and the last pass fuses sqrt, the
+// background zero and the per-label maximum.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -95,7 +95,7 @@ __global__ void __launch_bounds__(256) edt_x_serial(const CC *cc, int sx, int ro
   }
 }
 
-// Lower envelopes along y (axis 1) or z (axis 2), run-parallel. A run is a maximal stretch of one
+// Lower envelopes along y (axis 1) or z (axis 2) for lines too long for LDS, run-parallel. A run is a maximal stretch of one
 // nonzero id along a line; runs are independent (the walls at their ends stand for the
 // neighbouring id or the border), so each run gets its own thread and no wave waits on another
 // line's runs.
@@ -256,6 +256,329 @@ __global__ void __launch_bounds__(kRunBlock) edt_run_fh(const CC *cc, Dims dm, i
   }
 }
 
+// Lower envelopes along y (axis 1) or z (axis 2) in LDS: a block takes XT neighbouring lines whole,
+// its lane l = thread % XT their l-th, and finds for every voxel the nearest vertex of its run (the
+// position whose height plus squared distance is least, the walls at the run's ends being vertices of
+// height 0) by halving: nearest vertices move monotonically along a run, so a row's vertex lies between
+// those of the rows around it. Rows at multiples of 16 search outward until the distance alone is too far;
+// rows halfway between known ones search between the two vertices, at steps 8 and 4; the
+// four rows from each of those then share one pass over the candidates up to the next: some ten
+// candidates per voxel whatever the distances are.
+// The envelope of the long-line path gives the same values: w2 has a float's 24 bits and a distance
+// at most 12, so w2 * dq * dq is exact in float64 (and the fused sums below round once, as its
+// separate ones do), the least of the sums is the envelope's value, and candidates that tie give the
+// same bits.
+// LDS per line and position: 4 bytes of height, a start and a foreground bit, and a 16-bit vertex for
+// every fourth row. Four blocks to a compute unit (kLineLds and the registers allow that), so that
+// some load while others search. Every voxel is read once and written once, rows of XT at a time; a
+// thread per run instead (runs in line order, each lane at its own row, an intersection's division or
+// two per step) took 2 x (1.08 + 0.20) ms for 450 x 387 x 256 16-bit cells; y 0.44 and z 0.27 now, bound by
+// instructions (some 300 per row of a wave, half of them in float64). A solid 512^3 volume with a black
+// border: 26.8 -> 5.1 ms. Searching outward from every 64th row and halving from 32 is 4 % slower on cells.
+constexpr int kLineThreads = 256, kSeed = 16;
+constexpr size_t kLineLds = 40 << 10, kLineLdsMost = 156 << 10;
+constexpr int kWall = 1 << 15;
+
+constexpr size_t line_bytes(int xt, long long n) {
+  return size_t(xt) * (size_t(n + 4) * 4 + size_t((n >> 5) + 2) * 8 + size_t((n >> 2) + 2) * 2);
+}
+
+// The smaller of two numbers (fmin would first canonicalise what the loop carries).
+__device__ __forceinline__ double least(double a, double b) {
+  double r;
+  asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
+// A block's lines: heights, start and foreground bits, vertices; l is the lane's line of the XT.
+// A vertex is its position + 1, from 0 for the wall before row 0 to n + 1 for the one after the last;
+// a vertex code has kWall too for a wall.
+template <int XT> struct Line {
+  float *h;  // by vertex, and one more that a loop may load ahead
+  unsigned *start, *fg, *finite;  // finite: whether any height of the line is
+  uint16_t *near;
+  int l, n;
+  double w2;
+  float per_w;  // about 1 / w
+  bool bb;
+
+  __device__ __forceinline__ unsigned start_word(int k) const { return start[k * XT + l]; }
+  __device__ __forceinline__ bool foreground(int q) const { return fg[(q >> 5) * XT + l] >> (q & 31) & 1; }
+
+  // The starts at q, q-1, ... (bit 63 first, 32 valid bits) and at q+1, q+2, ... (bit 0 first, 32).
+  __device__ __forceinline__ unsigned long long starts_down(int q) const {
+    const int k = q >> 5;
+    const unsigned long long v = (unsigned long long)start_word(k) << 32 | (k ? start_word(k - 1) : 0u);
+    return v << (31 - (q & 31));
+  }
+  __device__ __forceinline__ unsigned long long starts_up(int q) const {
+    const int k = q >> 5;
+    const unsigned long long v = (unsigned long long)start_word(k + 1) << 32 | start_word(k);
+    return v >> (q & 31) >> 1;
+  }
+  // The codes of the first and last vertex of run [c, d]: its walls, or its ends where the volume's
+  // border is none.
+  __device__ __forceinline__ int first_code(int c) const { return c > 0 || bb ? c | kWall : c + 1; }
+  __device__ __forceinline__ int last_code(int d) const { return d + 1 < n || bb ? (d + 2) | kWall : d + 1; }
+
+  // The vertices between two codes of a run, in either order.
+  struct Range {
+    int lo, hi, first, last;  // vertices; the first and last that are no walls
+  };
+  __device__ __forceinline__ Range range(int a, int b) const {
+    const int x = min(a & (kWall - 1), b & (kWall - 1)), y = max(a & (kWall - 1), b & (kWall - 1));
+    const bool wx = (x == (a & (kWall - 1)) ? a : b) & kWall, wy = (y == (b & (kWall - 1)) ? b : a) & kWall;
+    return Range{x, y, x + int(wx), y - int(wy)};
+  }
+  __device__ __forceinline__ float stored(int v) const { return h[v * XT + l]; }
+  // Vertex v's height from what is stored at its place.
+  __device__ __forceinline__ static double height(float value, int v, const Range &r) {
+    return double(v < r.first || v > r.last ? 0.0f : value);
+  }
+  __device__ __forceinline__ double cost(int q, int code) const {
+    const int v = code & (kWall - 1);
+    const double dq = double(q + 1 - v);
+    return __builtin_fma(w2 * dq, dq, code & kWall ? 0.0 : double(h[v * XT + l]));
+  }
+
+  // The code of row q's best vertex between codes a and b.
+  __device__ __forceinline__ int between(int q, int a, int b) const {
+    const Range r = range(a, b);
+    double dq = double(q + 1 - r.lo);
+    double best = __builtin_fma(w2 * dq, dq, height(stored(r.lo), r.lo, r));
+    int vertex = r.lo, v = r.lo + 1, hi = r.hi;
+    if (hi - v > 6) {  // none beyond the distance that alone costs as much
+      const int reach = int(fminf(__builtin_amdgcn_sqrtf(float(best)) * per_w * 1.0001f + 2.0f, float(n)));
+      hi = min(hi, q + 1 + reach);
+      v = max(v, q + 1 - reach);
+      dq = double(q + 2 - v);
+    }
+    float value = stored(min(v, hi));
+    for (; v <= hi; ++v) {
+      const float next = stored(v + 1);
+      dq -= 1.0;
+      const double c = __builtin_fma(w2 * dq, dq, height(value, v, r));
+      if (c < best) {
+        best = c;
+        vertex = v;
+      }
+      value = next;
+    }
+    return vertex < r.first || vertex > r.last ? vertex | kWall : vertex;
+  }
+
+  // The code of row q's best vertex in run [c, d], outward until the distance alone costs more.
+  __device__ __forceinline__ int outward(int q, int c, int d) const {
+    const Range r = range(first_code(c), last_code(d));
+    int vertex = q + 1;
+    double best = double(h[vertex * XT + l]), dr = 1.0;
+    const int left = vertex - r.lo, right = r.hi - vertex, most = max(left, right);
+    float below = stored(max(q, 0)), above = stored(min(q + 2, n + 1));
+    for (int i = 1; i <= most; ++i, dr += 1.0) {
+      const double t = w2 * dr * dr;
+      if (t >= best) break;
+      const int x = q + 1 - i, y = q + 1 + i;
+      const float next_below = stored(max(x - 1, 0)), next_above = stored(min(y + 1, n + 1));
+      const double cx = t + height(below, x, r), cy = t + height(above, y, r);
+      if (i <= left && cx < best) {
+        best = cx;
+        vertex = x;
+      }
+      if (i <= right && cy < best) {
+        best = cy;
+        vertex = y;
+      }
+      below = next_below;
+      above = next_above;
+    }
+    return vertex < r.first || vertex > r.last ? vertex | kWall : vertex;
+  }
+};
+
+template <class CC, int XT>
+__global__ void __launch_bounds__(kLineThreads, 4) edt_lines(const CC *cc, Dims dm, int axis, float w, int bb, int nlines, int tiles,
+                                                             int finish, float *D, unsigned *label_max) {
+  extern __shared__ float edt_lds[];
+  constexpr int kRows = kLineThreads / XT;  // rows, words or groups of rows that the block takes at a time
+  // neighbouring tiles to one XCD: they share the cache lines at their edges
+  const int per = (tiles + 7) >> 3, tile = int(blockIdx.x & 7) * per + int(blockIdx.x >> 3);
+  if (tile >= tiles) return;  // whole block
+  const int l = threadIdx.x % XT, row = threadIdx.x / XT, t = tile * XT + l;
+  const LineGeom g = line_geom(dm, axis, t < nlines ? t : 0);
+  const int n = g.n, words = (n >> 5) + 2;
+  Line<XT> a;
+  a.h = edt_lds;
+  a.start = reinterpret_cast<unsigned *>(edt_lds + XT * (n + 3));
+  a.fg = a.start + XT * words;
+  a.finite = a.fg + XT * words;
+  a.near = reinterpret_cast<uint16_t *>(a.finite + XT);
+  a.l = l;
+  a.n = n;
+  a.w2 = double(w * w);
+  a.per_w = 1.0f / w;
+  a.bb = bb != 0;
+
+  if (row == 0) a.finite[l] = 0;
+  unsigned any = 0;
+  for (int k = row; k < words; k += kRows) {
+    unsigned start = 0, fg = 0;
+    if (t < nlines && k * 32 < n) {
+      const CC *at = cc + g.base + (long long)(k * 32) * g.stride;
+      CC prev = k ? at[-g.stride] : CC(0);
+#pragma unroll 1
+      for (int j0 = 0; j0 < 32; j0 += 16) {
+        CC lab[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) lab[j] = k * 32 + j0 + j < n ? at[(j0 + j) * g.stride] : CC(0);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          start |= unsigned(lab[j] != prev) << (j0 + j);
+          fg |= unsigned(lab[j] != CC(0)) << (j0 + j);
+          prev = lab[j];
+        }
+      }
+    }
+    if (k == 0) start |= 1u;                   // row 0
+    if (k == n >> 5) start |= 1u << (n & 31);  // the end of the last run
+    a.start[k * XT + l] = start;
+    a.fg[k * XT + l] = fg;
+    any |= fg;
+  }
+  const bool some = __syncthreads_or(int(any != 0));
+  if (!some) {
+    if (finish && t < nlines)
+      for (int q = row; q < n; q += kRows) D[g.base + q * g.stride] = 0.0f;
+    return;
+  }
+  constexpr int kLoads = 8;
+  bool finite = false;
+  for (int q0 = row; q0 < n; q0 += kLoads * kRows) {
+    float value[kLoads];
+    unsigned fg = 0;
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j) {
+      const int q = q0 + j * kRows;
+      const bool f = q < n && a.foreground(q);
+      fg |= unsigned(f) << j;
+      value[j] = D[g.base + (f ? q : 0) * g.stride];  // the line's first row stands in for one not needed
+    }
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j) {
+      const int q = q0 + j * kRows;
+      if (fg >> j & 1) {
+        a.h[(q + 1) * XT + l] = value[j];
+        finite |= value[j] < kInf;
+      }
+      if (finish && !(fg >> j & 1) && q < n && t < nlines) D[g.base + q * g.stride] = 0.0f;
+    }
+  }
+  if (finite) a.finite[l] = 1;
+  __syncthreads();
+  for (int q = row * kSeed; q < n; q += kRows * kSeed) {
+    if (!a.foreground(q)) continue;
+    int k = q >> 5;
+    unsigned v = a.start_word(k) & ((2u << (q & 31)) - 1u);
+    while (!v) v = a.start_word(--k);  // row 0 has one
+    const int c = k * 32 + 31 - __clz(int(v));
+    k = q >> 5;
+    v = a.start_word(k) & ~((2u << (q & 31)) - 1u);
+    while (!v) v = a.start_word(++k);  // n has one
+    const int d = k * 32 + __ffs(int(v)) - 2;
+    // a whole line without walls and heights has nothing to search for
+    const bool none = c == 0 && d == n - 1 && !bb && !a.finite[l];
+    a.near[(q >> 2) * XT + l] = uint16_t(none ? q + 1 : a.outward(q, c, d));
+  }
+  for (int s = kSeed / 2; s >= 4; s >>= 1) {
+    __syncthreads();
+    for (int q = s + row * 2 * s; q < n; q += kRows * 2 * s) {
+      if (!a.foreground(q)) continue;
+      // the vertices of rows q - s and q + s where the run has those, else its first and last
+      const unsigned long long down = a.starts_down(q) >> (64 - s) << (64 - s), up = a.starts_up(q) & ((1ULL << s) - 1ULL);
+      const int before = down ? a.first_code(q - __clzll((long long)down)) : int(a.near[((q - s) >> 2) * XT + l]);
+      const int after = up ? a.last_code(q + __ffsll((long long)up) - 1) : int(a.near[((q + s) >> 2) * XT + l]);
+      a.near[(q >> 2) * XT + l] = uint16_t(a.between(q, before, after));
+    }
+  }
+  __syncthreads();
+  for (int q0 = 4 * row; q0 < n; q0 += 4 * kRows) {
+    const unsigned fg = a.fg[(q0 >> 5) * XT + l] >> (q0 & 31) & 15u;
+    if (!fg) continue;
+    const unsigned starts = unsigned(a.starts_up(q0)) & 15u;  // at q0 + 1 .. q0 + 4
+    const int v0 = a.near[(q0 >> 2) * XT + l], v4 = a.near[((q0 + 4) >> 2) * XT + l];
+    double best[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int j0 = 0; j0 < 4;) {  // the runs among the four rows, rows j0 to j1 of each
+      const unsigned ends = starts >> j0;
+      const int j1 = ends ? j0 + __ffs(int(ends)) - 1 : 3;
+      if (fg >> j0 & 1) {
+        const auto r = a.range(j0 ? a.first_code(q0 + j0) : v0, ends ? a.last_code(q0 + j1) : v4);
+        double m[4] = {HUGE_VAL, HUGE_VAL, HUGE_VAL, HUGE_VAL}, dq = double(q0 + 1 - r.lo);
+        float stored = a.stored(r.lo);
+        for (int v = r.lo; v <= r.hi; ++v) {
+          const float next = a.stored(v + 1);
+          const double h = a.height(stored, v, r);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const double x = dq + double(j);
+            m[j] = least(m[j], __builtin_fma(a.w2 * x, x, h));
+          }
+          dq -= 1.0;
+          stored = next;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (j >= j0 && j <= j1) best[j] = m[j];
+      }
+      j0 = j1 + 1;
+    }
+    float *out = D + g.base + q0 * g.stride;
+    float value[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      value[j] = float(best[j]);
+      if (finish) value[j] = sqrtf(value[j]);
+      if (fg >> j & 1) out[j * g.stride] = value[j];
+    }
+    if (!finish || !label_max) continue;
+    // Each run's largest value among these rows goes to its label's maximum, unless the run goes on to
+    // a row q0 + 4 as large or came from a larger row q0 - 4: the groups that hold a run's maximum
+    // include a last one, which neither rule leaves out.
+    float top = 0.0f;
+    bool open = q0 && !(a.starts_down(q0) >> 60);  // the first run is that of q0 - 4
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      top = fmaxf(top, value[j]);
+      const bool ends = starts >> j & 1;
+      if ((ends || j == 3) && (fg >> j & 1) && top < kInf) {
+        bool tell = true;
+        if (!ends) tell = sqrtf(float(a.cost(q0 + 4, v4))) < top;
+        if (open && tell) tell = sqrtf(float(a.cost(q0 - 4, a.near[((q0 - 4) >> 2) * XT + l]))) <= top;
+        if (tell) {
+          unsigned *slot = label_max + (unsigned long long)cc[g.base + (q0 + j) * g.stride];
+          const unsigned bits = __float_as_uint(top);
+          if (ld_u(slot) < bits) atomicMax(slot, bits);
+        }
+      }
+      if (ends) {
+        top = 0.0f;
+        open = false;
+      }
+    }
+  }
+}
+
+template <class CC, int XT>
+void run_lines(Context &ctx, const CC *cc, Dims dm, int axis, float w, bool bb, int nlines, int n, bool finish, float *out,
+               unsigned *label_max) {
+  const size_t lds = line_bytes(XT, n);
+  if (lds > (64 << 10))
+    BROOK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(edt_lines<CC, XT>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  int(kLineLdsMost)));
+  const int tiles = (nlines + XT - 1) / XT;
+  edt_lines<CC, XT><<<unsigned((tiles + 7) / 8 * 8), kLineThreads, lds, ctx.stream()>>>(cc, dm, axis, w, bb, nlines, tiles, finish,
+                                                                                       out, label_max);
+  BROOK_LAUNCHED();
+}
+
 // finish for a single pass (x only): background 0, else sqrt.
 template <class CC>
 __global__ void __launch_bounds__(256) edt_finish(const CC *cc, long long n, float *D, unsigned *label_max) {
@@ -299,7 +622,19 @@ void run_edt(Context &ctx, const CC *cc, Dims dm, const float aniso[3], bool bb,
   for (int axis = 1; axis <= last; ++axis) {
     const int nlines = axis == 1 ? dm.sx * dm.sz : dm.sx * dm.sy;
     const unsigned lgrid = unsigned((nlines + 255) / 256);
-    const char *timer = axis == 1 ? "edt_y" : "edt_z";  // two scopes: the host read between them is not timed
+    const char *timer = axis == 1 ? "edt_y" : "edt_z";
+    const int n = axis == 1 ? dm.sy : dm.sz;
+    const float w = aniso[axis];
+    // As many lines to a block as leave room for a second one, down to the 8 whose rows still fill
+    // 32-byte sectors; lines beyond 160 KB of those take the run lists.
+    if (line_bytes(8, n) <= kLineLdsMost) {
+      KernelTimer line_timer(ctx, timer);
+      if (line_bytes(32, n) <= kLineLds) run_lines<CC, 32>(ctx, cc, dm, axis, w, bb, nlines, n, axis == last, out, label_max);
+      else if (line_bytes(16, n) <= kLineLds) run_lines<CC, 16>(ctx, cc, dm, axis, w, bb, nlines, n, axis == last, out, label_max);
+      else run_lines<CC, 8>(ctx, cc, dm, axis, w, bb, nlines, n, axis == last, out, label_max);
+      continue;
+    }
+    // (two timer scopes below: the host read between them is not timed)
     Buffer<int> line_runs(ctx, size_t(nlines)), run_at(ctx, size_t(nlines));
     Buffer<long long> line_spill(ctx, size_t(nlines)), spill_at(ctx, size_t(nlines));
     {
