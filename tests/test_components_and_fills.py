@@ -1,5 +1,6 @@
 """The component unions' left-out contacts against the oracle on random volumes (every density, rows
-and planes of one voxel, the remainders of a wave), and hole filling over more than one group of
+and planes of one voxel, the remainders of a wave,
+more than one stretch per wave), and hole filling over more than one group of
 boxes against the volume filled beforehand."""
 import numpy as np
 import pytest
@@ -18,7 +19,7 @@ def torch():
 
 
 @pytest.mark.parametrize("shape", [(1, 1, 1), (1, 9, 7), (9, 1, 7), (9, 7, 1), (63, 5, 6), (64, 4, 9), (65, 7, 5), (33, 31, 29),
-                                   (130, 20, 17)])
+                                   (130, 20, 17), (101, 103, 107)])
 @pytest.mark.parametrize("labels,density", [(1, 0.08), (1, 0.3), (2, 0.55), (3, 0.9), (2, 1.0)])
 def test_components_of_random_volumes(torch, shape, labels, density):
     from brook_amd import device
