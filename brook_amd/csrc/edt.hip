@@ -419,7 +419,7 @@ __global__ void __launch_bounds__(kLineThreads, 4) edt_lines(const CC *cc, Dims 
   a.bb = bb != 0;
 
   if (row == 0) a.finite[l] = 0;
-  unsigned any = 0;
+  unsigned any = 0, inner = 0;  // foreground; starts within the line
   for (int k = row; k < words; k += kRows) {
     unsigned start = 0, fg = 0;
     if (t < nlines && k * 32 < n) {
@@ -438,6 +438,8 @@ __global__ void __launch_bounds__(kLineThreads, 4) edt_lines(const CC *cc, Dims 
         }
       }
     }
+    const int left = n - k * 32;
+    inner |= start & (left >= 32 ? ~0u : left > 0 ? (1u << left) - 1u : 0u) & (k == 0 ? ~1u : ~0u);
     if (k == 0) start |= 1u;                   // row 0
     if (k == n >> 5) start |= 1u << (n & 31);  // the end of the last run
     a.start[k * XT + l] = start;
@@ -473,7 +475,11 @@ __global__ void __launch_bounds__(kLineThreads, 4) edt_lines(const CC *cc, Dims 
     }
   }
   if (finite) a.finite[l] = 1;
-  __syncthreads();
+  if (!__syncthreads_or(int(finite || inner || bb))) {  // no wall and no height in the block's lines
+    for (int q = row; q < n; q += kRows)
+      if (a.foreground(q)) D[g.base + q * g.stride] = kInf;
+    return;
+  }
   for (int q = row * kSeed; q < n; q += kRows * kSeed) {
     if (!a.foreground(q)) continue;
     int k = q >> 5;

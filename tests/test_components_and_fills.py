@@ -1,7 +1,6 @@
 """The component unions' left-out contacts against the oracle on random volumes (every density, rows
-and planes of one voxel, the remainders of a wave,
-more than one stretch per wave), and hole filling over more than one group of
-boxes against the volume filled beforehand."""
+and planes of one voxel, the remainders of a wave, more than one stretch per wave), and hole filling
+over more than one group of boxes against the volume filled beforehand."""
 import numpy as np
 import pytest
 
