@@ -43,7 +43,7 @@ def _kernel_table(stats, n, b_in, b_cc, F):
         "ccl": (["ccl_init", "ccl_union", "ccl_count", "ccl_mark", "ccl_relabel"], (b_in + b_cc) * n),
         "edt": (["edt_x", "edt_y", "edt_z"], (3 * b_cc + 4 + 8 + 8) * n),
         "prepare_labels": (["prepare_labels"], 12 * flood),
-        "init_records": (["init_records"], (b_cc + 16) * n),
+        "init_words": (["init_words"], (b_cc + 4) * n + 8 * F),
         "pdrf_alive": (["pdrf_alive"], b_cc * n + (4 + 4 + 4 + 8) * F),
         "trace_labels": (["trace_labels"], 12 * reached + 13 * claimed),
     }
@@ -391,7 +391,7 @@ def main():
         run()
     native.check(native.lib().brook_context_set_kernel_timing(ctx.handle, 1))
     names = ["ccl_init", "ccl_union", "ccl_count", "ccl_mark", "ccl_relabel", "edt_x", "edt_y", "edt_z",
-             "init_records", "prepare_labels", "pdrf_alive", "trace_labels"]
+             "init_words", "prepare_labels", "pdrf_alive", "trace_labels"]
     stat_names = ["railroad_reached_voxels", "invalidated_voxels", "flood_voxels", "foreground_voxels", "cc_bytes",
                   "paths", "components", "prep_ccl_ms", "prep_analyze_ms", "prep_edt_ms", "prep_borders_ms",
                   "prep_floods_ms", "prep_pdrf_order_ms", "trace_ms", "assembly_ms"]
