@@ -51,8 +51,9 @@ using Front = SplitList<kLdsFront>;
 using Far = SplitList<kLdsFar>;
 
 // List lengths (Shared::n). Front lengths rotate over three counters: round r reads n[r], appends to
-// n[r+1] and clears n[r+2] (read in round r-1), so a round needs one barrier. The far (waiting)
-// lengths rotate likewise over kFar .. kFar + 2, a step per phase (band).
+// n[r+1] and clears n[r+2] (read in round r-1), so a round needs one barrier. Waves leave the rounds by
+// reading n[r] = 0, so a barrier comes before the next append to n[r] (a band's promotions). The far
+// (waiting) lengths rotate likewise over kFar .. kFar + 2, a step per phase (band).
 constexpr int kFar = 3, kTouched = 6, kStale = 7, kDirty = 8, kCounters = 9;
 
 // What a round found about the railroad's far list, in the rotation of the front lengths (a wave
@@ -802,6 +803,9 @@ __device__ __forceinline__ bool invalidate(const TraceArgs &a, const Ball &ball,
     if (nf == 0 || !converged || ++rounds > budget) { converged = converged && nf == 0; break; }
     if (threadIdx.x == 0) { sh.prof[12] += nf; sh.prof[13] += 1; }
     const int ns = sh.n[kStale];
+    // The promotion below appends to the counter that every wave left the rounds by reading as 0: none
+    // may append before all have read it (a wave that read an append would begin a round of its own).
+    __syncthreads();
     if (ns) pull_stale(a, ball, sh, ln, to.far, nf, ns, to, reinterpret_cast<int *>(l.snap));
     // The next band: the one that holds the least waiting offer (an offer replaced since leaves it
     // too low at worst: an empty band).
