@@ -298,8 +298,7 @@ template <int XT> struct Line {
   unsigned *start, *fg, *finite;  // finite: whether any height of the line is
   uint16_t *near;
   int l, n;
-  double w2;
-  float per_w;  // about 1 / w
+  double w2, per_w2;  // the squared step and its inverse
   bool bb;
 
   __device__ __forceinline__ unsigned start_word(int k) const { return start[k * XT + l]; }
@@ -347,8 +346,8 @@ template <int XT> struct Line {
     double dq = double(q + 1 - r.lo);
     double best = __builtin_fma(w2 * dq, dq, height(stored(r.lo), r.lo, r));
     int vertex = r.lo, v = r.lo + 1, hi = r.hi;
-    if (hi - v > 6) {  // none beyond the distance that alone costs as much
-      const int reach = int(fminf(__builtin_amdgcn_sqrtf(float(best)) * per_w * 1.0001f + 2.0f, float(n)));
+    if (hi - v > 6) {  // none beyond the distance that alone costs as much (in rows: a float of any step's size)
+      const int reach = int(fminf(__builtin_amdgcn_sqrtf(float(best * per_w2)) * 1.0001f + 2.0f, float(n)));
       hi = min(hi, q + 1 + reach);
       v = max(v, q + 1 - reach);
       dq = double(q + 2 - v);
@@ -415,7 +414,7 @@ __global__ void __launch_bounds__(kLineThreads, 4) edt_lines(const CC *cc, Dims 
   a.l = l;
   a.n = n;
   a.w2 = double(w * w);
-  a.per_w = 1.0f / w;
+  a.per_w2 = 1.0 / a.w2;
   a.bb = bb != 0;
 
   if (row == 0) a.finite[l] = 0;

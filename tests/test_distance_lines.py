@@ -42,6 +42,17 @@ def test_lines_equal_the_oracle(torch, shape, kind, aniso, border):
     assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("step", [1e18, 1e-18, 2e-20, 3e-21, 1e-22, 1e-23])
+@pytest.mark.parametrize("border", [True, False])
+def test_steps_at_the_ends_of_their_range(torch, step, border):
+    """Steps whose squares are huge, subnormal or 0 in 32 bits: the same bits as the oracle's."""
+    from brook_amd import device
+    vol = np.asfortranarray((np.random.default_rng(3).random((9, 80, 70)) < 0.8).astype(np.uint8))
+    aniso = (step, step, 1.5 * step)
+    got = device.edt(vol, aniso, border).cpu().numpy()
+    assert np.array_equal(got, oracle.edt(oracle.ccl(vol)[0], aniso, border))
+
+
 @pytest.mark.parametrize("shape", [(40, 37, 70), (64, 65, 5)])
 def test_label_maxima(torch, shape):
     """The transform's per-label maxima decide roots and scales: skeletons of blobs equal the oracle's."""
