@@ -630,11 +630,15 @@ void run_edt(Context &ctx, const CC *cc, Dims dm, const float aniso[3], bool bb,
     const char *timer = axis == 1 ? "edt_y" : "edt_z";
     const int n = axis == 1 ? dm.sy : dm.sz;
     const float w = aniso[axis];
-    // As many lines to a block as leave room for a second one, down to the 8 whose rows still fill
-    // 32-byte sectors; lines beyond 160 KB of those take the run lists.
+    // As many lines to a block as leave room for three others on the compute unit (kLineLds), down to the 8
+    // whose rows still fill 32-byte sectors: those have up to all of its LDS, and longer lines take the run
+    // lists. Lines of up to 27 positions go to a thread each, 256 to a block: with 32 lines most threads had no
+    // row (z of 9000 x 9000 x 1 8.67 ms, now 1.80, the run lists 2.93; of 4000 x 4000 x 4 1.96, 0.41, 1.02;
+    // of 2000 x 2000 x 27 1.01, 0.53, 1.14). 64 or 128 lines were slower up to 27 (4.34, 2.67 ms; 0.62, 0.53).
     if (line_bytes(8, n) <= kLineLdsMost) {
       KernelTimer line_timer(ctx, timer);
-      if (line_bytes(32, n) <= kLineLds) run_lines<CC, 32>(ctx, cc, dm, axis, w, bb, nlines, n, axis == last, out, label_max);
+      if (line_bytes(kLineThreads, n) <= kLineLds) run_lines<CC, kLineThreads>(ctx, cc, dm, axis, w, bb, nlines, n, axis == last, out, label_max);
+      else if (line_bytes(32, n) <= kLineLds) run_lines<CC, 32>(ctx, cc, dm, axis, w, bb, nlines, n, axis == last, out, label_max);
       else if (line_bytes(16, n) <= kLineLds) run_lines<CC, 16>(ctx, cc, dm, axis, w, bb, nlines, n, axis == last, out, label_max);
       else run_lines<CC, 8>(ctx, cc, dm, axis, w, bb, nlines, n, axis == last, out, label_max);
       continue;

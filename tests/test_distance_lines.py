@@ -1,5 +1,5 @@
 """The distance transform's line kernel against the oracle, bit for bit: line lengths at the edges of
-its words, seeds and groups, each number of lines per block and the run lists beyond them, few and
+its words, seeds and groups, each number of lines per block (256 up to 27 positions) and the run lists beyond them, few and
 many runs per line, lines without walls, and the per-label maxima through the skeleton's radii."""
 import numpy as np
 import pytest
@@ -30,7 +30,7 @@ def _volume(shape, kind, rng):
     return vol
 
 
-@pytest.mark.parametrize("shape", [(5, 1, 1), (3, 2, 5), (31, 33, 3), (40, 63, 64), (33, 65, 66), (20, 96, 31), (7, 128, 129),
+@pytest.mark.parametrize("shape", [(5, 1, 1), (3, 2, 5), (31, 33, 3), (300, 27, 1), (257, 28, 2), (19, 27, 28), (17, 16, 15), (40, 63, 64), (33, 65, 66), (20, 96, 31), (7, 128, 129),
                                    (9, 534, 5), (6, 5, 545), (4, 1067, 3), (3, 4, 1100), (2, 3300, 2), (2, 2, 4300)])
 @pytest.mark.parametrize("kind,aniso,border", [("solid", (1, 1, 1), True), ("solid", (3, 0.3, 7), False), ("noise", (4, 4, 40), False),
                                                ("boxes", (0.37, 1.1, 0.9), True), ("boxes", (16, 16, 40), False)])
