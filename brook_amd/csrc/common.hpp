@@ -196,7 +196,15 @@ constexpr unsigned long long kFloodFree = kUnreached | kCostBits;  // the floods
 
 constexpr unsigned long long kDead = 0ULL, kFree = ~0ULL;
 
-constexpr long long word_pad(const Dims &d) { return (long long)d.sx * d.sy + d.sx + 1; }
+// The place of a step (dx, dy, dz) of up to one voxel from the word it starts at. Along a dimension of
+// one voxel no mask bit leads anywhere and the step has no length, so that a flat volume needs no plane of
+// padding on each side (two arrays of three times its words).
+__host__ __device__ constexpr int step_offset(const Dims &d, int dx, int dy, int dz) {
+  return dx + (d.sy > 1 ? d.sx * dy : 0) + (d.sz > 1 ? d.sx * d.sy * dz : 0);
+}
+constexpr long long word_pad(const Dims &d) {
+  return (d.sz > 1 ? (long long)d.sx * d.sy : 0) + (d.sy > 1 ? d.sx : 0) + 1;  // the longest step
+}
 // Volumes whose padded words lie within 32-bit byte offsets: the kernels' narrow form, which adds a
 // 32-bit offset per lane to a scalar base instead of computing 64-bit addresses.
 constexpr bool narrow_words(const Dims &d) {

@@ -58,7 +58,7 @@ template <bool Wide> __device__ __forceinline__ Lane<Wide> lane_of(const Dims &d
   const bool nb = q.cnt > 0;
   l.k = nb ? kSlots.k[l.slot] : 0;
   const int dx = nb ? kNX[l.k] : 0, dy = nb ? kNY[l.k] : 0, dz = nb ? kNZ[l.k] : 0;
-  l.off = dx + d.sx * (dy + d.sy * dz);
+  l.off = step_offset(d, dx, dy, dz);
   l.bit = nb ? 1u << l.k : 0u;
   l.offb = typename Lane<Wide>::Off((l.off + word_pad(d)) * 8);
   l.dx = float(dx);

@@ -397,7 +397,7 @@ __device__ __forceinline__ void backtrace(const TraceArgs &a, Shared &sh, int t,
   if (threadIdx.x >= 64) return;
   const int lane = threadIdx.x;
   const bool on = lane < 26;
-  const int off = on ? nb_offset(on ? lane : 0, a.d) : 0;
+  const int off = on ? step_offset(a.d, kNX[lane], kNY[lane], kNZ[lane]) : 0;
   const unsigned rank = on ? unsigned(kD3Rank[on ? lane : 0]) : 64u;
   int cur = (int)(unsigned)(sh.rail_best & 0xFFFFFFFFULL);
   int kept = 0;

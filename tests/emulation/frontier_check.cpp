@@ -242,7 +242,9 @@ int main() {
                         {"soma", {17, 15, 11}, 0, false, false, true, false, 1.0f, 1.5f},
                         {"graph", {21, 18, 7}, 0, false, false, false, true, 1.2f, 1.0f},
                         {"tube", {250, 2, 2}, 1, false, false, false, false, 0.5f, 1.0f},
-                        {"sheet", {47, 41, 1}, 2, false, false, false, false, 2.0f, 3.0f}};
+                        {"sheet", {47, 41, 1}, 2, false, false, false, false, 2.0f, 3.0f},
+                        {"sheet on edge", {29, 1, 33}, 0, false, false, false, false, 1.0f, 2.0f},
+                        {"column", {1, 1, 90}, 2, true, false, false, false, 1.0f, 1.0f}};
   const int waves = trace_part::brook::kWaves;
   std::vector<emu::Schedule> schedules;
   for (int s = 0; s < std::min(waves, 2); ++s) {  // the first or the last wave ahead of the others

@@ -46,6 +46,20 @@ int main() {
     const long long words = (long long)d.sx * d.sy * d.sz + 2 * word_pad(d);
     if (narrow_words(d) != (words * 8 <= (1LL << 32))) { std::printf("narrow %d %d %d\n", d.sx, d.sy, d.sz); return 1; }
   }
+  // every step of a voxel inside the volume has its flat offset, and every step lies within the padding;
+  // a volume of one plane or row is not padded along it
+  for (Dims d : {Dims{1, 1, 1}, Dims{7, 1, 1}, Dims{1, 9, 1}, Dims{1, 1, 5}, Dims{6, 5, 1}, Dims{6, 1, 4}, Dims{1, 3, 4}, Dims{5, 4, 3}}) {
+    long long longest = 0;
+    for (int k = 0; k < 26; ++k) {
+      const int off = step_offset(d, kDX[k], kDY[k], kDZ[k]);
+      longest = off > longest ? off : longest;
+      if (-off > word_pad(d)) { std::printf("step %d beyond the padding\n", k); return 1; }
+      const bool stays = (d.sx > 1 || !kDX[k]) && (d.sy > 1 || !kDY[k]) && (d.sz > 1 || !kDZ[k]);  // some voxel has that neighbour
+      if (stays && off != kDX[k] + d.sx * (kDY[k] + d.sy * kDZ[k])) { std::printf("step %d of %d %d %d\n", k, d.sx, d.sy, d.sz); return 1; }
+    }
+    if (longest != word_pad(d)) { std::printf("padding %lld of %d %d %d\n", word_pad(d), d.sx, d.sy, d.sz); return 1; }
+  }
+  if (word_pad(Dims{4000, 4000, 1}) != 4001) { std::printf("a plane of padding\n"); return 1; }
   std::printf("ok\n");
   return 0;
 }
