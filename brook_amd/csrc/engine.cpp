@@ -133,9 +133,13 @@ class Sample {
     all.push_back(this);
     for (auto &a : arenas_) a->sample->collect(all);
   }
-  // Rough device bytes a sample holds from its preamble to its assembly (40 B per voxel, 56 B per
-  // foreground voxel at the usual 40% occupancy, plus slack).
-  static int64_t footprint(int64_t n) { return n * 40 + (n * 2 / 5) * 56 + (int64_t(64) << 20); }
+  // Rough device bytes a sample holds from its preamble to its assembly (44 B per voxel, 20 of them the
+  // masks, road and claim words; 56 B per foreground voxel at the usual 40% occupancy; the two word
+  // arrays' padding; slack).
+  static int64_t footprint(const Dims &d) {
+    const int64_t n = int64_t(d.sx) * d.sy * d.sz;
+    return n * 44 + (n * 2 / 5) * 56 + 4 * word_pad(d) * int64_t(sizeof(unsigned long long)) + (int64_t(64) << 20);
+  }
 
   void preamble(Lap &lap) {
     preamble_components(lap, 0, false);
@@ -1210,7 +1214,7 @@ std::vector<Packed> skeletonize_batch(Context &ctx, const std::vector<LabelVolum
     std::vector<std::unique_ptr<Sample>> group;
     int64_t bytes = 0;
     while (i < volumes.size()) {
-      const int64_t need = Sample::footprint(volumes[i].size());
+      const int64_t need = Sample::footprint(volumes[i].dims);
       if (!group.empty() && bytes + need > budget) break;
       group.push_back(std::make_unique<Sample>(ctx, volumes[i], o, nullptr));
       bytes += need;

@@ -28,18 +28,19 @@ from concurrent.futures import Future
 from ._intake import DEFAULT_TEASAR_PARAMS
 from ._packed import PackedSkeletons
 
-# Device bytes a request holds while the engine runs it: 40 per voxel, 56 per foreground voxel at
-# up to 40% occupancy, plus slack (the engine's own group sizing uses the same figures).
-_BYTES_PER_VOXEL = 40 + 0.4 * 56
+# Device bytes a request holds while the engine runs it: 44 per voxel, 56 per foreground voxel at
+# up to 40% occupancy, 32 per word of padding (two arrays of 8-byte words, padded on both sides by
+# the longest step to a neighbour), plus slack (the engine's own group sizing uses the same figures).
+_BYTES_PER_VOXEL = 44 + 0.4 * 56
+_BYTES_PER_PAD = 32
 _SLACK = 64 << 20
 
 
 def request_bytes(labels) -> int:
     """Device-memory budget a request is admitted against."""
-    n = 1
-    for s in labels.shape:
-        n *= int(s)
-    return int(n * (_BYTES_PER_VOXEL + labels.dtype.itemsize)) + _SLACK
+    sx, sy, sz = (*(int(s) for s in labels.shape), 1, 1, 1)[:3]
+    pad = (sx * sy if sz > 1 else 0) + (sx if sy > 1 else 0) + 1
+    return int(sx * sy * sz * (_BYTES_PER_VOXEL + labels.dtype.itemsize)) + pad * _BYTES_PER_PAD + _SLACK
 
 
 class Request:

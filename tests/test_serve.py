@@ -65,6 +65,18 @@ def test_budget_admission_is_fifo_and_never_starves_a_large_request():
     assert rec.batches[1:] == [[(8, 8, 8)] * 2, [(8, 8, 8)], [(32, 32, 32)], [(8, 8, 8)]]
 
 
+def test_request_bytes_count_the_padding_by_shape():
+    """Two arrays of 8-byte words have the longest step to a neighbour as padding on both sides: a plane
+    and a row, less along dimensions of one voxel."""
+    def over(shape, pad):  # what is not per voxel
+        n = shape[0] * shape[1] * shape[2]
+        return request_bytes(np.zeros(shape, np.uint8)) - 45 * n - int(0.4 * 56 * n) - 32 * pad
+    slack = over((1, 1, 1), 1)
+    for shape, pad in [((100, 100, 100), 10101), ((1000, 500, 2), 501001), ((1000, 1000, 1), 1001), ((1000, 1, 9), 1001),
+                       ((1, 1, 7), 2)]:
+        assert abs(over(shape, pad) - slack) <= 2, shape
+
+
 def test_max_batch_one_is_serial():
     rec = Recorder()
     rec.gate.clear()
