@@ -611,9 +611,10 @@ __device__ __forceinline__ void offer_minima(const TraceArgs &a, Shared &sh, Sta
 }
 
 // One invalidation round over nc entries: every snapshot before any offer. A wave's entries stay in
-// its registers (up to one per lane) for fronts of up to a workgroup; longer fronts keep their
-// snapshots in device memory. Fronts that fit one batch per wave load their neighbours' words before
-// the barrier.
+// its registers, a lane each, in fronts of up to kHeld per wave (whole batches, so that none reaches past
+// lane 63); longer fronts keep their snapshots in device memory. Fronts that fit one batch per wave load
+// their neighbours' words before the barrier.
+constexpr int kHeld = 64 / (2 * kMaxPairs) * (2 * kMaxPairs);
 template <bool Wide>
 __device__ __forceinline__ void offer_round(const TraceArgs &a, const Ball &ball, Shared &sh, const Lane<Wide> &ln,
                                             const Front &cur, int nc, const OfferLists &to, unsigned long long *snap,
@@ -649,7 +650,7 @@ __device__ __forceinline__ void offer_round(const TraceArgs &a, const Ball &ball
   constexpr int P = kMaxPairs;
   int u[P];
   unsigned long long w[P];
-  if (nc <= kBlock) {
+  if (nc <= kWaves * kHeld) {
     const int per = (nc + kWaves - 1) / kWaves, b = ln.wave * per, n = min(per, nc - b);
     Offer e;
     if (ln.lane < n) {

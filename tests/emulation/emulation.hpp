@@ -229,7 +229,7 @@ template <class T> T from_lane(T v, int lane, const char *file, int line) {
   if (lane < 0 || lane > 63) fail("a value from a lane above 63", here(), here());
   return from_bits<T>(s[lane]);
 }
-inline int permute(int byte, int v, const char *file, int line) { return from_lane(v, byte >> 2 & 63, file, line); }
+inline int permute(int byte, int v, const char *file, int line) { return from_lane(v, byte >> 2, file, line); }
 inline int uniform(int v, const char *file, int line) {
   const unsigned long long *s = exchange(to_bits(v), file, line);
   for (int l = 0; l < 64; ++l)
