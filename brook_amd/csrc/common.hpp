@@ -90,23 +90,14 @@ template <class T> __device__ __forceinline__ void g_st(T *p, same_t<T> v) { *gp
 template <class T> __device__ __forceinline__ T g_min(T *p, same_t<T> v) {
   return __hip_atomic_fetch_min(gp(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-template <class T> __device__ __forceinline__ T g_max(T *p, same_t<T> v) {
-  return __hip_atomic_fetch_max(gp(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 template <class T> __device__ __forceinline__ T g_add(T *p, same_t<T> v) {
   return __hip_atomic_fetch_add(gp(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <class T> __device__ __forceinline__ T g_sub(T *p, same_t<T> v) {
-  return __hip_atomic_fetch_sub(gp(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 template <class T> __device__ __forceinline__ T g_or(T *p, same_t<T> v) {
   return __hip_atomic_fetch_or(gp(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 template <class T> __device__ __forceinline__ T g_and(T *p, same_t<T> v) {
   return __hip_atomic_fetch_and(gp(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <class T> __device__ __forceinline__ T g_xchg(T *p, same_t<T> v) {
-  return __hip_atomic_exchange(gp(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 // Compare-and-swap; returns the previous value.
 template <class T> __device__ __forceinline__ T g_cas(T *p, same_t<T> expected, same_t<T> desired) {
@@ -117,7 +108,6 @@ template <class T> __device__ __forceinline__ T g_cas(T *p, same_t<T> expected, 
 
 // Loads of memory that other threads change inside the same kernel: relaxed, agent scope, so the
 // access is served by L2 (the CU's vector L1 may hold a stale line otherwise).
-__device__ __forceinline__ float ld_f(const float *p) { return __hip_atomic_load(gp(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ int ld_i(const int *p) { return __hip_atomic_load(gp(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ unsigned ld_u(const unsigned *p) { return __hip_atomic_load(gp(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ unsigned long long ld_u64(const unsigned long long *p) {
@@ -126,14 +116,7 @@ __device__ __forceinline__ unsigned long long ld_u64(const unsigned long long *p
 __device__ __forceinline__ unsigned char ld_u8(const unsigned char *p) {
   return __hip_atomic_load(gp(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ void st_f(float *p, float v) { __hip_atomic_store(gp(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ void st_i(int *p, int v) { __hip_atomic_store(gp(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-__device__ __forceinline__ void st_u8(unsigned char *p, unsigned char v) {
-  __hip_atomic_store(gp(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void st_u64(unsigned long long *p, unsigned long long v) {
-  __hip_atomic_store(gp(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 
 // Loads and stores of per-voxel data that, during one kernel, only the workgroup owning the voxel's
 // component label touches (floods, tracer): workgroup scope is all the memory model needs, and the
@@ -147,14 +130,6 @@ __device__ __forceinline__ unsigned long long lp_u64(const unsigned long long *p
 }
 __device__ __forceinline__ void sp_u64(unsigned long long *p, unsigned long long v) {
   __hip_atomic_store(gp(p), v, __ATOMIC_RELAXED, BROOK_LABEL_SCOPE);
-}
-
-// atomicMin of a non-negative float through its int bits (monotone for floats >= 0, +inf included);
-// returns the previous value. A relaxed pre-check skips the atomic when it cannot improve.
-__device__ __forceinline__ float atomic_min_pos(float *addr, float val) {
-  float cur = ld_f(addr);
-  if (cur <= val) return cur;
-  return __int_as_float(g_min(reinterpret_cast<int *>(addr), __float_as_int(val)));
 }
 
 // Slot in a list whose length lives at *counter (any address space), for every lane that calls
@@ -238,31 +213,6 @@ __host__ __device__ __forceinline__ unsigned fast_quotient(unsigned n, const Fas
 template <class T> __device__ __forceinline__ T shfl_up_any(T v, unsigned delta) {
   if constexpr (sizeof(T) == 8) return T(__shfl_up((unsigned long long)v, delta, 64));
   else return T(__shfl_up((unsigned)v, delta, 64));
-}
-
-// A group of lanes per front entry: each of n entries gets G lanes of the workgroup (the largest power
-// of two up to 32 that fits every entry, at least 4); lane g of a group handles neighbours
-// [g*S, g*S + S), S = ceil(26 / G) <= kSpan. The frontier kernels use the layout of block / 32
-// entries: half a wave per entry, a neighbour per lane (front.hpp).
-constexpr int kSpan = 7;
-struct Group {
-  int G, i, g, lead, kb, cnt;  // lanes per entry, entry, lane in group, group's first lane, span
-};
-// The group of thread `tid` for n entries in a workgroup of `block` threads (host-callable, so the CPU
-// tests check the layout for every n, block and thread).
-__host__ __device__ constexpr Group group_at(int n, int block, int tid) {
-  Group q{};
-  q.G = 32;
-  while (q.G > 4 && n * q.G > block) q.G >>= 1;
-  int shift = 0;
-  while ((1 << shift) < q.G) ++shift;
-  const int span = (26 + q.G - 1) / q.G;
-  q.i = tid >> shift;
-  q.g = tid & (q.G - 1);
-  q.lead = (tid & 63) & ~(q.G - 1);  // lane of the group's first thread in its wave
-  q.kb = q.g * span;
-  q.cnt = span < 26 - q.kb ? span : 26 - q.kb;  // may be <= 0: nothing to do
-  return q;
 }
 
 // Mask of lanes 0..lane.

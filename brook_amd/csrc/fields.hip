@@ -401,7 +401,7 @@ __global__ void __launch_bounds__(kFloodBlock) prepare_labels(const FloodJob *__
     const Dims d = job.d;
     const LabelTables &t = job.t;
     if (threadIdx.x < 26) W[threadIdx.x] = g_ld(t.weights + threadIdx.x);
-    const Lane<Wide> ln = lane_of<Wide>(d, kFloodBlock);
+    const Lane<Wide> ln = lane_of<Wide>(d);
     __syncthreads();
     const int s0 = __builtin_amdgcn_readfirstlane(g_ld(t.seg_start + L));  // uniform: scalar registers
     const int cnt = __builtin_amdgcn_readfirstlane(g_ld(t.seg_count + L));

@@ -48,14 +48,13 @@ template <bool Wide> struct Lane {
   float dx, dy, dz;
   __device__ __forceinline__ Off at(int u) const { return (Off(unsigned(u)) << 3) + offb; }
 };
-template <bool Wide> __device__ __forceinline__ Lane<Wide> lane_of(const Dims &d, int block) {
-  const Group q = group_at(block / 32, block, int(threadIdx.x));  // 32 lanes per entry
+template <bool Wide> __device__ __forceinline__ Lane<Wide> lane_of(const Dims &d) {
   Lane<Wide> l;
   l.lane = int(threadIdx.x) & 63;
   l.half = l.lane >> 5;
   l.wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
-  l.slot = q.g;
-  const bool nb = q.cnt > 0;
+  l.slot = l.lane & 31;
+  const bool nb = l.slot < 26;
   l.k = nb ? kSlots.k[l.slot] : 0;
   const int dx = nb ? kNX[l.k] : 0, dy = nb ? kNY[l.k] : 0, dz = nb ? kNZ[l.k] : 0;
   l.off = step_offset(d, dx, dy, dz);

@@ -943,7 +943,7 @@ __global__ void __launch_bounds__(kBlock) soma_balls(const TraceArgs *__restrict
   const int2 q = queue[blockIdx.x];
   const TraceArgs a = all[__builtin_amdgcn_readfirstlane(q.x)];
   const int L = __builtin_amdgcn_readfirstlane(q.y);
-  const Lane<Wide> ln = lane_of<Wide>(a.d, kBlock);
+  const Lane<Wide> ln = lane_of<Wide>(a.d);
   const int seg = __builtin_amdgcn_readfirstlane(g_ld(a.seg_start + L));  // uniform: scalar registers
     const int count = __builtin_amdgcn_readfirstlane(g_ld(a.seg_count + L));
   const Lists l = lists_of(a, sh, seg);
@@ -981,7 +981,7 @@ __global__ void __launch_bounds__(kBlock) trace_labels(const TraceArgs *__restri
     const int sample = __builtin_amdgcn_readfirstlane(q.x);
     const TraceArgs a = all[sample];  // uniform: scalar registers
     const int L = __builtin_amdgcn_readfirstlane(q.y);
-    const Lane<Wide> ln = lane_of<Wide>(a.d, kBlock);
+    const Lane<Wide> ln = lane_of<Wide>(a.d);
     const int seg = __builtin_amdgcn_readfirstlane(g_ld(a.seg_start + L));  // uniform: scalar registers
     const int count = __builtin_amdgcn_readfirstlane(g_ld(a.seg_count + L));
     const Lists l = lists_of(a, sh, seg);

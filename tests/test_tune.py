@@ -24,7 +24,7 @@ def test_header_round_trip(tmp_path, monkeypatch):
 
 
 def test_search_space_is_what_the_kernels_accept():
-    for name in ("BROOK_NB_BATCH", "BROOK_FLOOD_NB_BATCH"):  # the chunkings for_parts implements
+    for name in ("BROOK_NB_BATCH", "BROOK_FLOOD_NB_BATCH"):  # those the label kernels are run with on the CPU
         assert set(tune.SPACE[name]) <= {9, 13, 26}
     for name in ("BROOK_TRACE_BLOCK", "BROOK_FLOOD_BLOCK"):
         assert all(v % 64 == 0 and v <= 1024 for v in tune.SPACE[name])  # whole waves, one workgroup
