@@ -1,6 +1,6 @@
 """The device postprocess where its forms meet, against the oracle: components around the size whose
 state fits LDS (loops about 2 700 vertices, trees about 5 300), repeated rows, join cells that fit
-one 64-bit key and cells that do not (a millionth wide, where a label's radii are 0)."""
+one 64-bit key and cells that do not (a millionth wide, where a label's radii are 0), waves of few and of many."""
 import numpy as np
 import pytest
 
@@ -61,9 +61,10 @@ def test_ticks_of_trees_by_size(post, n):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("radius,spread", [(2.0, 40.0), (0.0, 40.0), (1.5, 3e7), (0.0, 3e7)])
+@pytest.mark.parametrize("radius,spread", [(2.0, 40.0), (8.0, 40.0), (30.0, 40.0), (0.0, 40.0), (1.5, 3e7), (0.0, 3e7)])
 def test_joins_in_packed_and_wide_cells(post, radius, spread):
-    """Short chains of two labels; some ends meet a chain of the other end of the volume exactly."""
+    """Short chains of two labels; some ends meet a chain of the other end of the volume exactly. Their
+    vertices lie in a few cells (radius 30) up to one each."""
     rng = np.random.default_rng(int(spread) + int(radius * 10))
     parts = []
     for label in (1, 2):
