@@ -44,7 +44,7 @@ def _kernel_table(stats, n, b_in, b_cc, F):
         "edt": (["edt_x", "edt_y", "edt_z"], (3 * b_cc + 4 + 8 + 8) * n),
         "prepare_labels": (["prepare_labels"], 12 * flood),
         "init_words": (["init_words"], (b_cc + 4) * n + 8 * F),
-        "pdrf_alive": (["pdrf_alive"], b_cc * n + (4 + 4 + 4 + 8) * F),
+        "pdrf_alive": (["pdrf_alive"], b_cc * n + (4 + 4 + 8 + 8) * F),
         "trace_labels": (["trace_labels"], 12 * reached + 13 * claimed),
     }
     rows = {}

@@ -265,7 +265,7 @@ __global__ void __launch_bounds__(kRunBlock) edt_run_fh(const CC *cc, Dims dm, i
 // four rows from each of those then share one pass over the candidates up to the next: some ten
 // candidates per voxel whatever the distances are.
 // The envelope of the long-line path gives the same values: w2 has a float's 24 bits and a distance
-// at most 12, so w2 * dq * dq is exact in float64 (and the fused sums below round once, as its
+// at most 13, so w2 * dq * dq is exact in float64 (and the fused sums below round once, as its
 // separate ones do), the least of the sums is the envelope's value, and candidates that tie give the
 // same bits.
 // LDS per line and position: 4 bytes of height, a start and a foreground bit, and a 16-bit vertex for

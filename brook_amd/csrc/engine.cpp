@@ -395,7 +395,7 @@ class Sample {
         if (!evicted[id]) kept.push_back(id);
       labels_.swap(kept);
     }
-    // The early root searches built the records and voxel lists of the components as they were
+    // The early root searches built the words and voxel lists of the components as they were
     // before any soma painting: they serve the floods too unless a soma's voids were painted.
     std::vector<long long> early_roots;
     if (root_job_.valid()) early_roots = root_job_.get();
@@ -626,7 +626,7 @@ class Sample {
     target_ = target_dev_.download(*cx_);
     max_daf_ = max_daf_dev_.download(*cx_);
 
-    // PDRF (exponent a power of two: squarings), alive bits, rails, target order
+    // PDRF (exponent a power of two: squarings) and claim words, rails, target order
     std::vector<float> M(k_, 0.0f), inv(k_, 0.0f);
     std::vector<uint8_t> use(k_, 0);
     for (int id : labels_) {
@@ -1012,7 +1012,7 @@ class Sample {
   bool early_borders_ = false, borders_ready_ = false;
   double border_ms_[2] = {0, 0};  // device and host milliseconds of the border job
   std::future<std::vector<std::vector<Point>>> border_job_;
-  // The early root searches: the records and voxel lists they built, and per id the root found, or
+  // The early root searches: the words and voxel lists they built, and per id the root found, or
   // -1 (written by the job, read after joining it).
   Buffer<unsigned> early_mask_;
   Buffer<unsigned long long> early_road_;

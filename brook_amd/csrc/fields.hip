@@ -2,7 +2,7 @@
 //   * label voxel lists (segments laid out by id, from one wave-aggregated atomic per run),
 //   * one workgroup per label from a device work queue: root-search flood + argmax, DAF flood +
 //     argmax (label-gated geometric SSSP, the unique float32 min-plus fixpoint), no grid barriers,
-//   * PDRF and the alive bit in one streaming pass, the root rails, the target-order keys.
+//   * the PDRF's road words and the free claim words in one streaming pass, the root rails, the target-order keys.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -433,7 +433,7 @@ __global__ void __launch_bounds__(kFloodBlock) prepare_labels(const FloodJob *__
       g_st(t.target + L, key ? (long long)(0xFFFFFFFFu - (unsigned)key) : -1LL);
       g_st(t.max_daf + L, key ? __uint_as_float((unsigned)(key >> 32)) : 0.0f);
     }
-    for (int j = threadIdx.x; j < cnt; j += blockDim.x) {  // DAF out, words back to ~0
+    for (int j = threadIdx.x; j < cnt; j += blockDim.x) {  // DAF out, words back to kFloodFree
       const int v = g_ld(list + j);
       g_st(job.daf + v, __uint_as_float(road_dist(lp_u64(t.road + v))));
       sp_u64(t.road + v, kFloodFree);

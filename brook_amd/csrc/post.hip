@@ -641,7 +641,9 @@ struct Pieces {
 };
 
 // The components (of `count`) whose state fits LDS and the others, as lists on the device;
-// lds: the largest fitting state.
+// lds: the largest fitting state, which every block of the launch asks for, so one large component
+// leaves the small ones fewer waves: the loops of 20 000 components of 14 vertices take 2.0 ms, beside one
+// of 2500 vertices 8.6 (a lane per component 2.1 and 15.3).
 struct Split {
   Buffer<int> small, large;
   int nsmall = 0, nlarge = 0;
